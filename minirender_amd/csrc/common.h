@@ -93,11 +93,16 @@ enum Counter : int {
   kError = 3,        // set when a bounded wait hit its limit
   kClipped = 4,      // input triangles that crossed the near plane
   kTileTicket = 5,
-  kBinEntries = 6,   // total (tile, triangle) pairs (written by the scan)
+  kBinEntries = 6,   // total (tile, triangle) pairs (the scan's and the direct ones)
   kParts = 7,        // work items of split tiles (written by the scan)
   kHeavy = 8,        // tiles split over several work items
   kHeavyOverflow = 9,
   kListed = 10,      // tiles in the raster's tile list (written by the scan)
+  kDirect = 11,      // direct items of all jobs (0: the direct lists are empty)
+  kDirectPairs = 14, // (tile, direct item) pairs, at the end of the bin list
+  kDirectTilesListed = 15,  // tiles with such pairs only, at the end of the tile list
+  kWidePx = 12,      // bbox pixels of the items that want edge checkpoints ...
+  kWideRows = 13,    // ... and their bbox rows (they choose the column spacing)
   kNumCounters = 16
 };
 
@@ -117,10 +122,30 @@ MR_HD inline int64_t xcd_remap(int64_t b, int64_t n) {
 constexpr int kCtrStride = 16;
 constexpr int kCtrStride64 = kCtrStride / 2;  // the same spacing in 64-bit words
 
-// The edge-checkpoint buffer is cut into this many segments, each with its
-// own allocation counter (kCtrStride words apart): one shared counter would
-// serialize every binning wavefront's atomic.
+// The first half of the edge-checkpoint buffer is cut into this many
+// segments, each with its own allocation counter (kCtrStride words apart):
+// one shared counter would serialize every wavefront's atomic.  The second
+// half is one segment, for wavefronts that need more than an eighth of a
+// small one (few: their triangles are large); its entries and row tasks are
+// counted by two counters in the gaps between the segments'.
 constexpr int kCkptSegs = 64;
+constexpr int kCkptBigEntries = kCtrStride / 2;               // word of ckpt_ctr
+constexpr int kCkptBigRows = kCtrStride + kCtrStride / 2;
+
+// Items over kDirectTiles tiles or more are not binned with the others but
+// listed per job (kDirectCap of them or as many as the batch's scratch has
+// room for; further ones are binned), and the tiles test that list.
+// Binning costs a wavefront a step per 64 pairs, so one of 64 such triangles
+// keeps counting and scattering when the rest of the GPU is done (3,000
+// triangles over a 1080p frame, 1 M pairs: geometry 700 us, binning 1,230);
+// testing costs every tile the list.  From 16 tiles: textured 1080p terrain
+// with loose triangles 270 us a frame, 263 from 32, 310 (launch of the scan
+// alone 60 us) from 8, 336 without lists; 48 mixed frames in a batch 911, 957,
+// 898 and 990; 8.4 M-triangle 4K terrain 516, 544, 529 and 635 us of kernels.
+constexpr int kDirectTiles = 16;
+constexpr uint32_t kDirectCap = 4096;
+constexpr uint32_t kDirectMin = 16;  // lists shorter than this are not used
+constexpr uint32_t kDirectFlag = 0x80000000u;  // in BinItem::draw: listed, not binned
 
 constexpr int kRegion = 128;       // item slots per geometry wavefront (64 x 2)
 constexpr int kShadeBlock = 256;   // pixels per deferred-shading workgroup

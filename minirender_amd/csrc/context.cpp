@@ -374,9 +374,21 @@ static BatchArgs make_args(mr_ctx* c, Slot& sl, const BatchPlan& p) {
   if (a.bins_cap > 0xFFFFFFF0ull) a.bins_cap = 0xFFFFFFF0ull;
   a.ckpt_base = (int2*)s.ckpt_base.p;
   a.ckpt = (float2*)s.ckpt.p;
+  // The jobs' direct lists take at most the last quarter of the checkpoint
+  // buffer: no scratch of their own, so what fits a budget stays the same.
+  const uint64_t nj = p.jobs.size();
+  uint64_t ckpt_bytes = s.ckpt.bytes;
+  const uint64_t per_job = ckpt_bytes / 4 / nj;
+  const uint64_t line = kCtrStride * 4;
+  if (per_job >= line + kDirectMin * sizeof(BinItem)) {
+    a.direct_cap = (uint32_t)std::min<uint64_t>((per_job - line) / sizeof(BinItem), kDirectCap);
+    ckpt_bytes = (ckpt_bytes - nj * (line + a.direct_cap * sizeof(BinItem))) & ~(uint64_t)255;
+    a.direct_count = (uint32_t*)((char*)s.ckpt.p + ckpt_bytes);
+    a.direct = (BinItem*)(a.direct_count + nj * kCtrStride);
+  }
   // Checkpoint capacity, held to twice the row-task entries: the row tasks
   // of every item given checkpoints then fit in their segment.
-  a.ckpt_cap = std::min<uint64_t>(std::min<uint64_t>(s.ckpt.bytes / 8, 2 * (s.wide.bytes / 8)),
+  a.ckpt_cap = std::min<uint64_t>(std::min<uint64_t>(ckpt_bytes / 8, 2 * (s.wide.bytes / 8)),
                                   0xFFFFFFF0ull);
   a.ckpt_ctr = (unsigned long long*)s.ckpt_ctr.p;
   a.ckpt_rows = (unsigned long long*)s.wide.p;

@@ -334,6 +334,62 @@ struct TriSetup {
   int bx0, bx1, by0, by1;    // clamped pixel bbox, inclusive
 };
 
+// Reciprocal of a bound's slope (cover_rows pads what it is used for).
+MR_HD inline float approx_rcp(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rcpf(x);
+#else
+  return 1.0f / x;
+#endif
+}
+
+// Shrinks the rows [r0, r1] of the triangle's bbox to those in which it may
+// cover a pixel of its columns [c0, c1]; r1 < r0 when there is none.  A row
+// kept may cover nothing; a row dropped covers nothing in the raster.  There
+// an edge value is the serial chain e += n.x from the bbox's left column
+// (Renderer.cpp:240-243): its start is two products and a sum, and each of
+// its n steps rounds by at most 2^-24 of the values met, which |n.x| |x - p.x|
+// + |n.y| |y - p.y| over the row bounds (M).  The chain so stays within
+// (n + 8) 2^-24 M of the edge function, and a row whose edge function is below
+// -(n + 16) 2^-23 M at every column has all pixels outside.  The row where
+// that begins is solved for with one row and 1e-5 of slack.  NaN keeps rows.
+MR_HD inline void cover_rows(const TriSetup& s, int c0, int c1, int& r0, int& r1) {
+  const float xl = (float)c0 + 0.5f, xr = (float)c1 + 0.5f, xs = (float)s.bx0 + 0.5f;
+  const float yt = (float)r0 + 0.5f, yb = (float)r1 + 0.5f;
+  const float rel = (float)(c1 - s.bx0 + 16) * 1.1920929e-7f;
+  const float dx2 = bmax(fabsf(xs - s.p2x), fabsf(xr - s.p2x));
+  const float dy2 = bmax(fabsf(yt - s.p2y), fabsf(yb - s.p2y));
+  const float dx0 = bmax(fabsf(xs - s.p0x), fabsf(xr - s.p0x));
+  const float dy0 = bmax(fabsf(yt - s.p0y), fabsf(yb - s.p0y));
+  const float m1 = fabsf(s.n1x) * dx2 + fabsf(s.n1y) * dy2;
+  const float m2 = fabsf(s.n2x) * dx0 + fabsf(s.n2y) * dy0;
+  const float m0 = fabsf(s.n2x) * dx2 + fabsf(s.n2y) * dy2;  // e2 measured from p2
+  float lo = yt, hi = yb;
+  // Keep the rows where at + nx (x - ax) + ny (y - ay) >= -err at some column.
+  auto edge = [&](float nx, float ny, float ax, float ay, float at, float dy, float err) {
+    const float f = (bmax(nx * (xl - ax), nx * (xr - ax)) + at) + err;
+    if (fabsf(ny) > 1e-30f) {
+      const float q = -f * approx_rcp(ny);
+      const float t = ay + q;
+      const float pad = 1.0f + 1e-5f * (fabsf(ay) + fabsf(q));
+      if (ny > 0.0f) lo = bmax(lo, t - pad);
+      else hi = bmin(hi, t + pad);
+    } else if (f + 1e-30f * dy < 0.0f) {
+      hi = yt - 2.0f;
+    }
+  };
+  edge(s.n1x, s.n1y, s.p2x, s.p2y, 0.0f, dy2, rel * m1);
+  edge(s.n2x, s.n2y, s.p0x, s.p0y, 0.0f, dy0, rel * m2);
+  // (1 - e1) - e2, from vertex 2 where e1 is 0 (and e2 near 1, or far from
+  // it: the area the normals are divided by loses bits when a vertex lies
+  // far away).
+  const float at2 = 1.0f - (s.n2x * (s.p2x - s.p0x) + s.n2y * (s.p2y - s.p0y));
+  edge(-(s.n1x + s.n2x), -(s.n1y + s.n2y), s.p2x, s.p2y, at2, dy2,
+       2.0f * rel * (((1.0f + m1) + m2) + m0));
+  r0 = (int)floorf(bmin(lo, yb + 2.0f) - 0.5f);
+  r1 = (int)floorf(bmax(hi, yt - 2.0f) - 0.5f);
+}
+
 // A vertex projected to the screen (Renderer.cpp:191-203, 225-227): pixel
 // position and the depth attribute the raster interpolates, -1/z_eye under a
 // perspective projection or NDC z under an orthographic one.  It depends on

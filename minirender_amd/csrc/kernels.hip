@@ -4,7 +4,7 @@
 //   k_clear   look-back words, tile counts and merge counters when the
 //             scratch is new (afterwards the shading kernel leaves them
 //             zero); batch and checkpoint counters when the batch has no
-//             triangles (else geometry zeroes them)
+//             triangles (else the vertex kernel zeroes them)
 //   k_vertex  (a) eye-space transform and projection once per vertex of each
 //             (attribute arrays, modelview) group of a job (Renderer.cpp:340-349,
 //             191-203): the per-material meshes of a model share one group
@@ -12,21 +12,23 @@
 //             triangle (Renderer.cpp:351-380, 163-236).  Each wavefront
 //             compacts its survivors into its own region of the item stream
 //             (ballot + popcount prefix, no global atomic) and counts its
-//             (tile, triangle) pairs with one atomic per distinct tile
+//             (tile, triangle) pairs with one atomic per distinct tile.
+//             Triangles over many tiles go to their job's direct list instead
 //   k_scan    (c) exclusive scan of the tile counts (decoupled look-back);
 //             tiles with more pairs than one work item are split into parts,
 //             the others with pairs listed for the raster, empty ones marked.
-//             For a batch of at most kCkptScanRegions regions, the launch's
-//             other workgroups, beside the one-workgroup scan, allocate the
-//             edge checkpoints and row tasks of triangles at least 64 pixels
-//             wide spanning several tile columns
+//             Beside the scan the launch's other workgroups match the direct
+//             lists with the tiles and, for a batch of at most
+//             kCkptScanRegions regions, allocate the edge checkpoints and row
+//             tasks of triangles at least 64 pixels wide spanning several
+//             tile columns
 //   k_bin     (c) scatter of (triangle id, draw) into the tiles' bin lists:
 //             per wavefront step, one atomic instruction for all distinct
 //             tiles.  For larger batches binning allocates the checkpoints
 //             itself (it reads the items anyway)
 //   k_rows    (c) row pre-pass: one lane per row of such a triangle walks it
-//             once and stores the edge values where it enters each tile
-//             column; for the smaller batches the tail of the binning
+//             once and stores the edge values where it enters each checkpoint
+//             column (of a tile's width or more); for the smaller batches the tail of the binning
 //             kernel (k_bin_rows)
 //   k_tile    (d) per-tile raster (listed tiles, parts of split tiles, row
 //             bands) with the tile's 64-bit (depth key, draw-order id) buffer
@@ -101,17 +103,27 @@ __device__ u64 lookback(u64* status, int idx, u64 aggregate, u64* counters) {
 // Each stage is a device function of its workgroup index vb in a grid of
 // nvb workgroups of 256 threads: run by its own kernel (vb = blockIdx.x),
 // or by the persistent kernel, whose workgroups take stage work from queues.
+// Counters of a batch: the batch counters, the checkpoint segments' and the
+// lengths of the direct lists.
+__device__ __forceinline__ void zero_counters(const BatchArgs& a) {
+  if (threadIdx.x < kNumCounters) a.counters[threadIdx.x] = 0;
+  if (threadIdx.x < kCkptSegs) a.ckpt_ctr[threadIdx.x * kCtrStride] = 0;
+  if (threadIdx.x == 0) a.ckpt_ctr[kCkptBigEntries] = a.ckpt_ctr[kCkptBigRows] = 0;
+  if (a.direct_cap)
+    for (int i = threadIdx.x; i < a.njobs * 8; i += 256)
+      a.direct_count[(size_t)(i >> 3) * kCtrStride + (i & 7)] = 0;
+}
+
 __device__ __forceinline__ void stage_clear(const BatchArgs& a, int vb, int nvb) {
-  // The checkpoint segment counters too: a batch without triangles (no
-  // geometry, which zeroes them otherwise) must not leave the row pre-pass
-  // the last batch's row tasks.
-  if (vb == 0 && threadIdx.x < kCkptSegs) a.ckpt_ctr[threadIdx.x * kCtrStride] = 0;
-  const int n = max(max(a.scan_blocks, a.ntiles), (int)kNumCounters);
+  // (A batch without triangles runs no vertex kernel, which zeroes them
+  // otherwise: it must not leave the row pre-pass the last batch's tasks.)
+  if (vb == 0) zero_counters(a);
+  const int n = max(a.scan_blocks, a.ntiles);
   for (int i = vb * 256 + (int)threadIdx.x; i < n; i += nvb * 256) {
-    if (i < kNumCounters) a.counters[i] = 0;
     if (i < a.scan_blocks) a.scan_status[i] = 0;
     if (i < a.ntiles) {
       a.tile_count[(size_t)i * kCtrStride64] = 0;
+      a.tile_count[(size_t)i * kCtrStride64 + 1] = 0;
       a.tile_done[i] = 0;
     }
   }
@@ -405,6 +417,9 @@ __device__ inline void vertex_record(const BatchArgs& a, const DrawDesc& D, cons
 }
 
 __device__ __forceinline__ void stage_vertex(const BatchArgs& a, int vb, int nvb) {
+  // Geometry adds to the batch counters and the checkpoint allocation follows
+  // it: both start from zero.
+  if (vb == 0) zero_counters(a);
   // Contiguous range per workgroup (a multiple of kVertexStep): one group
   // search, then stepping.
   const int64_t chunk = ((a.total_verts + (int64_t)nvb * kVertexStep - 1) /
@@ -558,13 +573,115 @@ __device__ void wave_tile_pairs(const BatchArgs& a, bool active, uint32_t id, ui
   }
 }
 
+// Direct items of a wavefront step: up to two per lane (d0, d1), appended to
+// their job's list by one atomic per job.  Clears the flag of an item that
+// finds no room; it is then binned.
+__device__ inline void direct_append(const BatchArgs& a, int job, bool& d0, const BinItem& i0,
+                                     bool& d1, const BinItem& i1) {
+  const int lane = threadIdx.x & 63;
+  const u64 lt = (1ull << lane) - 1ull;
+  u64 pend = __ballot(d0 || d1);
+  if (lane == (int)__builtin_ctzll(pend)) atomicAdd(&a.counters[kDirect], 1ull);
+  while (pend) {
+    const int l = __builtin_ctzll(pend);
+    const int jj = __builtin_amdgcn_readlane(job, l);
+    const bool mine = (d0 || d1) && ((pend >> lane) & 1ull) && job == jj;
+    const u64 g0 = __ballot(mine && d0), g1 = __ballot(mine && d1);
+    uint32_t base = 0;
+    uint32_t* const line = a.direct_count + (size_t)jj * kCtrStride;
+    if (lane == l) base = atomicAdd(line, (uint32_t)(__popcll(g0) + __popcll(g1)));
+    // Bounding box of the job's list (as maxima: the words start at zero).
+    uint32_t box[4] = {0, 0, 0, 0};
+    if (mine) {
+      const BinItem& p = d0 ? i0 : i1;
+      const BinItem& q = d1 ? i1 : i0;
+      box[0] = (uint32_t)(kMaxDim - min(p.bx0, q.bx0));
+      box[1] = max(p.bx1, q.bx1);
+      box[2] = (uint32_t)(kMaxDim - min(p.by0, q.by0));
+      box[3] = max(p.by1, q.by1);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) box[k] = max(box[k], (uint32_t)__shfl_xor(box[k], o));
+      if (lane == l) atomicMax(line + 1 + k, box[k]);
+    }
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, l);
+    pend &= ~(g0 | g1);
+    if (mine) {
+      uint32_t pos = base + (uint32_t)(__popcll(g0 & lt) + __popcll(g1 & lt));
+      BinItem* const list = a.direct + (size_t)jj * a.direct_cap;
+      if (d0) {
+        if (pos < a.direct_cap) list[pos] = i0;
+        else d0 = false;
+        pos++;
+      }
+      if (d1) {
+        if (pos < a.direct_cap) list[pos] = i1;
+        else d1 = false;
+      }
+    }
+  }
+}
+
+// Whether an item wants edge checkpoints: at least kCkptMinSpan pixels wide
+// and over several tile columns.  Narrower triangles are walked from their
+// bbox's left column (fewer than kCkptMinSpan steps beyond a tile).
+constexpr int kCkptMinSpan = 64;
+__device__ inline bool wants_ckpt(int bx0, int bx1, int sw) {
+  return bx1 - bx0 + 1 >= kCkptMinSpan && (bx1 >> sw) > (bx0 >> sw);
+}
+
+// The large items of a geometry step (l0, l1: the lane's first and second
+// sub-triangle is one): lists the direct ones, and adds the pixels and rows
+// of those that want checkpoints to the sums the allocation picks its column
+// spacing from.  Returns which of the two were listed (bits 0 and 1).
+constexpr int kLargeSpan = 24;  // < the span of 16 tiles of 8 x 8, and of kCkptMinSpan
+__device__ inline int large_items(const BatchArgs& a, bool l0, bool l1, const TriSetup& s0,
+                                  const TriSetup& s1, uint32_t id0, uint32_t id1, uint32_t draw,
+                                  int job, int sw, int sh) {
+  auto tiles_of = [&](const TriSetup& s) {
+    return ((s.bx1 >> sw) - (s.bx0 >> sw) + 1) * ((s.by1 >> sh) - (s.by0 >> sh) + 1);
+  };
+  bool d0 = a.direct_cap && l0 && tiles_of(s0) >= kDirectTiles;
+  bool d1 = a.direct_cap && l1 && tiles_of(s1) >= kDirectTiles;
+  if (__ballot(d0 || d1)) {
+    const BinItem i0 = {id0, draw, (uint16_t)s0.bx0, (uint16_t)s0.bx1, (uint16_t)s0.by0,
+                        (uint16_t)s0.by1};
+    const BinItem i1 = {id1, draw, (uint16_t)s1.bx0, (uint16_t)s1.bx1, (uint16_t)s1.by0,
+                        (uint16_t)s1.by1};
+    direct_append(a, job, d0, i0, d1, i1);
+  }
+  const bool w0 = l0 && wants_ckpt(s0.bx0, s0.bx1, sw);
+  const bool w1 = l1 && wants_ckpt(s1.bx0, s1.bx1, sw);
+  if (__ballot(w0 || w1)) {
+    u64 px = 0;
+    uint32_t rows = 0;
+    if (w0) rows = (uint32_t)(s0.by1 - s0.by0 + 1), px = (u64)rows * (s0.bx1 - s0.bx0 + 1);
+    if (w1) {
+      const uint32_t r = (uint32_t)(s1.by1 - s1.by0 + 1);
+      rows += r;
+      px += (u64)r * (s1.bx1 - s1.bx0 + 1);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      px += __shfl_xor(px, o);
+      rows += __shfl_xor(rows, o);
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicAdd(&a.counters[kWidePx], px);
+      atomicAdd(&a.counters[kWideRows], (u64)rows);
+    }
+  }
+  return (d0 ? 1 : 0) | (d1 ? 2 : 0);
+}
+
 // (a)+(b): one lane per input triangle; wavefront w writes its survivors to
-// items[w * kRegion ...] and their number to region_count[w].
+// items[w * kRegion ...] and their number to region_count[w].  Those over
+// kDirectTiles tiles or more go to their job's direct list: a wavefront's 64
+// triangles of hundreds of tiles each would count (and later scatter) their
+// pairs 64 at a time, one wavefront alone.
 __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) {
-  // The batch counters and checkpoint segment counters are first used by the
-  // scan and the binner: clear them here.
-  if (vb == 0 && threadIdx.x < kNumCounters) a.counters[threadIdx.x] = 0;
-  if (vb == 0 && threadIdx.x < kCkptSegs) a.ckpt_ctr[threadIdx.x * kCtrStride] = 0;
   const int lane = threadIdx.x & 63;
   const int sw = __ffs(a.tile_w) - 1, sh = __ffs(a.tile_h) - 1;
   uint32_t nclipped = 0;
@@ -587,7 +704,7 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
     int sub0 = 0, sub1 = 0, ns = 0;
     bool clipped = false;
     uint32_t draw = 0;
-    int tbase = 0, tiles_x = 1;
+    int tbase = 0, tiles_x = 1, job = 0;
     // The wave's draw: step the uniform draw index to the wave's first
     // triangle; lanes past the next draw's start step further (draw
     // boundaries inside a wavefront are rare).
@@ -602,6 +719,7 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
         ns = tri_setup(a, D, J, (int)(g - D.tri_begin), s0, sub0, s1, sub1, clipped);
         tbase = D.tile_base;
         tiles_x = D.tiles_x;
+        job = D.job;
       };
       if (__ballot(d == dw) == __ballot(1)) {
         const DrawDesc Du = uniform_draw(a, dw);
@@ -628,15 +746,27 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
     if (ns == 2)
       a.items[pos + 1] = BinItem{id1, draw, (uint16_t)s1.bx0, (uint16_t)s1.bx1,
                                  (uint16_t)s1.by0, (uint16_t)s1.by1};
+    // Direct items and those that want checkpoints are at least kLargeSpan
+    // pixels in width and height together; few wavefronts hold any.
+    bool d0 = false, d1 = false;
+    const bool l0 = ns >= 1 && (s0.bx1 - s0.bx0) + (s0.by1 - s0.by0) >= kLargeSpan;
+    const bool l1 = ns == 2 && (s1.bx1 - s1.bx0) + (s1.by1 - s1.by0) >= kLargeSpan;
+    if (__ballot(l0 || l1)) {
+      const int large = large_items(a, l0, l1, s0, s1, id0, id1, draw, job, sw, sh);
+      d0 = large & 1;
+      d1 = large & 2;
+      if (d0) a.items[pos].draw = draw | kDirectFlag;
+      if (d1) a.items[pos + 1].draw = draw | kDirectFlag;
+    }
     // Pairs and walk work per tile, in one 64-bit atomic per group.
     auto count = [&](int key, uint32_t n, uint32_t work) -> uint32_t {
       atomicAdd(&a.tile_count[(size_t)key * kCtrStride64], ((u64)work << 32) | (u64)n);
       return 0u;
     };
-    wave_tile_pairs<false>(a, ns >= 1, id0, draw, tbase, tiles_x, s0.bx0, s0.bx1, s0.by0,
+    wave_tile_pairs<false>(a, ns >= 1 && !d0, id0, draw, tbase, tiles_x, s0.bx0, s0.bx1, s0.by0,
                            s0.by1, sw, sh, count);
     if (b2)
-      wave_tile_pairs<false>(a, ns == 2, id1, draw, tbase, tiles_x, s1.bx0, s1.bx1, s1.by0,
+      wave_tile_pairs<false>(a, ns == 2 && !d1, id1, draw, tbase, tiles_x, s1.bx0, s1.bx1, s1.by0,
                              s1.by1, sw, sh, count);
   }
   __shared__ uint32_t sh_clipped;
@@ -676,6 +806,7 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a) {
   __shared__ u64 sh_w[kScanBlock / 64];
   __shared__ u64 sh_excl;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const u64 ndirect = a.counters[kDirect];  // in flight with the tile counts
   // (A single workgroup needs no ticket: it is workgroup 0.)
   if (tid == 0) sh_blk = a.scan_blocks == 1 ? 0 : (int)atomicAdd(&a.counters[kScanTicket], 1ull);
   __syncthreads();
@@ -689,6 +820,22 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a) {
     v[i] = (uint32_t)tc;
     nbv[i] = band_count(a, v[i], (uint32_t)(tc >> 32));
     sum += v[i];
+  }
+  // Bit i of `listed`: tile base + i belongs to a job with direct items.
+  uint32_t listed = 0;
+  if (ndirect != 0ull && base < a.ntiles) {
+    int j = job_lookup(a.tile_hint, a.job_tile_base, a.njobs, base);
+    int next = 0;
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+      if (base + i < a.ntiles && (i == 0 || base + i >= next)) {
+        if (i) j++;
+        any = a.direct_count[(size_t)j * kCtrStride] != 0;
+        next = j + 1 < a.njobs ? a.job_tile_base[j + 1] : 0x7FFFFFFF;
+      }
+      listed |= (any ? 1u : 0u) << i;
+    }
   }
   u64 x = sum;  // wave inclusive scan
 #pragma unroll
@@ -800,41 +947,68 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a) {
         }
         ps += nbv[i];
       } else if (v[i] > 0) {
-        a.tile_list[ls++] = make_uint4((uint32_t)t, o, v[i], 0u);
+        a.tile_list[ls++] = make_uint4((uint32_t)t, o, v[i], (listed >> i) & 1u);
       } else {
         slot = kEmptyTile;  // shading writes its pixels' background
       }
-      a.tile_heavy[t] = slot;
+      // (stage_direct decides on the tiles without pairs of jobs with lists.)
+      if (v[i] > 0 || !((listed >> i) & 1u)) a.tile_heavy[t] = slot;
     }
     run += v[i];
   }
 }
 
 
-// Edge checkpoints of the wavefront's items: an item at least
-// kCkptMinSpan pixels wide that spans ntx > 1 tile columns gets ntx entries
-// per pixel row (one per column, where the row enters it) and one row task
-// per pixel row for the row pre-pass, all taken from the checkpoint segment
-// of the wavefront (wavefronts spread over kCkptSegs segments) by one 64-bit
-// atomic: entries in the low 40 bits of the segment counter, row tasks in
-// the high 24.  Every such row holds at least two entries, so a segment's
-// row tasks fit in half its entry count.  The base is stored pre-offset by
-// the item's first row and column, so that a reader needs only the row and
-// the tile column.  Items narrower than kCkptMinSpan pixels get no entry
-// (their readers test the width first); wide ones that found no room get
-// {0, 0}.  Either way the raster and shading walk such rows from the bbox's
-// left column (fewer than kCkptMinSpan steps beyond a tile for the narrow).
-constexpr int kCkptMinSpan = 64;
+// Spacing of the checkpoint columns, 2^cs pixels: the tile width, or the
+// smallest power of two above it (256 at most) with which the batch's
+// checkpoints fit a quarter of the buffer (its segments fill unevenly).
+// Overlapping large triangles would fill it many times over at the tile's
+// width, and a row without checkpoints is walked from its bbox's left column
+// by every tile and pixel: up to 255 steps from the checkpoint left of it are
+// far fewer: 3,000 triangles over a 1080p frame (17 M checkpoints at the
+// tile's width, room for 4 M) took the raster 3.8 ms and shading 0.24 ms
+// without the spacing, 0.16 and 0.057 ms with it and cover_rows.
+constexpr int kCkptMaxShift = 8;
+__device__ inline int ckpt_shift(const BatchArgs& a, int sw) {
+  const u64 px = a.counters[kWidePx], rows = a.counters[kWideRows];
+  int cs = sw;
+  while (cs < kCkptMaxShift && (px >> cs) + 2 * rows > a.ckpt_cap / 4) cs++;
+  return cs;
+}
+
+// Checkpoint segments: kCkptSegs small ones over the first half of the
+// buffer, and the second half as one (see kCkptSegs).
+struct CkptSeg {
+  u64 first, cap, rows_first, rows_cap;
+};
+__device__ inline CkptSeg ckpt_seg(const BatchArgs& a, int seg) {
+  const u64 half = a.ckpt_cap / 2, cap = half / kCkptSegs;
+  if (seg < kCkptSegs) return CkptSeg{seg * cap, cap, seg * (cap / 2), cap / 2};
+  return CkptSeg{half, half, half / 2, half / 2};
+}
+
+// Edge checkpoints of the wavefront's items: an item that wants them
+// (wants_ckpt) and spans several checkpoint columns gets one entry per pixel
+// row and column (where the row enters it) and one row task per pixel row for
+// the row pre-pass, all taken from the checkpoint segment of the wavefront
+// (wavefronts spread over the small segments) by one 64-bit atomic: entries
+// in the low 40 bits of the segment counter, row tasks in the high 24.
+// Every such row holds at least two entries, so a segment's row tasks fit in
+// half its entry count.  The base is stored pre-offset by the item's first
+// row and column, so that a reader needs only the row and the column.  Wide
+// items that found no room, or lie in one column, get {0, 0}: the raster and
+// shading walk their rows from the bbox's left column.
 constexpr u64 kCkptEntryMask = (1ull << 40) - 1;
 
-__device__ inline void ckpt_alloc(const BatchArgs& a, bool act, const BinItem& it, int sw,
+__device__ inline void ckpt_alloc(const BatchArgs& a, bool act, const BinItem& it, int sw, int cs,
                                   uint32_t item, int vb) {
   const int lane = threadIdx.x & 63;
-  const int btx = it.bx0 >> sw;
-  const int ntx = act ? (it.bx1 >> sw) - btx + 1 : 0;
+  const bool wide = act && wants_ckpt(it.bx0, it.bx1, sw);
+  if (__ballot(wide) == 0ull) return;  // the common case: no wide triangle here
+  const int btx = it.bx0 >> cs;
+  const int ntx = (it.bx1 >> cs) - btx + 1;
   const int rows = it.by1 - it.by0 + 1;
-  const bool want = ntx > 1 && it.bx1 - it.bx0 + 1 >= kCkptMinSpan;
-  if (__ballot(want) == 0ull) return;  // the common case: no wide triangle here
+  const bool want = wide && ntx > 1;
   const u64 need = want ? (u64)ntx * (u64)rows : 0ull;
   const uint32_t nrow = want ? (uint32_t)rows : 0u;
   u64 P = need;  // inclusive prefixes over the wave
@@ -850,45 +1024,52 @@ __device__ inline void ckpt_alloc(const BatchArgs& a, bool act, const BinItem& i
   }
   const u64 total = __shfl(P, 63);
   if (total == 0ull) {
-    if (want) a.ckpt_base[it.id] = make_int2(0, 0);
+    if (wide) a.ckpt_base[it.id] = make_int2(0, 0);
     return;
   }
   const uint32_t rtotal = __shfl(R, 63);
-  const u64 seg_cap = a.ckpt_cap / kCkptSegs;
-  const u64 seg_rows = seg_cap / 2;
-  const int seg = (int)(((uint32_t)vb * 4u + (threadIdx.x >> 6)) % kCkptSegs);
-  u64 old = 0;
-  if (lane == 63) old = atomicAdd(&a.ckpt_ctr[seg * kCtrStride], ((u64)rtotal << 40) | total);
-  old = __shfl(old, 63);
-  const u64 base = old & kCkptEntryMask, rbase = old >> 40;
-  bool ok = false;
-  if (want) {
-    const u64 first = base + P - need;  // within the segment
-    const int64_t off = (int64_t)(seg * seg_cap + first) - (int64_t)it.by0 * ntx - btx;
-    ok = need && first + need <= seg_cap && off >= INT32_MIN && off <= INT32_MAX;
-    a.ckpt_base[it.id] = ok ? make_int2((int)off, ntx) : make_int2(0, 0);
+  const int small = (int)(((uint32_t)vb * 4u + (threadIdx.x >> 6)) % kCkptSegs);
+  const bool big = total > ckpt_seg(a, small).cap / 8;
+  const CkptSeg sg = ckpt_seg(a, big ? kCkptSegs : small);
+  u64 base = 0, rbase = 0;
+  if (big) {
+    if (lane == 63) {
+      base = atomicAdd(&a.ckpt_ctr[kCkptBigEntries], total);
+      rbase = atomicAdd(&a.ckpt_ctr[kCkptBigRows], (u64)rtotal);
+    }
+    base = __shfl(base, 63);
+    rbase = __shfl(rbase, 63);
+  } else {
+    u64 old = 0;
+    if (lane == 63)
+      old = atomicAdd(&a.ckpt_ctr[small * kCtrStride], ((u64)rtotal << 40) | total);
+    old = __shfl(old, 63);
+    base = old & kCkptEntryMask;
+    rbase = old >> 40;
   }
-  // Row tasks of the items that got checkpoints: (item << 32) | row, the
-  // wavefront's rows spread over its lanes (owners by binary search of the
-  // prefix).  An item that got no room reserved its tasks all the same:
+  bool ok = false;
+  if (wide) {
+    const u64 first = base + P - need;  // within the segment
+    const int64_t off = (int64_t)(sg.first + first) - (int64_t)it.by0 * ntx - btx;
+    ok = need && first + need <= sg.cap && rbase + R <= sg.rows_cap && off >= INT32_MIN &&
+         off <= INT32_MAX;
+    a.ckpt_base[it.id] = ok ? make_int2((int)off, ntx | cs << 16) : make_int2(0, 0);
+  }
+  // Row tasks of the items that got checkpoints: (item << 32) | row, item by
+  // item with the whole wavefront.  An item that got no room reserved its tasks all the same:
   // they are written as "no task" (~0) and skipped.
   const uint32_t ex = R - nrow;
-  for (uint32_t j = 0; j < rtotal; j += 64) {
-    const uint32_t q = j + lane;
-    int lo = 0, hi = 63;
-#pragma unroll
-    for (int st = 0; st < 6; st++) {
-      const int mid = (lo + hi) >> 1;
-      if (__shfl(R, mid) > q) hi = mid; else lo = mid + 1;
-    }
-    const uint32_t oex = __shfl(ex, lo);
-    const int oby0 = __shfl((int)it.by0, lo);
-    const uint32_t oitem = __shfl(item, lo);
-    const bool ook = __shfl((int)ok, lo) != 0;
-    const u64 slot = rbase + q;
-    if (q < rtotal && slot < seg_rows)
-      a.ckpt_rows[(u64)seg * seg_rows + slot] =
-          ook ? ((u64)oitem << 32) | (uint32_t)(oby0 + (int)(q - oex)) : ~0ull;
+  u64 pend = __ballot(nrow != 0u);
+  while (pend) {
+    const int l = __builtin_ctzll(pend);
+    pend &= pend - 1;
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)nrow, l);
+    const uint32_t row0 = (uint32_t)__builtin_amdgcn_readlane((int)it.by0, l);
+    const u64 oitem = (u64)(uint32_t)__builtin_amdgcn_readlane((int)item, l) << 32;
+    const bool ook = __builtin_amdgcn_readlane((int)ok, l) != 0;
+    const u64 slot0 = rbase + (uint32_t)__builtin_amdgcn_readlane((int)ex, l);
+    for (uint32_t q = lane; q < n && slot0 + q < sg.rows_cap; q += 64)
+      a.ckpt_rows[sg.rows_first + slot0 + q] = ook ? oitem | (row0 + q) : ~0ull;
   }
 }
 
@@ -904,6 +1085,7 @@ __device__ __forceinline__ void stage_bin(const BatchArgs& a, int vb, int nvb) {
     a.heavy_keys[i] = ~0ull;
   const int sw = __ffs(a.tile_w) - 1, sh = __ffs(a.tile_h) - 1;
   const int64_t nw = (int64_t)nvb * 4;
+  const int cs = kAlloc ? ckpt_shift(a, sw) : 0;
   u64 nitems = 0;
   auto reserve = [&](int key, uint32_t n, uint32_t) -> uint32_t {
     return atomicAdd(&a.tile_cursor[(size_t)key * kCtrStride], n);
@@ -934,6 +1116,8 @@ __device__ __forceinline__ void stage_bin(const BatchArgs& a, int vb, int nvb) {
       // The job's tile grid, through scalar loads when the wavefront's items
       // share one draw (the common case).
       // (Lane 0 is active in every step: j < cnt.)
+      const bool binned = act && !(it.draw & kDirectFlag);
+      it.draw &= ~kDirectFlag;
       const uint32_t d0 = __builtin_amdgcn_readfirstlane(it.draw);
       const uint32_t dd = act ? it.draw : d0;
       int tbase, tiles_x;
@@ -945,8 +1129,8 @@ __device__ __forceinline__ void stage_bin(const BatchArgs& a, int vb, int nvb) {
         tbase = a.draws[dd].tile_base;
         tiles_x = a.draws[dd].tiles_x;
       }
-      if (kAlloc) ckpt_alloc(a, act, it, sw, (uint32_t)(r * kRegion + j + lane), vb);
-      wave_tile_pairs<true>(a, act, it.id, it.draw, tbase, tiles_x, it.bx0, it.bx1, it.by0,
+      if (kAlloc) ckpt_alloc(a, act, it, sw, cs, (uint32_t)(r * kRegion + j + lane), vb);
+      wave_tile_pairs<true>(a, binned, it.id, it.draw, tbase, tiles_x, it.bx0, it.bx1, it.by0,
                             it.by1, sw, sh, reserve);
     }
     r = rn;
@@ -962,37 +1146,40 @@ __device__ __forceinline__ void stage_bin(const BatchArgs& a, int vb, int nvb) {
 }
 
 
-// Row pre-pass: one lane per row task of an item with edge checkpoints (a
-// triangle at least kCkptMinSpan pixels wide spanning several tile
-// columns): walk the row once from the bbox's left column (Renderer.cpp:
-// 240-243) and store the two edge values where it enters each later tile
-// column.  The raster starts such rows from these checkpoints and shading
-// from the one of its pixel's tile column: the same serial chain of
-// additions as one walk from the left column, done once per row instead of
-// once per (row, tile column).  Tasks sit in kCkptSegs segments; a
-// wavefront takes 64 consecutive tasks of one segment.
+// Row pre-pass: one lane per row task of an item with edge checkpoints:
+// walk the row once from the bbox's left column (Renderer.cpp:240-243) and
+// store the two edge values where it enters each later checkpoint column.
+// The raster starts such rows from the checkpoint at or left of its tile and
+// shading from the one of its pixel: the same serial chain of additions as
+// one walk from the left column, done once per row instead of once per (row,
+// tile column).  Tasks sit in the segments; a wavefront takes 64 consecutive
+// tasks of one: first the small segments' in turn, then the large one's.
 __device__ __forceinline__ void stage_rows(const BatchArgs& a, int vb, int nvb) {
   const int lane = threadIdx.x & 63;
   const int sw = __ffs(a.tile_w) - 1;
-  const u64 seg_rows = (a.ckpt_cap / kCkptSegs) / 2;
-  // Tasks per segment (lane s holds segment s) and the largest count.
-  const u64 mine = min(a.ckpt_ctr[lane * kCtrStride] >> 40, seg_rows);
+  if (a.counters[kWidePx] == 0ull) return;
+  const int cs = ckpt_shift(a, sw);
+  // Tasks per small segment (lane s holds segment s) and the largest count.
+  const u64 mine = min(a.ckpt_ctr[lane * kCtrStride] >> 40, ckpt_seg(a, 0).rows_cap);
+  const u64 large = min(a.ckpt_ctr[kCkptBigRows], ckpt_seg(a, kCkptSegs).rows_cap);
   u64 most = mine;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) most = max(most, (u64)__shfl_xor(most, o));
   const u64 nw = (u64)nvb * 4;
-  for (u64 u = (u64)vb * 4 + (threadIdx.x >> 6); (u / kCkptSegs) * 64 < most; u += nw) {
-    const int seg = (int)(u % kCkptSegs);
-    const u64 first = (u / kCkptSegs) * 64;
-    const u64 count = __shfl(mine, seg);
+  const u64 units = (most + 63) / 64 * kCkptSegs, all = units + (large + 63) / 64;
+  for (u64 u = (u64)vb * 4 + (threadIdx.x >> 6); u < all; u += nw) {
+    const bool big = u >= units;
+    const int seg = big ? kCkptSegs : (int)(u % kCkptSegs);
+    const u64 first = (big ? u - units : u / kCkptSegs) * 64;
+    const u64 count = big ? large : (u64)__shfl(mine, seg & 63);
     if (first >= count) continue;
     const u64 t = first + lane;
-    const u64 task = t < count ? a.ckpt_rows[(u64)seg * seg_rows + t] : ~0ull;
+    const u64 task = t < count ? a.ckpt_rows[ckpt_seg(a, seg).rows_first + t] : ~0ull;
     if (task == ~0ull) continue;
     const BinItem it = a.items[task >> 32];
     const int row = (int)(uint32_t)task;
     const int64_t g = it.id >> 1;
-    const DrawDesc& D = a.draws[it.draw];
+    const DrawDesc& D = a.draws[it.draw & ~kDirectFlag];
     TriSetup s;
     tri_setup_sub(a, D, a.jobs[D.job], (int)(g - D.tri_begin), (int)(it.id & 1u), s);
     const int2 cb = a.ckpt_base[it.id];
@@ -1000,10 +1187,10 @@ __device__ __forceinline__ void stage_rows(const BatchArgs& a, int vb, int nvb) 
     edge_start(s.n1x, s.n1y, s.n2x, s.n2y, s.p0x, s.p0y, s.p2x, s.p2y, (float)s.bx0 + 0.5f,
                (float)row + 0.5f, e1, e2);
     int c = s.bx0;
-    float2* out = a.ckpt + ((int64_t)cb.x + (int64_t)row * cb.y);
-    for (int tx = (s.bx0 >> sw) + 1; tx <= (s.bx1 >> sw); tx++) {
-      advance2(e1, s.n1x, e2, s.n2x, (tx << sw) - c);
-      c = tx << sw;
+    float2* out = a.ckpt + ((int64_t)cb.x + (int64_t)row * (cb.y & 0xFFFF));
+    for (int tx = (s.bx0 >> cs) + 1; tx <= (s.bx1 >> cs); tx++) {
+      advance2(e1, s.n1x, e2, s.n2x, (tx << cs) - c);
+      c = tx << cs;
       out[tx] = make_float2(e1, e2);
     }
   }
@@ -1015,6 +1202,8 @@ __device__ __forceinline__ void stage_rows(const BatchArgs& a, int vb, int nvb) 
 __device__ __forceinline__ void stage_ckpt(const BatchArgs& a, int vb, int nvb) {
   const int lane = threadIdx.x & 63;
   const int sw = __ffs(a.tile_w) - 1;
+  if (a.counters[kWidePx] == 0ull) return;
+  const int cs = ckpt_shift(a, sw);
   const int64_t nw = (int64_t)nvb * 4;
   int64_t r = (int64_t)vb * 4 + (threadIdx.x >> 6);
   uint32_t cnt = r < a.nregions ? a.region_count[r] : 0u;
@@ -1024,30 +1213,179 @@ __device__ __forceinline__ void stage_ckpt(const BatchArgs& a, int vb, int nvb) 
     for (uint32_t j = 0; j < cnt; j += 64) {
       const bool act = j + lane < cnt;
       const BinItem it = act ? a.items[r * kRegion + j + lane] : BinItem{0, 0, 0, 0, 0, 0};
-      ckpt_alloc(a, act, it, sw, (uint32_t)(r * kRegion + j + lane), vb);
+      ckpt_alloc(a, act, it, sw, cs, (uint32_t)(r * kRegion + j + lane), vb);
     }
     r = rn;
     cnt = cnt_n;
   }
 }
 
+// Direct entries: the (id, draw) pairs of each tile's direct items, written
+// from the end of the bin list downwards.  A workgroup takes kDirectStep
+// consecutive tiles, each by eight lanes that test an eighth of the job's list
+// each, kDirectGroup items at a time: these pass through LDS, whose reads
+// every half wavefront shares, and a lane keeps its hits as bits until its
+// tiles' entries are counted and allocated (by one atomic per workgroup).
+// With one group in all the hits are written from there, else it is tested
+// again.  A tile's range goes to the word behind its pair count (zero for
+// tiles without direct entries).  The steps of a few lists are what a launch
+// waits for: testing 600 items took 20 us with 256 at a time and two passes.
+constexpr int kDirectStep = 32;
+constexpr int kDirectGroup = 1024;
+__device__ __forceinline__ void stage_direct(const BatchArgs& a, int vb, int nvb) {
+  if (a.counters[kDirect] == 0ull) return;
+  constexpr int kMasks = kDirectGroup / 256;  // per lane: 32 items each
+  __shared__ uint4 list[kDirectGroup];
+  __shared__ uint32_t cnt[8][kDirectStep];
+  __shared__ uint32_t first[kDirectStep];
+  const int tid = threadIdx.x, lt = tid % kDirectStep, part = tid / kDirectStep;
+  const int64_t step = (int64_t)nvb * kDirectStep;
+  for (int64_t t0 = (int64_t)vb * kDirectStep; t0 < a.ntiles; t0 += step) {
+    const int t = (int)t0 + lt;
+    const int t_end = (int)min(t0 + kDirectStep, (int64_t)a.ntiles);
+    const int j0 = job_lookup(a.tile_hint, a.job_tile_base, a.njobs, t0);
+    int groups = 0;    // of the lists of the jobs here
+    bool own = false;  // this tile's job has a list
+    for (int j = j0; j < a.njobs && a.job_tile_base[j] < t_end; j++) {
+      const int nd = (int)min(a.direct_count[(size_t)j * kCtrStride], a.direct_cap);
+      groups += (nd + kDirectGroup - 1) / kDirectGroup;
+      if (t >= a.job_tile_base[j]) own = nd != 0;
+    }
+    if (groups == 0) continue;
+    own = own && t < t_end;
+    uint32_t n = 0, slot = 0;
+    bool room = true;
+    uint32_t mask[kMasks] = {};
+    for (int pass = 0; pass < 2; pass++) {
+      // (The tiles usually lie in one job.)
+      for (int j = j0; j < a.njobs && a.job_tile_base[j] < t_end; j++) {
+        const uint32_t* const line = a.direct_count + (size_t)j * kCtrStride;
+        const int nd = (int)min(line[0], a.direct_cap);
+        if (nd == 0) continue;
+        const JobDesc& J = a.jobs[j];
+        const int local = t - J.tile_base;
+        const bool mine = t < t_end && local >= 0 && local < J.tiles_x * J.tiles_y;
+        const int ty = local / J.tiles_x, tx = local - ty * J.tiles_x;
+        const int x0 = tx * a.tile_w, y0 = ty * a.tile_h;
+        const int x1 = x0 + a.tile_w - 1, y1 = y0 + a.tile_h - 1;
+        const uint4* const src = (const uint4*)(a.direct + (size_t)j * a.direct_cap);
+        for (int i0 = 0; i0 < nd; i0 += kDirectGroup) {
+          if (pass == 0 || groups > 1) {
+#pragma unroll
+            for (int m = 0; m < kMasks; m++) {
+              const int i = i0 + m * 256 + tid;
+              if (i0 + m * 256 < nd)  // items past the list meet no tile
+                list[m * 256 + tid] = i < nd ? src[i] : make_uint4(0u, 0u, 0xFFFFu, 0xFFFFu);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < kMasks; m++) {
+              mask[m] = 0;
+              if (!mine || i0 + m * 256 >= nd) continue;
+#pragma unroll 8
+              for (int i = 0; i < 32; i++) {
+                const uint4 it = list[m * 256 + 8 * i + part];  // {id, draw, columns, rows}
+                const bool hit = x1 >= (int)(it.z & 0xFFFFu) && x0 <= (int)(it.z >> 16) &&
+                                 y1 >= (int)(it.w & 0xFFFFu) && y0 <= (int)(it.w >> 16);
+                mask[m] |= (hit ? 1u : 0u) << i;
+              }
+            }
+          }
+#pragma unroll
+          for (int m = 0; m < kMasks; m++) {
+            if (pass == 0) {
+              n += (uint32_t)__popc(mask[m]);
+            } else if (room) {
+              for (uint32_t b = mask[m]; b; b &= b - 1) {
+                const uint4 it = list[m * 256 + 8 * (__ffs(b) - 1) + part];
+                a.bins[slot++] = make_uint2(it.x, it.y);
+              }
+            }
+          }
+          if (groups > 1) __syncthreads();  // the list is loaded again
+        }
+      }
+      if (pass) break;
+      cnt[part][lt] = n;
+      __syncthreads();
+      uint32_t before = 0, total = 0;
+#pragma unroll
+      for (int w = 0; w < 8; w++) {
+        if (w < part) before += cnt[w][lt];
+        total += cnt[w][lt];
+      }
+      if (tid < 64) {  // (lanes 32..63 see the same tiles and add nothing)
+        uint32_t P = tid < kDirectStep ? total : 0u;  // inclusive prefix over the tiles
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const uint32_t y = __shfl_up(P, o);
+          if (tid >= o) P += y;
+        }
+        const uint32_t all = __shfl(P, 63);
+        u64 pos = 0;
+        if (tid == 0 && all) pos = atomicAdd(&a.counters[kDirectPairs], (u64)all);
+        pos = __shfl(pos, 0);
+        const bool fits = pos + all <= a.bins_cap;  // else binning flags the overflow
+        if (tid < kDirectStep) {
+          first[tid] = fits ? (uint32_t)(a.bins_cap - pos - all) + P - total : 0xFFFFFFFFu;
+          if (own && total && fits)
+            a.tile_count[(size_t)t * kCtrStride64 + 1] = ((u64)total << 32) | first[tid];
+        }
+        // Tiles without pairs: those with direct entries are listed for the
+        // raster from the end of its list, the others are empty.
+        const bool bare = tid < kDirectStep && own &&
+                          (uint32_t)a.tile_count[(size_t)t * kCtrStride64] == 0u;
+        const u64 lm = __ballot(bare && total > 0);
+        u64 at = 0;
+        if (tid == 0 && lm) at = atomicAdd(&a.counters[kDirectTilesListed], (u64)__popcll(lm));
+        at = __shfl(at, 0) + __popcll(lm & ((1ull << tid) - 1ull));
+        if (bare && total > 0)
+          a.tile_list[a.ntiles - 1 - (int64_t)at] = make_uint4((uint32_t)t, 0u, 0u, 1u);
+        if (bare) a.tile_heavy[t] = total > 0 ? kNoSlot : kEmptyTile;
+      }
+      __syncthreads();
+      room = first[lt] != 0xFFFFFFFFu;
+      slot = first[lt] + before;
+    }
+    __syncthreads();  // cnt, first and the list are used again
+  }
+}
+
+// The bin list holds the scan's pairs from its start and the direct pairs
+// from its end: more than it holds is an overflow.  Run by one thread after
+// both are known and before the raster.
+__device__ inline void check_direct_room(const BatchArgs& a) {
+  const u64 direct = a.counters[kDirectPairs];
+  if (direct == 0ull) return;
+  a.counters[kBinEntries] += direct;
+  if (a.counters[kBinEntries] > a.bins_cap) atomicOr(&a.counters[kBinOverflow], 1ull);
+}
+
 // The scan's workgroups first, then (ckpt_in_scan) the checkpoint
-// allocation's, which needs only geometry's items and so runs beside the
-// scan: one launch for both.
+// allocation's and the direct entries', which need only geometry's items and
+// so run beside the scan: one launch for all.
 __global__ __launch_bounds__(kScanBlock) void k_scan(BatchArgs a) {
-  static_assert(kScanBlock == 256, "the checkpoint pass runs in workgroups of 256");
-  if ((int)blockIdx.x < a.scan_blocks) stage_scan(a);
-  else stage_ckpt(a, (int)blockIdx.x - a.scan_blocks, (int)gridDim.x - a.scan_blocks);
+  static_assert(kScanBlock == 256, "the other passes run in workgroups of 256");
+  const int nd = direct_grid(a);
+  const int b = (int)blockIdx.x - a.scan_blocks;
+  if (b < 0) stage_scan(a);
+  else if (b < nd) stage_direct(a, b, nd);
+  else stage_ckpt(a, b - nd, (int)gridDim.x - a.scan_blocks - nd);
 }
 
 // Binning that takes the checkpoints (k_rows walks them next), and binning
 // followed by the row pre-pass of the row tasks the scan's launch wrote
 // (ckpt_in_scan): kernels of their own, each with only its own code.
 __global__ __launch_bounds__(256, 7) void k_bin(BatchArgs a) {
-  stage_bin<true>(a, blockIdx.x, gridDim.x);
+  // (The allocation's registers spill: a batch without wide triangles runs
+  // the loop without it.)
+  if (blockIdx.x == 0 && threadIdx.x == 0) check_direct_room(a);
+  if (a.counters[kWidePx] == 0ull) stage_bin<false>(a, blockIdx.x, gridDim.x);
+  else stage_bin<true>(a, blockIdx.x, gridDim.x);
 }
 
 __global__ __launch_bounds__(256, 7) void k_bin_rows(BatchArgs a) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) check_direct_room(a);
   stage_bin<false>(a, blockIdx.x, gridDim.x);
   stage_rows(a, blockIdx.x, gridDim.x);
 }
@@ -1067,11 +1405,28 @@ __device__ inline void raster_pixel(u64* keys, int p, float e1, float e2, float 
   if (key < keys[p]) atomicMin(&keys[p], key);
 }
 
+constexpr int kCoverRowsMin = 4;  // wide entries of a wavefront from which rows are tested
+
+// Raster work items of the batch: parts and row bands, and tiles rastered
+// whole (those with bin entries, then those with direct entries only).
+struct TileItems {
+  int64_t parts, whole, listed;
+};
+__device__ inline TileItems tile_items(const BatchArgs& a) {
+  TileItems r;
+  // After a merge-slot or part-list overflow the part list is incomplete:
+  // split tiles are then skipped (the frame is re-run with larger buffers).
+  r.parts = a.counters[kHeavyOverflow] ? 0 : (int64_t)min(a.counters[kParts], (u64)a.parts_cap);
+  r.whole = (int64_t)min(a.counters[kListed], (u64)a.ntiles);
+  r.listed = min(r.whole + (int64_t)a.counters[kDirectTilesListed], (int64_t)a.ntiles);
+  return r;
+}
+
 // (d): one workgroup per raster work item: first the parts of split tiles
-// (listed by the scan), then every tile.  The grid has parts_cap + ntiles
-// workgroups; workgroups past the actual number of items exit at once.
-// remap: listed tiles in XCD-interleaved order (own launch, where
-// consecutive workgroups go to different XCDs), else in list order.
+// (listed by the scan), then every tile rastered whole.  The grid has
+// parts_cap + ntiles workgroups; workgroups past the actual number of items
+// exit at once.  remap: listed tiles in XCD-interleaved order (own launch,
+// where consecutive workgroups go to different XCDs), else in list order.
 template <int TW, int TH, int NT>
 __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool remap) {
   constexpr int NP = TW * TH;
@@ -1085,14 +1440,13 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
   __shared__ int wave_rows[NT / 64];
   __shared__ int sh_last;
   const int tid = threadIdx.x;
-  // After a merge-slot or part-list overflow the part list is incomplete:
-  // split tiles are then skipped (the frame is re-run with larger buffers).
-  const int64_t nparts_all =
-      a.counters[kHeavyOverflow] ? 0 : (int64_t)min(a.counters[kParts], (u64)a.parts_cap);
+  bool direct = a.counters[kDirect] != 0ull;
+  const TileItems items = tile_items(a);
+  if (b >= items.parts + items.listed) return;
   int tile, part;
   uint32_t cnt, off;  // the tile's bin entries: number and first
   int band_lo = 0, band_hi = TH - 1;  // tile rows of this work item
-  if (b < nparts_all) {
+  if (b < items.parts) {
     const uint2 pp = a.parts[b];
     tile = (int)pp.x;
     part = (int)pp.y;
@@ -1109,36 +1463,46 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     // Tiles rastered whole come from the scan's list, with their bin range
     // (one load fewer before the bin entries); tiles without bin entries
     // are not in it (shading writes their background).
-    const int64_t t = b - nparts_all;
-    const int64_t nlisted = (int64_t)min(a.counters[kListed], (u64)a.ntiles);
-    if (t >= nlisted) return;
-    const uint4 le = a.tile_list[remap ? xcd_remap(t, nlisted) : t];
+    // (Tiles with direct entries only are listed from the end.)
+    const int64_t t = b - items.parts;
+    const int64_t li = remap ? xcd_remap(t, items.listed) : t;
+    const uint4 le = a.tile_list[li < items.whole ? li : a.ntiles - 1 - (li - items.whole)];
     tile = (int)le.x;
     part = 0;
     off = le.y;
     cnt = le.z;
+    direct = le.w != 0;  // the tile's job has direct items
   }
   {
     const uint32_t nparts = cnt <= a.frag_size ? 1u : (cnt + a.frag_size - 1) / a.frag_size;
-    if (b >= nparts_all && nparts > 1) return;  // rendered through its parts
     const int j = job_lookup(a.tile_hint, a.job_tile_base, a.njobs, tile);
     const JobDesc& J = a.jobs[j];
     const bool persp = J.persp != 0;
     const int local = tile - J.tile_base;
     const int tyi = local / J.tiles_x, txi = local - tyi * J.tiles_x;
     const int x0 = txi * TW, y0 = tyi * TH;
-    for (int p = tid; p < TH * KS; p += NT) keys[p] = ~0ull;
     uint32_t avail = cnt;  // entries actually written (bin-list overflow)
     if ((u64)off >= a.bins_cap) avail = 0;
     else if ((u64)off + cnt > a.bins_cap) avail = (uint32_t)(a.bins_cap - off);
     const uint32_t e_begin = (uint32_t)part * a.frag_size;
     const uint32_t e_end = min(avail, e_begin + a.frag_size);
+    // The entries: the bin entries, then (by the first part of a split tile)
+    // the direct ones.
+    const uint32_t nbin = e_end > e_begin ? e_end - e_begin : 0u;
+    uint32_t nall = nbin, off2 = 0;
+    if (direct && part == 0) {
+      const u64 range = a.tile_count[(size_t)tile * kCtrStride64 + 1];
+      off2 = (uint32_t)range - nbin;
+      nall += (uint32_t)(range >> 32);
+    }
+    for (int p = tid; p < TH * KS; p += NT) keys[p] = ~0ull;
     __syncthreads();
-    for (uint32_t base = e_begin; base < e_end; base += NT) {
+    for (uint32_t base = 0; base < nall; base += NT) {
       // One lane per entry: setup, and the tile rows it covers.
       int nrows = 0;
-      if (base + tid < e_end) {
-        const uint2 be = a.bins[off + base + tid];
+      const uint32_t q0 = base + tid;
+      if (q0 < nall) {
+        const uint2 be = a.bins[q0 + (q0 < nbin ? off + e_begin : off2)];
         const uint32_t id = be.x;
         const int64_t g = id >> 1;
         TriSetup s;
@@ -1150,7 +1514,15 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
           const DrawDesc& D = a.draws[be.y];
           tri_setup_sub(a, D, J, (int)(g - D.tri_begin), (int)(id & 1u), s);
         }
-        nrows = max(min(s.by1, y0 + band_hi) - max(s.by0, y0 + band_lo) + 1, 0);
+        // Rows of this item, without those it covers no pixel of (a triangle
+        // no wider than the tile covers pixels in nearly all of its rows, and
+        // the test pays for a few wide ones in the wavefront at least).
+        int r0 = max(s.by0, y0 + band_lo), r1 = min(s.by1, y0 + band_hi);
+        const bool wide = s.bx1 - s.bx0 >= TW && r1 >= r0;
+        if (__popcll(__ballot(wide)) >= kCoverRowsMin && wide)
+          cover_rows(s, max(s.bx0, x0), min(s.bx1, x0 + TW - 1), r0, r1);
+        nrows = max(r1 - r0 + 1, 0);
+        s.by0 = r0;  // the first row taken
         setups[tid] = s;
         setup_id[tid] = id;
       }
@@ -1177,29 +1549,31 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
       for (int q = tid; q < total; q += NT) {
         const int i = owner_search<NT>(row_start, q);
         const TriSetup& s = setups[i];
-        const int row = max(s.by0, y0 + band_lo) + (q - row_start[i]);
+        const int row = s.by0 + (q - row_start[i]);
         const int cx0 = max(s.bx0, x0), cx1 = min(s.bx1, x0 + TW - 1);
         const uint32_t id = setup_id[i];
         // A row entering a tile column after its triangle's first starts
-        // from the edge checkpoint the row pre-pass left there (the same
-        // serial chain from the bbox's left column); without checkpoints
+        // from the edge checkpoint the row pre-pass left at or before it (the
+        // same serial chain from the bbox's left column); without checkpoints
         // (none allocated) it walks from the left column itself.
         float e1 = 0.0f, e2 = 0.0f;
-        bool from_ckpt = false;
+        int steps = -1;
         if (cx0 > s.bx0 && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {  // only these have any
           const int2 cb = a.ckpt_base[id];
-          if (cb.y) {
-            const float2 st = a.ckpt[(int64_t)cb.x + (int64_t)row * cb.y + x0 / TW];
+          const int cs = cb.y >> 16, col = x0 >> cs;
+          if (cb.y && col > (s.bx0 >> cs)) {
+            const float2 st = a.ckpt[(int64_t)cb.x + (int64_t)row * (cb.y & 0xFFFF) + col];
             e1 = st.x;
             e2 = st.y;
-            from_ckpt = true;
+            steps = x0 - (col << cs);
           }
         }
-        if (!from_ckpt) {
+        if (steps < 0) {
           edge_start(s.n1x, s.n1y, s.n2x, s.n2y, s.p0x, s.p0y, s.p2x, s.p2y,
                      (float)s.bx0 + 0.5f, (float)row + 0.5f, e1, e2);
-          advance2(e1, s.n1x, e2, s.n2x, cx0 - s.bx0);
+          steps = cx0 - s.bx0;
         }
+        advance2(e1, s.n1x, e2, s.n2x, steps);
         // The triangle's steps and depths in registers for the row: read from
         // the workgroup's setup table once, not again after each key update.
         const float n1x = s.n1x, n2x = s.n2x, z0 = s.z0, z1 = s.z1, z2 = s.z2;
@@ -1310,7 +1684,6 @@ __device__ __forceinline__ void shade_lit(const BatchArgs& a, const JobDesc& J, 
   const auto* ip = G(D.idx) + 3 * tri;
   const auto* in = G(D.nidx) + 3 * tri;
   const int sw = __ffs(a.tile_w) - 1;
-  const int ctx = c >> sw;
   const int i0 = ip[0], i1 = ip[1], i2 = ip[2];
   // Normal and texcoord indices that share the position index buffer are
   // not loaded again.
@@ -1365,27 +1738,28 @@ __device__ __forceinline__ void shade_lit(const BatchArgs& a, const JobDesc& J, 
   else
     setup_edges((float)J.W, vc[0], vc[1], vc[2], s);
   // Edge values at the pixel, from the same serial walk along the row as the
-  // raster's: from the row pre-pass's checkpoint where the row enters the
-  // pixel's tile column, or from the bbox's left column.  Only triangles at
+  // raster's: from the row pre-pass's checkpoint at or left of the
+  // pixel, or from the bbox's left column.  Only triangles at
   // least kCkptMinSpan pixels wide can have checkpoints (the raster's test):
   // the others read no checkpoint base.
   float e1 = 0.0f, e2 = 0.0f;
-  bool from_ckpt = false;
-  if (ctx > (s.bx0 >> sw) && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {
+  int steps = -1;
+  if ((c >> sw) > (s.bx0 >> sw) && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {
     const int2 cb = a.ckpt_base[id];
-    if (cb.y) {
-      const float2 st = a.ckpt[(int64_t)cb.x + (int64_t)row * cb.y + ctx];
+    const int cs = cb.y >> 16, col = c >> cs;
+    if (cb.y && col > (s.bx0 >> cs)) {
+      const float2 st = a.ckpt[(int64_t)cb.x + (int64_t)row * (cb.y & 0xFFFF) + col];
       e1 = st.x;
       e2 = st.y;
-      advance2(e1, s.n1x, e2, s.n2x, c - (ctx << sw));
-      from_ckpt = true;
+      steps = c - (col << cs);
     }
   }
-  if (!from_ckpt) {
+  if (steps < 0) {
     edge_start(s.n1x, s.n1y, s.n2x, s.n2y, s.p0x, s.p0y, s.p2x, s.p2y,
                (float)s.bx0 + 0.5f, (float)row + 0.5f, e1, e2);
-    advance2(e1, s.n1x, e2, s.n2x, c - s.bx0);
+    steps = c - s.bx0;
   }
+  advance2(e1, s.n1x, e2, s.n2x, steps);
   float k[3];
   const float z = depth_of(e1, e2, s.z0, s.z1, s.z2, J.persp != 0, k);
   if (!J.rgb8 && !J.rgb && !(J.normals && J.save_normals)) {
@@ -1622,6 +1996,7 @@ __device__ __forceinline__ void stage_shade(const BatchArgs& a, int vb, bool rem
        i += (int64_t)a.shade_blocks * kShadeBlock) {
     if (i < a.ntiles) {
       a.tile_count[(size_t)i * kCtrStride64] = 0;
+      a.tile_count[(size_t)i * kCtrStride64 + 1] = 0;
       a.tile_done[i] = 0;
     }
     if (i < a.scan_blocks) a.scan_status[i] = 0;
@@ -1668,10 +2043,8 @@ __device__ inline u64 ctl_load(const u64* p) {
 // grid of its own launch is a bound, whose workgroups past the count exit).
 __device__ inline int64_t persist_stage_size(const BatchArgs& a, const PersistPlan& q, int s) {
   if (s != kPTile) return q.nvb[s];
-  const int64_t nparts_all =
-      a.counters[kHeavyOverflow] ? 0 : (int64_t)min(a.counters[kParts], (u64)a.parts_cap);
-  const int64_t nlisted = (int64_t)min(a.counters[kListed], (u64)a.ntiles);
-  return min((int64_t)q.nvb[s], nparts_all + nlisted);
+  const TileItems items = tile_items(a);
+  return min((int64_t)q.nvb[s], items.parts + items.listed);
 }
 
 // Queue x's share of a stage of n workgroups: first workgroup, count, and
@@ -1725,8 +2098,14 @@ __device__ __forceinline__ void persist_run(const BatchArgs& a, const PersistPla
     case kPVertex: stage_vertex(a, (int)vb, q.nvb[s]); break;
     case kPGeom: stage_geom(a, (int)vb, q.nvb[s]); break;
     case kPScan: stage_scan(a); break;
-    case kPBin: stage_bin<true>(a, (int)vb, q.nvb[s]); break;
-    case kPRows: stage_rows(a, (int)vb, q.nvb[s]); break;
+    case kPBin:
+      stage_direct(a, (int)vb, q.nvb[s]);
+      stage_bin<true>(a, (int)vb, q.nvb[s]);
+      break;
+    case kPRows:
+      if (vb == 0 && threadIdx.x == 0) check_direct_room(a);
+      stage_rows(a, (int)vb, q.nvb[s]);
+      break;
     case kPTile: stage_tile<TW, TW, 256>(a, vb, false); break;
     default: stage_shade(a, (int)vb, false); break;
   }
@@ -1971,7 +2350,8 @@ hipError_t launch_geometry(const BatchArgs& a, hipStream_t s) {
 
 hipError_t launch_scan(const BatchArgs& a, hipStream_t s) {
   const int32_t ckpt_blocks = a.ckpt_in_scan ? bin_grid(a) : 0;
-  hipLaunchKernelGGL(k_scan, dim3(a.scan_blocks + ckpt_blocks), dim3(kScanBlock), 0, s, a);
+  hipLaunchKernelGGL(k_scan, dim3(a.scan_blocks + direct_grid(a) + ckpt_blocks), dim3(kScanBlock), 0,
+                     s, a);
   return hipGetLastError();
 }
 

@@ -11,16 +11,26 @@ namespace mr {
 struct BatchArgs {
   BinItem* items;            // [nregions * kRegion] survivors, per wavefront
   uint32_t* region_count;    // [nregions] survivors of each wavefront
+  // Direct items of each job, and per job a line of words: their number
+  // (which may exceed the list), then kMaxDim - first column, last column,
+  // kMaxDim - first row and last row of their bounding box.  Both lie behind
+  // the checkpoints, in the checkpoint buffer's last quarter.
+  BinItem* direct;           // [njobs * direct_cap]
+  uint32_t* direct_count;    // [njobs * kCtrStride], null when direct_cap is 0
+  uint32_t direct_cap;
   int64_t nregions;
   // [ntiles * kCtrStride64] per tile: (walk work << 32) | (tile, triangle)
   // pairs, where a pair's walk work is its bbox pixels in the tile + 4 per
-  // row + 16 (for the group leader's pair, times the group size)
+  // row + 16 (for the group leader's pair, times the group size); in the next
+  // word, (direct entries << 32) | the first one's place in the bin list
   unsigned long long* tile_count;
   uint32_t* tile_off;        // [ntiles] exclusive scan of the pair counts
-  uint32_t* tile_cursor;     // [ntiles] scatter cursors
+  uint32_t* tile_cursor;     // [ntiles * kCtrStride] scatter cursors
   uint32_t* tile_heavy;      // [ntiles] merge slot of a split tile, kNoSlot, or kEmptyTile
-  uint4* tile_list;          // [ntiles] {tile, first bin entry, entries, 0} of the tiles
-                             // rastered whole (first counters[kListed])
+  uint4* tile_list;          // [ntiles] {tile, first bin entry, entries, 1 if its job
+                             // has direct items} of the tiles rastered whole: from the
+                             // start those with entries (counters[kListed]), from the end
+                             // those with direct entries only (kDirectTilesListed)
   uint32_t* tile_done;       // [ntiles] finished parts of a split tile
   uint2* parts;              // [parts_cap] (tile, part) of split tiles
   uint32_t parts_cap;
@@ -29,18 +39,18 @@ struct BatchArgs {
   // Edge checkpoints: the edge values of each row of a triangle spanning
   // several tile columns where the row enters each of them after the first
   // (written by the row pre-pass, read by the raster and shading).
-  // Checkpoint of (row, tile
-  // column tx) of a survivor id: ckpt[ckpt_base[id].x + row *
-  // ckpt_base[id].y + tx], with .x a signed offset (the entries of the first
-  // column are allocated, never written); .y == 0: no checkpoints.
+  // Checkpoint of (row, column k of 2^cs pixels) of a survivor id, with
+  // .y = columns | cs << 16: ckpt[ckpt_base[id].x + row * columns + k], with
+  // .x a signed offset (the entries of the first column are allocated, never
+  // written); .y == 0: no checkpoints.
   int2* ckpt_base;           // [2 * total_tris]
   float2* ckpt;              // [ckpt_cap], kCkptSegs equal segments
   uint64_t ckpt_cap;
   unsigned long long* ckpt_ctr;  // [kCkptSegs * kCtrStride] segment fill counters
   // Row tasks of the row pre-pass, (item index << 32) | pixel row, in
-  // kCkptSegs segments of (ckpt_cap / kCkptSegs) / 2 (a task per row of an
+  // segments of half as many as the checkpoints' (a task per row of an
   // item with checkpoints, each row holding two entries or more); the
-  // segment counters ckpt_ctr count them in their high 24 bits.
+  // small segments' counters ckpt_ctr count them in their high 24 bits.
   unsigned long long* ckpt_rows;
   unsigned long long* heavy_keys;  // [heavy_cap * tile pixels] merge buffers
   uint32_t heavy_cap;
@@ -114,10 +124,20 @@ __host__ __device__ inline int32_t geom_grid(const BatchArgs& a) {
   return (int32_t)(blocks < g ? blocks : g);
 }
 __host__ __device__ inline int32_t bin_grid(const BatchArgs& a) {
+  // (At least a workgroup per 2048 pixels: the row pre-pass at the end has
+  // many rows of few large triangles.)
   int64_t blocks = (a.nregions + 3) / 4;
+  if (blocks < a.shade_blocks / 8) blocks = a.shade_blocks / 8;
   if (blocks < 1) blocks = 1;
   const int64_t cap = (int64_t)a.num_cus * 7;  // one resident round (7 per CU)
   return (int32_t)(blocks < cap ? blocks : cap);
+}
+
+// Workgroups that write the direct entries, 32 tiles a step each.
+__host__ __device__ inline int32_t direct_grid(const BatchArgs& a) {
+  if (a.direct_cap == 0) return 0;
+  const int32_t steps = (a.ntiles + 31) / 32;
+  return steps < 1024 ? steps : 1024;
 }
 
 hipError_t launch_clear(const BatchArgs& a, hipStream_t s);

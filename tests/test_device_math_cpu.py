@@ -11,6 +11,9 @@ reference's, built with g++ from the same headers the HIP kernels use.
                  the bbox end bound last_center equals the last pixel of the
                  reference's fp32 loop x <= pmax + 0.5f (Renderer.cpp:238,243)
                  near every power of two from 2 to 16384.
+  rows_check     no row that cover_rows (exact.h) drops for a tile covers a
+                 pixel there in the raster's serial walk (Renderer.cpp:
+                 238-245), and it drops most of the rows that cover none.
 """
 import subprocess
 from pathlib import Path
@@ -47,5 +50,13 @@ def test_ff_matches_serial(ff_bin, seed):
 
 def test_remap_and_clip(helpers_bin):
     r = subprocess.run([str(helpers_bin), "300000"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip() == "ok"
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_cover_rows_is_conservative(tmp_path_factory, seed):
+    rows_bin = _build(tmp_path_factory, "rows_check")
+    r = subprocess.run([str(rows_bin), "1000000", str(seed)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.strip() == "ok"
