@@ -60,6 +60,7 @@ struct JobDesc {
   int32_t lighting;
   int32_t save_normals;
   int32_t shade_base;  // first shading block of this job
+  int64_t tri_begin, tri_end;  // flat triangles of this job in the batch
   uint32_t* win;       // device scratch: draw-order id of each pixel's winner
   uint8_t* rgb8;       // device outputs (any may be null)
   float* depth;
@@ -116,6 +117,25 @@ MR_HD inline int64_t xcd_remap(int64_t b, int64_t n) {
   const int64_t x = b % kXcds, k = b / kXcds;
   return x * q + (x < rem ? x : rem) + k;
 }
+
+// The same with each XCD owning every eighth chunk of `kChunk` consecutive
+// items (the rest past the last whole round of chunks as it comes): chunks of
+// neighbouring pixels still share an L2, and work that changes over the frame
+// (sky above, ground below) is dealt to all XCDs alike.  kChunk a power of
+// two: a division by a variable costs every workgroup more than it gains.
+template <uint32_t kChunk>
+MR_HD inline uint32_t xcd_chunks(uint32_t b, uint32_t n) {
+  constexpr uint32_t kXcds = 8, kRound = kXcds * kChunk;
+  if (b >= n / kRound * kRound) return b;
+  const uint32_t x = b % kXcds, k = b / kXcds;
+  return (k / kChunk * kXcds + x) * kChunk + k % kChunk;
+}
+
+// Chunk of the raster's and shading's work, tiles or blocks.  Measured against
+// one range per XCD: raster 108 -> 67 us on the textured 1080p terrain, 140 ->
+// 113 at 4K, shading 36 -> 31 and 121 -> 100 us, 339 -> 319 on a batch of 48
+// mixed frames; 4 and 64 alike on single frames, 64 slower on batches.
+constexpr uint32_t kXcdChunk = 16;
 
 // Per-tile counters are spread one per 64-byte line: the atomics of the
 // binner then spread over all memory channels instead of a few.

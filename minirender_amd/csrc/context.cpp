@@ -137,6 +137,8 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
   plan.ntiles = 0;
   plan.npixels = 0;
   plan.shade_blocks = 0;
+  plan.max_width = 0;
+  plan.small_tests = plan.max_regions = 0;
   const int tw = c->tile_w, th = c->tile_h;
   for (int j = 0; j < nframes; j++) {
     const mr_frame* f = &frames[j];
@@ -164,6 +166,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     plan.npixels += npix;
     if (plan.shade_blocks > 0x7FFFFFFF) return MR_ERR_ARG;
     J.draw_begin = (int32_t)plan.draws.size();
+    J.tri_begin = plan.total_tris;
     for (int i = 0; i < 3; i++) {
       J.bg[i] = f->background[i];
       J.light[i] = f->light[i];
@@ -240,12 +243,19 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     }
     if (order >= 0xFFFFFFFFull) return MR_ERR_ARG;
     J.draw_end = (int32_t)plan.draws.size();
+    J.tri_end = plan.total_tris;
+    plan.max_width = std::max(plan.max_width, J.W);
+    const int64_t regions = ((J.tri_end + 63) >> 6) - (J.tri_begin >> 6);
+    plan.max_regions = std::max(plan.max_regions, regions);
+    plan.small_tests += (int64_t)J.tiles_x * J.tiles_y * regions;
   }
   if (2 * plan.total_tris >= 0xFFFFFFFFll || plan.total_verts >= 0x7FFFFFFFll) return MR_ERR_ARG;
   // Job hints for the raster's and shading's job lookup: every kHintSpan-th
   // tile (block), its job and the next job's first tile (block).
+  // (One job needs none.)
   plan.hints.clear();
-  for (int k = 0; k < 2; k++) {
+  plan.tile_hints = 0;
+  for (int k = 0; k < 2 && nframes > 1; k++) {
     const int32_t* base = plan.job_bases.data() + (size_t)k * nframes;
     const int64_t n = k == 0 ? plan.ntiles : plan.shade_blocks;
     int j = 0;
@@ -379,12 +389,10 @@ static BatchArgs make_args(mr_ctx* c, Slot& sl, const BatchPlan& p) {
   const uint64_t nj = p.jobs.size();
   uint64_t ckpt_bytes = s.ckpt.bytes;
   const uint64_t per_job = ckpt_bytes / 4 / nj;
-  const uint64_t line = kCtrStride * 4;
-  if (per_job >= line + kDirectMin * sizeof(BinItem)) {
-    a.direct_cap = (uint32_t)std::min<uint64_t>((per_job - line) / sizeof(BinItem), kDirectCap);
-    ckpt_bytes = (ckpt_bytes - nj * (line + a.direct_cap * sizeof(BinItem))) & ~(uint64_t)255;
-    a.direct_count = (uint32_t*)((char*)s.ckpt.p + ckpt_bytes);
-    a.direct = (BinItem*)(a.direct_count + nj * kCtrStride);
+  if (per_job >= kDirectMin * sizeof(BinItem)) {
+    a.direct_cap = (uint32_t)std::min<uint64_t>(per_job / sizeof(BinItem), kDirectCap);
+    ckpt_bytes = (ckpt_bytes - nj * a.direct_cap * sizeof(BinItem)) & ~(uint64_t)255;
+    a.direct = (BinItem*)((char*)s.ckpt.p + ckpt_bytes);
   }
   // Checkpoint capacity, held to twice the row-task entries: the row tasks
   // of every item given checkpoints then fit in their segment.
@@ -428,10 +436,24 @@ static BatchArgs make_args(mr_ctx* c, Slot& sl, const BatchPlan& p) {
 }
 
 // persistent: every stage in one launch of the persistent kernel (profiling
-// then times the whole launch as stage 0).
+// then times the whole launch as stage 0).  tables: the batch tables in host
+// memory when the first kernel takes them in its argument.
 static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
-                         bool persistent, uint64_t wait_us) {
+                         bool persistent, uint64_t wait_us, const void* tables = nullptr,
+                         size_t table_bytes = 0) {
   hipStream_t st = s.stream;
+  if (a.small) {
+    s.last_launches = 2;
+    if (profile) HIP_TRY(hipEventRecord(s.ev[0], st));
+    if (profile) HIP_TRY(hipEventRecord(s.ev[1], st));
+    HIP_TRY(launch_front(a, tables, table_bytes, st));
+    if (profile)
+      for (int i = 2; i <= 5; i++) HIP_TRY(hipEventRecord(s.ev[i], st));
+    HIP_TRY(launch_small(a, st));
+    if (profile)
+      for (int i = 6; i <= kStages; i++) HIP_TRY(hipEventRecord(s.ev[i], st));
+    return MR_OK;
+  }
   if (persistent) {
     unsigned long long* ctl = (unsigned long long*)s.sc.ctl.p;
     unsigned long long* stamps = profile ? ctl + kCtlBytes / 8 : nullptr;
@@ -443,13 +465,17 @@ static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
     s.last_launches = 1;
     return MR_OK;
   }
-  s.last_launches = (clear ? 1 : 0) + (a.total_verts ? 1 : 0) + (a.total_tris ? 1 : 0) +
-                    (a.ckpt_in_scan ? 4 : 5);
+  s.last_launches = (clear ? 1 : 0) + (a.total_verts && !a.front ? 1 : 0) +
+                    (a.total_tris ? 1 : 0) + (a.ckpt_in_scan ? 4 : 5);
   if (profile) HIP_TRY(hipEventRecord(s.ev[0], st));
   if (clear) HIP_TRY(launch_clear(a, st));
   if (profile) HIP_TRY(hipEventRecord(s.ev[1], st));
-  HIP_TRY(launch_vertex(a, st));
-  HIP_TRY(launch_geometry(a, st));
+  if (a.front) {
+    HIP_TRY(launch_front(a, tables, table_bytes, st));
+  } else {
+    HIP_TRY(launch_vertex(a, st));
+    HIP_TRY(launch_geometry(a, st));
+  }
   if (profile) HIP_TRY(hipEventRecord(s.ev[2], st));
   HIP_TRY(launch_scan(a, st));
   if (profile) HIP_TRY(hipEventRecord(s.ev[3], st));
@@ -514,23 +540,43 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   }
   s.last_geom_grid = p.total_tris ? geom_grid(a) : 0;
   s.last_bin_grid = bin_grid(a);
+  // The kernels the batch runs (see BatchArgs): chosen from its size alone.
+  a.front = !persistent && p.total_tris > 0 && p.total_tris <= kFrontTris;
+  a.small = a.front && a.host_counters && p.max_width <= kSmallWidth &&
+            p.ntiles <= kSmallTiles && p.small_tests <= kSmallTests &&
+            p.max_regions <= kSmallRegions &&
+            (uint64_t)a.nregions * (kRegion * sizeof(SetupRec) + 8) <= x.ckpt.bytes;
+  a.recs = (SetupRec*)x.ckpt.p;
+  a.region_box = (uint2*)(a.recs + a.nregions * kRegion);
   // The clear kernel runs only when the counters it zeroes are not known to
-  // be zero: new buffers, more tiles than cleared before, or no geometry
-  // kernel (which clears the batch counters).
+  // be zero: new buffers, more tiles than cleared before, no vertex kernel
+  // (which clears the batch counters) and no shading kernel that left them
+  // zero.  A small batch uses none of them.
   const bool same_bufs = s.clean_ref[0] == x.tile_count.p && s.clean_ref[1] == x.tile_done.p &&
-                         s.clean_ref[2] == x.scan_status.p;
-  const bool clear = !same_bufs || p.total_tris == 0 || p.ntiles > s.clean_tiles ||
-                     a.scan_blocks > s.clean_scan;
+                         s.clean_ref[2] == x.scan_status.p && s.clean_ref[3] == x.counters.p &&
+                         s.clean_ref[4] == x.ckpt_ctr.p;
+  const bool clear = !a.small &&
+                     (!same_bufs || p.total_tris == 0 || p.ntiles > s.clean_tiles ||
+                      a.scan_blocks > s.clean_scan || (a.front && !s.clean_counters));
   // Zero prefixes after this batch: the clear kernel (if run) zeroes this
   // batch's range, the shading kernel re-zeroes it, entries past it keep
   // their state.
   const int64_t next_tiles = std::max<int64_t>(p.ntiles, same_bufs ? s.clean_tiles : 0);
   const int64_t next_scan = std::max<int64_t>(a.scan_blocks, same_bufs ? s.clean_scan : 0);
+  const int64_t prev_tiles = s.clean_tiles, prev_scan = s.clean_scan;
+  const bool prev_counters = s.clean_counters;
   s.clean_tiles = s.clean_scan = 0;  // until the launches below succeed
+  // Eager launches of a batch that starts with k_front hand it small tables
+  // in its argument; a captured batch reads them from the staging when it is
+  // replayed.
+  const bool capture = c->graphs && !profile && s.own_stream && s.stream == s.own_stream;
+  const bool inl = a.front && !capture && p.layout.bytes <= kInlineWords * 4;
   auto issue = [&]() -> int {
-    HIP_TRY(hipMemcpyAsync(x.tables.p, x.h_tables.p, p.layout.bytes, hipMemcpyHostToDevice,
-                           s.stream));
-    int r = launch_stages(a, s, profile, clear, persistent, c->wait_us);
+    if (!inl)
+      HIP_TRY(hipMemcpyAsync(x.tables.p, x.h_tables.p, p.layout.bytes, hipMemcpyHostToDevice,
+                             s.stream));
+    int r = launch_stages(a, s, profile, clear, persistent, c->wait_us,
+                          inl ? x.h_tables.p : nullptr, p.layout.bytes);
     if (r) return r;
     if (!a.host_counters)
       HIP_TRY(hipMemcpyAsync(x.h_counters.p, a.counters, kNumCounters * 8,
@@ -539,7 +585,7 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   };
   // Graphs only on the slot's own stream (a caller's stream may be the null
   // stream, which cannot be captured) and without per-stage events.
-  if (c->graphs && !profile && s.own_stream && s.stream == s.own_stream) {
+  if (capture) {
     const void* hp[5] = {x.h_tables.p, x.h_counters.p, (const void*)p.layout.bytes,
                          (const void*)(uintptr_t)clear, persistent ? x.ctl.p : nullptr};
     std::vector<unsigned char> key(sizeof(BatchArgs) + sizeof(hp));
@@ -555,9 +601,9 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
     // geometry launches, raster template, persistent or not) updates the
     // parameters of an instantiated graph in place instead of instantiating
     // a new one, so a service of mixed batches keeps replaying a few graphs.
-    const int32_t topo_v[7] = {clear ? 1 : 0, a.total_verts ? 1 : 0, a.total_tris ? 1 : 0,
+    const int32_t topo_v[8] = {clear ? 1 : 0, a.total_verts ? 1 : 0, a.total_tris ? 1 : 0,
                                a.tile_w, a.raster_threads, persistent ? 1 : 0,
-                               persistent ? 0 : a.ckpt_in_scan};
+                               persistent ? 0 : a.ckpt_in_scan, 2 * a.small + a.front};
     std::vector<unsigned char> topo((const unsigned char*)topo_v,
                                     (const unsigned char*)topo_v + sizeof(topo_v));
     if (hit == s.graphs.size()) {
@@ -612,11 +658,21 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
     if ((rc = issue())) return rc;
   }
   HIP_TRY(hipEventRecord(s.done, s.stream));
+  if (a.small) {  // left as they were
+    s.clean_tiles = prev_tiles;
+    s.clean_scan = prev_scan;
+    s.clean_counters = prev_counters;
+    return MR_OK;
+  }
   s.clean_ref[0] = x.tile_count.p;
   s.clean_ref[1] = x.tile_done.p;
   s.clean_ref[2] = x.scan_status.p;
+  s.clean_ref[3] = x.counters.p;
+  s.clean_ref[4] = x.ckpt_ctr.p;
   s.clean_tiles = next_tiles;
   s.clean_scan = next_scan;
+  // The shading kernel that hands the host the counters leaves them zero.
+  s.clean_counters = a.host_counters != nullptr;
   return MR_OK;
 }
 
@@ -637,6 +693,7 @@ int finish_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
       return MR_ERR_DEVICE;
     }
     if (!hc[kBinOverflow] && !hc[kHeavyOverflow]) break;
+    s.clean_counters = false;  // the flags stay set
     if (attempt >= 3 || hc[kBinEntries] >= 0xFFFFFFF0ull) return MR_ERR_NOMEM;
     s.retries++;
     int rc;

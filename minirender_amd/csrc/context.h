@@ -87,6 +87,9 @@ struct BatchPlan {
   int64_t ntiles = 0;
   int64_t npixels = 0;
   int64_t shade_blocks = 0;
+  int32_t max_width = 0;
+  int64_t max_regions = 0;  // of one job
+  int64_t small_tests = 0;  // regions the tiles of a small batch test together
   TableLayout layout;
 };
 
@@ -117,7 +120,8 @@ struct Slot {
   // Leading tile counters / look-back words known to be zero (the shading
   // kernel re-zeroes what a batch used), valid for the buffers in clean_ref.
   int64_t clean_tiles = 0, clean_scan = 0;
-  const void* clean_ref[3] = {nullptr, nullptr, nullptr};
+  bool clean_counters = false;  // batch and checkpoint counters too
+  const void* clean_ref[5] = {};
 };
 
 }  // namespace mr

@@ -169,12 +169,7 @@ MR_HD inline float advance(float s, float d, int n) {
 // and unrolled by 8, so a wavefront spends about one instruction per add on
 // loop control instead of three or four (lanes with different n run the same
 // instruction stream under their execution mask).
-MR_HD inline void advance2(float& e1, float d1, float& e2, float d2, int n) {
-  if (n > 256) {
-    e1 = ff_add(e1, d1, n);
-    e2 = ff_add(e2, d2, n);
-    return;
-  }
+MR_HD inline void walk2(float& e1, float d1, float& e2, float d2, int n) {
   float a = e1, b = e2;
   for (int i = n >> 3; i > 0; i--) {
 #pragma unroll
@@ -202,6 +197,17 @@ MR_HD inline void advance2(float& e1, float d1, float& e2, float d2, int n) {
   }
   e1 = a;
   e2 = b;
+}
+
+// walk2, by ff_add for long runs (whose fp64 divisions and branches cost as
+// much as about a thousand steps).
+MR_HD inline void advance2(float& e1, float d1, float& e2, float d2, int n) {
+  if (n > 1024) {
+    e1 = ff_add(e1, d1, n);
+    e2 = ff_add(e2, d2, n);
+    return;
+  }
+  walk2(e1, d1, e2, d2, n);
 }
 
 // Row start of the edge walk at the bbox's left column (Renderer.cpp:240-242).

@@ -8,6 +8,8 @@
 //   k_vertex  (a) eye-space transform and projection once per vertex of each
 //             (attribute arrays, modelview) group of a job (Renderer.cpp:340-349,
 //             191-203): the per-material meshes of a model share one group
+//   k_front   vertex and geometry kernel in one, for batches of at most
+//             kFrontTris triangles
 //   k_geom    (a)+(b) index gather, near clip, setup and cull of every input
 //             triangle (Renderer.cpp:351-380, 163-236).  Each wavefront
 //             compacts its survivors into its own region of the item stream
@@ -37,6 +39,8 @@
 //   k_shade   (e) deferred Blinn-Phong + texture, one lane per pixel in image
 //             order, writing RGB8 / depth / winner / float colour / normals /
 //             range image (background for the pixels of empty tiles)
+//   k_small   (c)-(e) of a small batch in one kernel behind k_front: its tiles
+//             test the items themselves, nothing is counted or binned
 //   k_persist every stage above in one launch of a resident grid fed by
 //             device work queues (optional; the same stage functions)
 //
@@ -103,15 +107,26 @@ __device__ u64 lookback(u64* status, int idx, u64 aggregate, u64* counters) {
 // Each stage is a device function of its workgroup index vb in a grid of
 // nvb workgroups of 256 threads: run by its own kernel (vb = blockIdx.x),
 // or by the persistent kernel, whose workgroups take stage work from queues.
-// Counters of a batch: the batch counters, the checkpoint segments' and the
-// lengths of the direct lists.
+// Counters of a batch: the batch counters and the checkpoint segments'.
 __device__ __forceinline__ void zero_counters(const BatchArgs& a) {
   if (threadIdx.x < kNumCounters) a.counters[threadIdx.x] = 0;
   if (threadIdx.x < kCkptSegs) a.ckpt_ctr[threadIdx.x * kCtrStride] = 0;
   if (threadIdx.x == 0) a.ckpt_ctr[kCkptBigEntries] = a.ckpt_ctr[kCkptBigRows] = 0;
-  if (a.direct_cap)
-    for (int i = threadIdx.x; i < a.njobs * 8; i += 256)
-      a.direct_count[(size_t)(i >> 3) * kCtrStride + (i & 7)] = 0;
+}
+
+// A tile's line of words (tile_count): pairs and work, direct entries, and in
+// a job's first tile the length and box of the job's direct list.
+__device__ __forceinline__ void zero_tile(const BatchArgs& a, int i) {
+  ulonglong2* const line = (ulonglong2*)(a.tile_count + (size_t)i * kCtrStride64);
+  line[0] = line[1] = line[2] = make_ulonglong2(0ull, 0ull);
+  a.tile_done[i] = 0;
+}
+
+// The direct list's line of the job with first tile `tile_base`: the number
+// of its items, then kMaxDim - first column, last column, kMaxDim - first row
+// and last row of their bounding box.
+__device__ __forceinline__ uint32_t* direct_line(const BatchArgs& a, int tile_base) {
+  return (uint32_t*)(a.tile_count + (size_t)tile_base * kCtrStride64 + 2);
 }
 
 __device__ __forceinline__ void stage_clear(const BatchArgs& a, int vb, int nvb) {
@@ -121,11 +136,7 @@ __device__ __forceinline__ void stage_clear(const BatchArgs& a, int vb, int nvb)
   const int n = max(a.scan_blocks, a.ntiles);
   for (int i = vb * 256 + (int)threadIdx.x; i < n; i += nvb * 256) {
     if (i < a.scan_blocks) a.scan_status[i] = 0;
-    if (i < a.ntiles) {
-      a.tile_count[(size_t)i * kCtrStride64] = 0;
-      a.tile_count[(size_t)i * kCtrStride64 + 1] = 0;
-      a.tile_done[i] = 0;
-    }
+    if (i < a.ntiles) zero_tile(a, i);
   }
 }
 
@@ -163,6 +174,19 @@ __device__ inline int wave_search_last(const int64_t* begin, int n, int64_t x) {
     span = __builtin_amdgcn_readfirstlane(span);
   }
   return lo;
+}
+
+// Maximum over the wavefront (every lane active): rows of 16 lanes by DPP,
+// then the four rows' through scalar registers; no trips through LDS.
+__device__ inline uint32_t wave_max(uint32_t v) {
+  auto step = [&](uint32_t o) { v = v > o ? v : o; };
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));   // lane ^ 1
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));   // lane ^ 2
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true));  // half-row mirror
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true));  // row mirror
+  const uint32_t a = __builtin_amdgcn_readlane((int)v, 0), b = __builtin_amdgcn_readlane((int)v, 16);
+  const uint32_t c = __builtin_amdgcn_readlane((int)v, 32), d = __builtin_amdgcn_readlane((int)v, 48);
+  return max(max(a, b), max(c, d));
 }
 
 // Job of tile (shading block) x from the job hints: the job of x's span of
@@ -290,6 +314,27 @@ __device__ inline void corners(const BatchArgs& a, const DrawDesc& D, int t, int
   }
 }
 
+// The same from the corners' positions (the vertex kernel's arithmetic), for
+// batches whose geometry stands in for the vertex kernel: the record of every
+// corner is written for the kernels that follow (several lanes may write one
+// vertex's: the same bits).
+__device__ inline void corners_pos(const BatchArgs& a, const DrawDesc& D, const JobDesc& J, int t,
+                                   int vi[3], f3 e[3], ScreenVtx v[3]) {
+  const auto* ip = G(D.idx) + 3 * t;
+  vi[0] = ip[0];
+  vi[1] = ip[1];
+  vi[2] = ip[2];
+  f3 p[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) p[k] = load3(D.pos, vi[k]);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    e[k] = xform(D.mv, p[k]);
+    v[k] = project_vertex(J.P, J.persp != 0, (float)J.W, (float)J.H, e[k]);
+    a.vscr[D.vbase + vi[k]] = make_float4(v[k].px, v[k].py, v[k].zv, e[k].z);
+  }
+}
+
 // The corners' eye x, y, transformed again from the positions (the vertex
 // kernel's arithmetic on the same modelview: the same bits, Renderer.cpp:
 // 344-345); only a triangle across the near plane or of a draw without the
@@ -309,14 +354,16 @@ __device__ inline void corner_eyes(const DrawDesc& D, const int vi[3], f3 e[3]) 
 // Near test, clip and setup of triangle t (Renderer.cpp:169-236).  Returns
 // the number of surviving sub-triangles (0..2) and their sub-indices.
 // Unclipped triangles use the per-vertex projections; clipped ones project
-// their clipped corners here.
+// their clipped corners here.  kVerts: corners from positions (corners_pos).
+template <bool kVerts>
 __device__ inline int tri_setup(const BatchArgs& a, const DrawDesc& D, const JobDesc& J, int t,
                                 TriSetup& s0, int& sub0, TriSetup& s1,
                                 int& sub1, bool& clipped) {
   int vi[3];
   f3 e[3];
   ScreenVtx v[3];
-  corners(a, D, t, vi, e, v);
+  if (kVerts) corners_pos(a, D, J, t, vi, e, v);
+  else corners(a, D, t, vi, e, v);
   const float zn = J.znear;
   const bool persp = J.persp != 0;
   const float w = (float)J.W, h = (float)J.H;
@@ -325,7 +372,7 @@ __device__ inline int tri_setup(const BatchArgs& a, const DrawDesc& D, const Job
   if (!D.no_clip && (b0 || b1 || b2)) {
     if (b0 && b1 && b2) return 0;
     clipped = true;
-    corner_eyes(D, vi, e);
+    if (!kVerts) corner_eyes(D, vi, e);
     f3 a0, a1, a2, c0, c1, c2;
     const int ns = clip_positions(zn, e[0], e[1], e[2], a0, a1, a2, c0, c1, c2);
     int n = 0;
@@ -576,8 +623,8 @@ __device__ void wave_tile_pairs(const BatchArgs& a, bool active, uint32_t id, ui
 // Direct items of a wavefront step: up to two per lane (d0, d1), appended to
 // their job's list by one atomic per job.  Clears the flag of an item that
 // finds no room; it is then binned.
-__device__ inline void direct_append(const BatchArgs& a, int job, bool& d0, const BinItem& i0,
-                                     bool& d1, const BinItem& i1) {
+__device__ inline void direct_append(const BatchArgs& a, int job, int tile_base, bool& d0,
+                                     const BinItem& i0, bool& d1, const BinItem& i1) {
   const int lane = threadIdx.x & 63;
   const u64 lt = (1ull << lane) - 1ull;
   u64 pend = __ballot(d0 || d1);
@@ -588,7 +635,7 @@ __device__ inline void direct_append(const BatchArgs& a, int job, bool& d0, cons
     const bool mine = (d0 || d1) && ((pend >> lane) & 1ull) && job == jj;
     const u64 g0 = __ballot(mine && d0), g1 = __ballot(mine && d1);
     uint32_t base = 0;
-    uint32_t* const line = a.direct_count + (size_t)jj * kCtrStride;
+    uint32_t* const line = direct_line(a, __builtin_amdgcn_readlane(tile_base, l));
     if (lane == l) base = atomicAdd(line, (uint32_t)(__popcll(g0) + __popcll(g1)));
     // Bounding box of the job's list (as maxima: the words start at zero).
     uint32_t box[4] = {0, 0, 0, 0};
@@ -639,7 +686,7 @@ __device__ inline bool wants_ckpt(int bx0, int bx1, int sw) {
 constexpr int kLargeSpan = 24;  // < the span of 16 tiles of 8 x 8, and of kCkptMinSpan
 __device__ inline int large_items(const BatchArgs& a, bool l0, bool l1, const TriSetup& s0,
                                   const TriSetup& s1, uint32_t id0, uint32_t id1, uint32_t draw,
-                                  int job, int sw, int sh) {
+                                  int job, int tile_base, int sw, int sh) {
   auto tiles_of = [&](const TriSetup& s) {
     return ((s.bx1 >> sw) - (s.bx0 >> sw) + 1) * ((s.by1 >> sh) - (s.by0 >> sh) + 1);
   };
@@ -650,7 +697,7 @@ __device__ inline int large_items(const BatchArgs& a, bool l0, bool l1, const Tr
                         (uint16_t)s0.by1};
     const BinItem i1 = {id1, draw, (uint16_t)s1.bx0, (uint16_t)s1.bx1, (uint16_t)s1.by0,
                         (uint16_t)s1.by1};
-    direct_append(a, job, d0, i0, d1, i1);
+    direct_append(a, job, tile_base, d0, i0, d1, i1);
   }
   const bool w0 = l0 && wants_ckpt(s0.bx0, s0.bx1, sw);
   const bool w1 = l1 && wants_ckpt(s1.bx0, s1.bx1, sw);
@@ -681,10 +728,14 @@ __device__ inline int large_items(const BatchArgs& a, bool l0, bool l1, const Tr
 // kDirectTiles tiles or more go to their job's direct list: a wavefront's 64
 // triangles of hundreds of tiles each would count (and later scatter) their
 // pairs 64 at a time, one wavefront alone.
+//
+// kVerts: no vertex kernel ran before (k_front).  kSmall: the batch's raster
+// tests every item itself (k_small): items are written, nothing is counted.
+template <bool kVerts, bool kSmall>
 __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) {
   const int lane = threadIdx.x & 63;
   const int sw = __ffs(a.tile_w) - 1, sh = __ffs(a.tile_h) - 1;
-  uint32_t nclipped = 0;
+  uint32_t nclipped = 0, nitems = 0, npairs = 0;
   // Each workgroup takes one contiguous range of triangles (a multiple of
   // 256), so a wavefront finds its draw once and then only steps over draw
   // boundaries; its draw and job descriptors are read with scalar loads.
@@ -716,7 +767,7 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
       if (g >= next_begin)
         while (d + 1 < a.ndraws && a.draw_begin[d + 1] <= g) d++;
       auto setup = [&](const DrawDesc& D, const JobDesc& J) {
-        ns = tri_setup(a, D, J, (int)(g - D.tri_begin), s0, sub0, s1, sub1, clipped);
+        ns = tri_setup<kVerts>(a, D, J, (int)(g - D.tri_begin), s0, sub0, s1, sub1, clipped);
         tbase = D.tile_base;
         tiles_x = D.tiles_x;
         job = D.job;
@@ -736,7 +787,10 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
     const u64 b1 = __ballot(ns >= 1), b2 = __ballot(ns == 2);
     const int64_t region = wfirst >> 6;
     if (lane == 0) a.region_count[region] = (uint32_t)(__popcll(b1) + __popcll(b2));
-    if (!b1) continue;
+    if (!b1) {
+      if (kSmall && lane == 0) a.region_box[region] = make_uint2(0xFFFFu, 0xFFFFu);  // meets no tile
+      continue;
+    }
     const u64 lt = (1ull << lane) - 1ull;
     const int64_t pos = region * kRegion + __popcll(b1 & lt) + __popcll(b2 & lt);
     const uint32_t id0 = (uint32_t)(2 * g + sub0), id1 = (uint32_t)(2 * g + sub1);
@@ -746,13 +800,36 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
     if (ns == 2)
       a.items[pos + 1] = BinItem{id1, draw, (uint16_t)s1.bx0, (uint16_t)s1.bx1,
                                  (uint16_t)s1.by0, (uint16_t)s1.by1};
+    if (kSmall) {  // the region's box, the raster's setups; statistics
+      uint32_t box[4] = {0, 0, 0, 0};  // (as maxima)
+      if (ns >= 1) {
+        box[0] = 0xFFFFu - s0.bx0, box[1] = s0.bx1, box[2] = 0xFFFFu - s0.by0, box[3] = s0.by1;
+        if (ns == 2) {
+          box[0] = max(box[0], 0xFFFFu - s1.bx0), box[1] = max(box[1], (uint32_t)s1.bx1);
+          box[2] = max(box[2], 0xFFFFu - s1.by0), box[3] = max(box[3], (uint32_t)s1.by1);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) box[k] = wave_max(box[k]);
+      if (lane == 0)
+        a.region_box[region] = make_uint2((0xFFFFu - box[0]) | box[1] << 16,
+                                          (0xFFFFu - box[2]) | box[3] << 16);
+      if (ns >= 1) a.recs[pos] = SetupRec{s0, id0};
+      if (ns == 2) a.recs[pos + 1] = SetupRec{s1, id1};
+      auto pairs = [&](const TriSetup& s) {
+        return (uint32_t)(((s.bx1 >> sw) - (s.bx0 >> sw) + 1) * ((s.by1 >> sh) - (s.by0 >> sh) + 1));
+      };
+      nitems += (uint32_t)(__popcll(b1) + __popcll(b2));
+      npairs += (ns >= 1 ? pairs(s0) : 0u) + (ns == 2 ? pairs(s1) : 0u);
+      continue;
+    }
     // Direct items and those that want checkpoints are at least kLargeSpan
     // pixels in width and height together; few wavefronts hold any.
     bool d0 = false, d1 = false;
     const bool l0 = ns >= 1 && (s0.bx1 - s0.bx0) + (s0.by1 - s0.by0) >= kLargeSpan;
     const bool l1 = ns == 2 && (s1.bx1 - s1.bx0) + (s1.by1 - s1.by0) >= kLargeSpan;
     if (__ballot(l0 || l1)) {
-      const int large = large_items(a, l0, l1, s0, s1, id0, id1, draw, job, sw, sh);
+      const int large = large_items(a, l0, l1, s0, s1, id0, id1, draw, job, tbase, sw, sh);
       d0 = large & 1;
       d1 = large & 2;
       if (d0) a.items[pos].draw = draw | kDirectFlag;
@@ -769,16 +846,48 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
       wave_tile_pairs<false>(a, ns == 2 && !d1, id1, draw, tbase, tiles_x, s1.bx0, s1.bx1, s1.by0,
                              s1.by1, sw, sh, count);
   }
-  __shared__ uint32_t sh_clipped;
-  if (threadIdx.x == 0) sh_clipped = 0;
+  __shared__ uint32_t sh_clipped, sh_items, sh_pairs;
+  if (threadIdx.x == 0) sh_clipped = sh_items = sh_pairs = 0;
   __syncthreads();
   if (lane == 0 && nclipped) atomicAdd(&sh_clipped, nclipped);
+  if (kSmall) {
+    if (lane == 0 && nitems) atomicAdd(&sh_items, nitems);
+    if (npairs) atomicAdd(&sh_pairs, npairs);
+  }
   __syncthreads();
-  if (threadIdx.x == 0 && vb < kStatSlots) a.block_stats[vb] = sh_clipped;
+  if (threadIdx.x == 0 && vb < kStatSlots) {
+    a.block_stats[vb] = sh_clipped;
+    if (kSmall) a.block_stats[kStatSlots + vb] = ((u64)sh_items << 32) | sh_pairs;
+  }
 }
 
 __global__ __launch_bounds__(256, 7) void k_geom(BatchArgs a) {
-  stage_geom(a, blockIdx.x, gridDim.x);
+  stage_geom<false, false>(a, blockIdx.x, gridDim.x);
+}
+
+// The first kernel of a small or middling batch: geometry from the vertex
+// positions (each transformed once per corner instead of once), without the
+// vertex kernel's launch and its round trip through memory.  The batch tables
+// come inside the kernel argument when they fit (nwords): then nothing is
+// uploaded before it, and its first workgroup writes the tables for the
+// kernels that follow.
+using KernargTables = const __attribute__((address_space(4))) TableArgs;
+
+template <bool kSmall>
+__global__ __launch_bounds__(256, kSmall ? 4 : 6) void k_front(TableArgs) {
+  KernargTables* const pk = (KernargTables*)__builtin_amdgcn_kernarg_segment_ptr();
+  const TableArgs& arg = *(const TableArgs*)pk;
+  BatchArgs a = arg.a;
+  if (arg.nwords) {
+    const char* const inl = (const char*)arg.words;
+    const char* const base = (const char*)a.jobs;  // the tables' first
+    if (blockIdx.x == 0)
+      for (uint32_t i = threadIdx.x; i < arg.nwords; i += 256) ((uint32_t*)a.jobs)[i] = arg.words[i];
+    a.draws = (const DrawDesc*)(inl + ((const char*)a.draws - base));
+    a.draw_begin = (const int64_t*)(inl + ((const char*)a.draw_begin - base));
+    a.jobs = (const JobDesc*)inl;
+  }
+  stage_geom<true, kSmall>(a, blockIdx.x, gridDim.x);
 }
 
 // Row bands of a tile rastered by several workgroups (each with all of the
@@ -831,7 +940,7 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a) {
     for (int i = 0; i < kScanItems; i++) {
       if (base + i < a.ntiles && (i == 0 || base + i >= next)) {
         if (i) j++;
-        any = a.direct_count[(size_t)j * kCtrStride] != 0;
+        any = *direct_line(a, a.job_tile_base[j]) != 0;
         next = j + 1 < a.njobs ? a.job_tile_base[j + 1] : 0x7FFFFFFF;
       }
       listed |= (any ? 1u : 0u) << i;
@@ -1247,7 +1356,7 @@ __device__ __forceinline__ void stage_direct(const BatchArgs& a, int vb, int nvb
     int groups = 0;    // of the lists of the jobs here
     bool own = false;  // this tile's job has a list
     for (int j = j0; j < a.njobs && a.job_tile_base[j] < t_end; j++) {
-      const int nd = (int)min(a.direct_count[(size_t)j * kCtrStride], a.direct_cap);
+      const int nd = (int)min(*direct_line(a, a.job_tile_base[j]), a.direct_cap);
       groups += (nd + kDirectGroup - 1) / kDirectGroup;
       if (t >= a.job_tile_base[j]) own = nd != 0;
     }
@@ -1259,8 +1368,7 @@ __device__ __forceinline__ void stage_direct(const BatchArgs& a, int vb, int nvb
     for (int pass = 0; pass < 2; pass++) {
       // (The tiles usually lie in one job.)
       for (int j = j0; j < a.njobs && a.job_tile_base[j] < t_end; j++) {
-        const uint32_t* const line = a.direct_count + (size_t)j * kCtrStride;
-        const int nd = (int)min(line[0], a.direct_cap);
+        const int nd = (int)min(*direct_line(a, a.job_tile_base[j]), a.direct_cap);
         if (nd == 0) continue;
         const JobDesc& J = a.jobs[j];
         const int local = t - J.tile_base;
@@ -1407,6 +1515,124 @@ __device__ inline void raster_pixel(u64* keys, int p, float e1, float e2, float 
 
 constexpr int kCoverRowsMin = 4;  // wide entries of a wavefront from which rows are tested
 
+// Workgroup memory of the raster.  Key rows are padded by one entry: pixels of
+// one column in different rows fall in different LDS banks.
+template <int TW, int TH, int NT>
+struct RasterLds {
+  static constexpr int KS = TW + 1;
+  u64 keys[TH * KS];
+  TriSetup setups[NT];
+  uint32_t setup_id[NT];
+  int row_start[NT];
+  int wave_rows[NT / 64];
+};
+
+// Draw one entry per thread (have: there is one) into the keys of the tile at
+// (x0, y0), rows band_lo .. band_hi of it.  kRec: the entry is be.x of the
+// batch's setup records, and no edge checkpoints were taken; else it is
+// {id, draw}, set up here, and rows of wide triangles start from their
+// checkpoints.  Ends with a barrier.
+template <int TW, int TH, int NT, bool kRec>
+__device__ __forceinline__ void raster_chunk(const BatchArgs& a, const JobDesc& J,
+                                             RasterLds<TW, TH, NT>& lds, bool have, uint2 be,
+                                             int x0, int y0, int band_lo, int band_hi) {
+  constexpr int KS = RasterLds<TW, TH, NT>::KS;
+  const int tid = threadIdx.x;
+  const bool persp = J.persp != 0;
+  // One lane per entry: setup, and the tile rows it covers.
+  int nrows = 0;
+  if (have) {
+    uint32_t id = be.x;
+    TriSetup s;
+    if (kRec) {
+      const SetupRec r = a.recs[be.x];
+      s = r.s;
+      id = r.id;
+    } else {
+      const int64_t g = id >> 1;
+      const uint32_t d0 = __builtin_amdgcn_readfirstlane(be.y);
+      if (__ballot(be.y == d0) == __ballot(1)) {
+        const DrawDesc Du = uniform_draw(a, (int)d0);
+        tri_setup_sub(a, Du, J, (int)(g - Du.tri_begin), (int)(id & 1u), s);
+      } else {
+        const DrawDesc& D = a.draws[be.y];
+        tri_setup_sub(a, D, J, (int)(g - D.tri_begin), (int)(id & 1u), s);
+      }
+    }
+    // Rows of this item, without those it covers no pixel of (a triangle
+    // no wider than the tile covers pixels in nearly all of its rows, and
+    // the test pays for a few wide ones in the wavefront at least).
+    int r0 = max(s.by0, y0 + band_lo), r1 = min(s.by1, y0 + band_hi);
+    const bool wide = s.bx1 - s.bx0 >= TW && r1 >= r0;
+    if (__popcll(__ballot(wide)) >= kCoverRowsMin && wide)
+      cover_rows(s, max(s.bx0, x0), min(s.bx1, x0 + TW - 1), r0, r1);
+    nrows = max(r1 - r0 + 1, 0);
+    s.by0 = r0;  // the first row taken
+    lds.setups[tid] = s;
+    lds.setup_id[tid] = id;
+  }
+  // Exclusive scan of the row counts over the workgroup.
+  int incl = nrows;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o);
+    if ((tid & 63) >= o) incl += y;
+  }
+  if ((tid & 63) == 63) lds.wave_rows[tid >> 6] = incl;
+  __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; w++) {
+    if (w < (tid >> 6)) before += lds.wave_rows[w];
+    total += lds.wave_rows[w];
+  }
+  lds.row_start[tid] = before + incl - nrows;
+  __syncthreads();
+  // One lane per (triangle, tile row): start the row at the tile's left
+  // edge (exact advance of the serial recurrence), then step across the
+  // tile as the reference's column loop does (Renderer.cpp:238-269).
+  for (int q = tid; q < total; q += NT) {
+    const int i = owner_search<NT>(lds.row_start, q);
+    const TriSetup& s = lds.setups[i];
+    const int row = s.by0 + (q - lds.row_start[i]);
+    const int cx0 = max(s.bx0, x0), cx1 = min(s.bx1, x0 + TW - 1);
+    const uint32_t id = lds.setup_id[i];
+    // A row entering a tile column after its triangle's first starts
+    // from the edge checkpoint the row pre-pass left at or before it (the
+    // same serial chain from the bbox's left column); without checkpoints
+    // (none allocated) it walks from the left column itself.
+    float e1 = 0.0f, e2 = 0.0f;
+    int steps = -1;
+    if (!kRec && cx0 > s.bx0 && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {  // only these have any
+      const int2 cb = a.ckpt_base[id];
+      const int cs = cb.y >> 16, col = x0 >> cs;
+      if (cb.y && col > (s.bx0 >> cs)) {
+        const float2 st = a.ckpt[(int64_t)cb.x + (int64_t)row * (cb.y & 0xFFFF) + col];
+        e1 = st.x;
+        e2 = st.y;
+        steps = x0 - (col << cs);
+      }
+    }
+    if (steps < 0) {
+      edge_start(s.n1x, s.n1y, s.n2x, s.n2y, s.p0x, s.p0y, s.p2x, s.p2y,
+                 (float)s.bx0 + 0.5f, (float)row + 0.5f, e1, e2);
+      steps = cx0 - s.bx0;
+    }
+    if (kRec) walk2(e1, s.n1x, e2, s.n2x, steps);  // (less than kSmallWidth)
+    else advance2(e1, s.n1x, e2, s.n2x, steps);
+    // The triangle's steps and depths in registers for the row: read from
+    // the workgroup's setup table once, not again after each key update.
+    const float n1x = s.n1x, n2x = s.n2x, z0 = s.z0, z1 = s.z1, z2 = s.z2;
+    const int prow = (row - y0) * KS - x0;
+    for (int c = cx0; c <= cx1; c++) {
+      raster_pixel(lds.keys, prow + c, e1, e2, z0, z1, z2, persp, id);
+      e1 = e1 + n1x;
+      e2 = e2 + n2x;
+    }
+  }
+  __syncthreads();
+}
+
 // Raster work items of the batch: parts and row bands, and tiles rastered
 // whole (those with bin entries, then those with direct entries only).
 struct TileItems {
@@ -1429,15 +1655,9 @@ __device__ inline TileItems tile_items(const BatchArgs& a) {
 // where consecutive workgroups go to different XCDs), else in list order.
 template <int TW, int TH, int NT>
 __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool remap) {
-  constexpr int NP = TW * TH;
-  // Key rows padded by one entry: pixels of one column in different rows
-  // fall in different LDS banks.
-  constexpr int KS = TW + 1;
-  __shared__ u64 keys[TH * KS];
-  __shared__ TriSetup setups[NT];
-  __shared__ uint32_t setup_id[NT];
-  __shared__ int row_start[NT];
-  __shared__ int wave_rows[NT / 64];
+  constexpr int NP = TW * TH, KS = RasterLds<TW, TH, NT>::KS;
+  __shared__ RasterLds<TW, TH, NT> lds;
+  u64* const keys = lds.keys;
   __shared__ int sh_last;
   const int tid = threadIdx.x;
   bool direct = a.counters[kDirect] != 0ull;
@@ -1465,7 +1685,7 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     // are not in it (shading writes their background).
     // (Tiles with direct entries only are listed from the end.)
     const int64_t t = b - items.parts;
-    const int64_t li = remap ? xcd_remap(t, items.listed) : t;
+    const int64_t li = remap ? (int64_t)xcd_chunks<kXcdChunk>((uint32_t)t, (uint32_t)items.listed) : t;
     const uint4 le = a.tile_list[li < items.whole ? li : a.ntiles - 1 - (li - items.whole)];
     tile = (int)le.x;
     part = 0;
@@ -1477,7 +1697,6 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     const uint32_t nparts = cnt <= a.frag_size ? 1u : (cnt + a.frag_size - 1) / a.frag_size;
     const int j = job_lookup(a.tile_hint, a.job_tile_base, a.njobs, tile);
     const JobDesc& J = a.jobs[j];
-    const bool persp = J.persp != 0;
     const int local = tile - J.tile_base;
     const int tyi = local / J.tiles_x, txi = local - tyi * J.tiles_x;
     const int x0 = txi * TW, y0 = tyi * TH;
@@ -1498,93 +1717,10 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     for (int p = tid; p < TH * KS; p += NT) keys[p] = ~0ull;
     __syncthreads();
     for (uint32_t base = 0; base < nall; base += NT) {
-      // One lane per entry: setup, and the tile rows it covers.
-      int nrows = 0;
       const uint32_t q0 = base + tid;
-      if (q0 < nall) {
-        const uint2 be = a.bins[q0 + (q0 < nbin ? off + e_begin : off2)];
-        const uint32_t id = be.x;
-        const int64_t g = id >> 1;
-        TriSetup s;
-        const uint32_t d0 = __builtin_amdgcn_readfirstlane(be.y);
-        if (__ballot(be.y == d0) == __ballot(1)) {
-          const DrawDesc Du = uniform_draw(a, (int)d0);
-          tri_setup_sub(a, Du, J, (int)(g - Du.tri_begin), (int)(id & 1u), s);
-        } else {
-          const DrawDesc& D = a.draws[be.y];
-          tri_setup_sub(a, D, J, (int)(g - D.tri_begin), (int)(id & 1u), s);
-        }
-        // Rows of this item, without those it covers no pixel of (a triangle
-        // no wider than the tile covers pixels in nearly all of its rows, and
-        // the test pays for a few wide ones in the wavefront at least).
-        int r0 = max(s.by0, y0 + band_lo), r1 = min(s.by1, y0 + band_hi);
-        const bool wide = s.bx1 - s.bx0 >= TW && r1 >= r0;
-        if (__popcll(__ballot(wide)) >= kCoverRowsMin && wide)
-          cover_rows(s, max(s.bx0, x0), min(s.bx1, x0 + TW - 1), r0, r1);
-        nrows = max(r1 - r0 + 1, 0);
-        s.by0 = r0;  // the first row taken
-        setups[tid] = s;
-        setup_id[tid] = id;
-      }
-      // Exclusive scan of the row counts over the workgroup.
-      int incl = nrows;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(incl, o);
-        if ((tid & 63) >= o) incl += y;
-      }
-      if ((tid & 63) == 63) wave_rows[tid >> 6] = incl;
-      __syncthreads();
-      int before = 0, total = 0;
-#pragma unroll
-      for (int w = 0; w < NT / 64; w++) {
-        if (w < (tid >> 6)) before += wave_rows[w];
-        total += wave_rows[w];
-      }
-      row_start[tid] = before + incl - nrows;
-      __syncthreads();
-      // One lane per (triangle, tile row): start the row at the tile's left
-      // edge (exact advance of the serial recurrence), then step across the
-      // tile as the reference's column loop does (Renderer.cpp:238-269).
-      for (int q = tid; q < total; q += NT) {
-        const int i = owner_search<NT>(row_start, q);
-        const TriSetup& s = setups[i];
-        const int row = s.by0 + (q - row_start[i]);
-        const int cx0 = max(s.bx0, x0), cx1 = min(s.bx1, x0 + TW - 1);
-        const uint32_t id = setup_id[i];
-        // A row entering a tile column after its triangle's first starts
-        // from the edge checkpoint the row pre-pass left at or before it (the
-        // same serial chain from the bbox's left column); without checkpoints
-        // (none allocated) it walks from the left column itself.
-        float e1 = 0.0f, e2 = 0.0f;
-        int steps = -1;
-        if (cx0 > s.bx0 && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {  // only these have any
-          const int2 cb = a.ckpt_base[id];
-          const int cs = cb.y >> 16, col = x0 >> cs;
-          if (cb.y && col > (s.bx0 >> cs)) {
-            const float2 st = a.ckpt[(int64_t)cb.x + (int64_t)row * (cb.y & 0xFFFF) + col];
-            e1 = st.x;
-            e2 = st.y;
-            steps = x0 - (col << cs);
-          }
-        }
-        if (steps < 0) {
-          edge_start(s.n1x, s.n1y, s.n2x, s.n2y, s.p0x, s.p0y, s.p2x, s.p2y,
-                     (float)s.bx0 + 0.5f, (float)row + 0.5f, e1, e2);
-          steps = cx0 - s.bx0;
-        }
-        advance2(e1, s.n1x, e2, s.n2x, steps);
-        // The triangle's steps and depths in registers for the row: read from
-        // the workgroup's setup table once, not again after each key update.
-        const float n1x = s.n1x, n2x = s.n2x, z0 = s.z0, z1 = s.z1, z2 = s.z2;
-        const int prow = (row - y0) * KS - x0;
-        for (int c = cx0; c <= cx1; c++) {
-          raster_pixel(keys, prow + c, e1, e2, z0, z1, z2, persp, id);
-          e1 = e1 + n1x;
-          e2 = e2 + n2x;
-        }
-      }
-      __syncthreads();
+      uint2 be = make_uint2(0, 0);
+      if (q0 < nall) be = a.bins[q0 + (q0 < nbin ? off + e_begin : off2)];
+      raster_chunk<TW, TH, NT, false>(a, J, lds, q0 < nall, be, x0, y0, band_lo, band_hi);
     }
     // The job's size and winner buffer in registers: the stores below could
     // alias the job table for all the compiler knows, which would reload
@@ -1673,7 +1809,9 @@ __device__ inline f3 unproject_pixel(const JobDesc& J, int c, int row, float ze)
   return f3{(b1 * a22 - b2 * a12) * idet, (a11 * b2 - a21 * b1) * idet, ze};
 }
 
-// Shading of a covered pixel whose winner `id` belongs to draw D.
+// Shading of a covered pixel whose winner `id` belongs to draw D.  kCkpt: the
+// batch has edge checkpoints.
+template <bool kCkpt>
 __device__ __forceinline__ void shade_lit(const BatchArgs& a, const JobDesc& J, const DrawDesc& D,
                                           uint32_t id, int c, int row, uint32_t pix) {
   const int64_t g = id >> 1;
@@ -1744,7 +1882,7 @@ __device__ __forceinline__ void shade_lit(const BatchArgs& a, const JobDesc& J, 
   // the others read no checkpoint base.
   float e1 = 0.0f, e2 = 0.0f;
   int steps = -1;
-  if ((c >> sw) > (s.bx0 >> sw) && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {
+  if (kCkpt && (c >> sw) > (s.bx0 >> sw) && s.bx1 - s.bx0 + 1 >= kCkptMinSpan) {
     const int2 cb = a.ckpt_base[id];
     const int cs = cb.y >> 16, col = c >> cs;
     if (cb.y && col > (s.bx0 >> cs)) {
@@ -1759,7 +1897,8 @@ __device__ __forceinline__ void shade_lit(const BatchArgs& a, const JobDesc& J, 
                (float)s.bx0 + 0.5f, (float)row + 0.5f, e1, e2);
     steps = c - s.bx0;
   }
-  advance2(e1, s.n1x, e2, s.n2x, steps);
+  if (kCkpt) advance2(e1, s.n1x, e2, s.n2x, steps);
+  else walk2(e1, s.n1x, e2, s.n2x, steps);  // (less than kSmallWidth)
   float k[3];
   const float z = depth_of(e1, e2, s.z0, s.z1, s.z2, J.persp != 0, k);
   if (!J.rgb8 && !J.rgb && !(J.normals && J.save_normals)) {
@@ -1887,7 +2026,8 @@ __device__ inline void shade_background(const JobDesc& J, uint32_t pix, int c, i
 }
 
 // Deferred shading of one pixel from its winner (Renderer.cpp:271-305).
-__device__ void shade_pixel(const BatchArgs& a, const JobDesc& J,
+template <bool kCkpt>
+__device__ __forceinline__ void shade_pixel(const BatchArgs& a, const JobDesc& J,
                             const int64_t* dcache, int ncached, uint32_t id,
                             int c, int row) {
   const uint32_t pix = (uint32_t)row * (uint32_t)J.W + (uint32_t)c;
@@ -1908,7 +2048,7 @@ __device__ void shade_pixel(const BatchArgs& a, const JobDesc& J,
       shade_background(J, pix, c, row);
       return;
     }
-    shade_lit(a, J, Du, id, c, row, pix);
+    shade_lit<kCkpt>(a, J, Du, id, c, row, pix);
   } else {
     const DrawDesc& Dc = a.draws[d];
     const int64_t tri = (int64_t)(id >> 1) - Dc.tri_begin;
@@ -1916,7 +2056,7 @@ __device__ void shade_pixel(const BatchArgs& a, const JobDesc& J,
       shade_background(J, pix, c, row);
       return;
     }
-    shade_lit(a, J, Dc, id, c, row, pix);
+    shade_lit<kCkpt>(a, J, Dc, id, c, row, pix);
   }
 }
 
@@ -1949,9 +2089,18 @@ __device__ void reduce_stats(const BatchArgs& a, int tid) {
     a.counters[kItems] = sr;
     // Every counter is final here (the kernels that add to them are done):
     // hand them to the host with the batch, no copy of its own.
+    // They are left zero for the next batch, but for the flags that the other
+    // shading workgroups read: the host clears those before it runs an
+    // overflowed batch again.
     if (a.host_counters)
-      for (int i = 0; i < kNumCounters; i++)
+      for (int i = 0; i < kNumCounters; i++) {
         a.host_counters[i] = i == kClipped ? sc : (i == kItems ? sr : a.counters[i]);
+        if (i != kBinOverflow && i != kHeavyOverflow) a.counters[i] = 0;
+      }
+  }
+  if (a.host_counters) {
+    if (tid < kCkptSegs) a.ckpt_ctr[tid * kCtrStride] = 0;
+    if (tid == 0) a.ckpt_ctr[kCkptBigEntries] = a.ckpt_ctr[kCkptBigRows] = 0;
   }
 }
 
@@ -1966,7 +2115,7 @@ __device__ void reduce_stats(const BatchArgs& a, int tid) {
 __device__ __forceinline__ void stage_shade(const BatchArgs& a, int vb, bool remap) {
   __shared__ int64_t dcache[kMaxLdsDraws];
   const int tid = threadIdx.x;
-  const int b = remap ? (int)xcd_remap(vb, a.shade_blocks) : vb;
+  const int b = remap ? (int)xcd_chunks<kXcdChunk>((uint32_t)vb, (uint32_t)a.shade_blocks) : vb;
   const int j = __builtin_amdgcn_readfirstlane(
       job_lookup(a.shade_hint, a.job_shade_base, a.njobs, b));
   const JobDesc J = uniform_job(a, j);
@@ -1994,11 +2143,7 @@ __device__ __forceinline__ void stage_shade(const BatchArgs& a, int vb, bool rem
   // look-back words: leave them zero for the next batch on this scratch.
   for (int64_t i = (int64_t)vb * kShadeBlock + tid; i < a.ntiles || i < a.scan_blocks;
        i += (int64_t)a.shade_blocks * kShadeBlock) {
-    if (i < a.ntiles) {
-      a.tile_count[(size_t)i * kCtrStride64] = 0;
-      a.tile_count[(size_t)i * kCtrStride64 + 1] = 0;
-      a.tile_done[i] = 0;
-    }
+    if (i < a.ntiles) zero_tile(a, (int)i);
     if (i < a.scan_blocks) a.scan_status[i] = 0;
   }
   if (!one_draw) __syncthreads();
@@ -2006,11 +2151,148 @@ __device__ __forceinline__ void stage_shade(const BatchArgs& a, int vb, bool rem
   // After a bin-list or part-list overflow some tiles were not rastered (their
   // winner ids are stale): nothing is shaded, the batch is re-run.
   const bool overflow = a.counters[kBinOverflow] != 0ull || a.counters[kHeavyOverflow] != 0ull;
-  if (inside && !overflow) shade_pixel(a, J, dcache, ncached, id, c, row);
+  if (inside && !overflow) shade_pixel<true>(a, J, dcache, ncached, id, c, row);
 }
 
 __global__ __launch_bounds__(kShadeBlock, 7) void k_shade(BatchArgs a) {
   stage_shade(a, blockIdx.x, true);
+}
+
+// ---- small batches ----------------------------------------------------------
+//
+// Raster and shading of a batch whose tiles test the job's items themselves
+// (no counting, scan or binning, and no kernel boundary before shading): one
+// workgroup per tile tests the boxes of its job's regions, then the items of
+// the regions its tile meets, kSmallRound regions at a time, draws those whose
+// bbox meets the tile from the setup records geometry wrote and shades its
+// pixels.  The frames this is for are bound by the chain of launches and of
+// dependent loads in each; no edge checkpoints are taken (their rows are at
+// most kSmallWidth steps).
+constexpr int kSmallRound = 16;
+
+template <int TW, int NT>
+__global__ __launch_bounds__(NT, 4) void k_small(BatchArgs a) {
+  constexpr int TH = TW, NP = TW * TH, NW = NT / 64, KS = RasterLds<TW, TH, NT>::KS;
+  __shared__ RasterLds<TW, TH, NT> lds;
+  __shared__ int64_t dcache[kMaxLdsDraws];
+  __shared__ uint16_t regs[kSmallRegions];           // regions met, from the job's first on
+  __shared__ uint16_t match[kSmallRound * kRegion];  // items met: (place in the round, slot)
+  __shared__ uint32_t nregs, nmatch;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = (int)blockIdx.x;  // (neighbours on other XCDs: an even share of the frame)
+  const int j = __builtin_amdgcn_readfirstlane(
+      job_lookup(a.tile_hint, a.job_tile_base, a.njobs, tile));
+  // What testing needs of the job; shading reads all of it, again, below.
+  typedef const __attribute__((address_space(4))) JobDesc* ConstJob;
+  const ConstJob cj = (ConstJob)(a.jobs + j);
+  const int tiles_x = cj->tiles_x, local = tile - cj->tile_base;
+  const int draw0 = cj->draw_begin, ndraws = cj->draw_end - draw0;
+  const int tyi = local / tiles_x, txi = local - tyi * tiles_x;
+  const int x0 = txi * TW, y0 = tyi * TH;
+  const int64_t r0 = cj->tri_begin >> 6;
+  const int nr = cj->tri_end > cj->tri_begin ? (int)(((cj->tri_end + 63) >> 6) - r0) : 0;
+  if (tid == 0) nregs = nmatch = 0;
+  for (int p = tid; p < TH * KS; p += NT) lds.keys[p] = ~0ull;
+  __syncthreads();
+  const u64 lt = (1ull << lane) - 1ull;
+  auto append = [&](uint32_t* n, uint16_t* list, bool hit, uint32_t what) {
+    const u64 m = __ballot(hit);
+    if (m == 0ull) return;
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(n, (uint32_t)__popcll(m));
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    if (hit) list[at + __popcll(m & lt)] = (uint16_t)what;
+  };
+  auto meets = [&](uint32_t bx, uint32_t by) {  // first | last << 16
+    return (int)(bx & 0xFFFFu) < x0 + TW && (int)(bx >> 16) >= x0 &&
+           (int)(by & 0xFFFFu) < y0 + TH && (int)(by >> 16) >= y0;
+  };
+  for (int i = tid; i - tid < nr; i += NT) {
+    const uint2 box = a.region_box[r0 + min(i, nr - 1)];
+    append(&nregs, regs, i < nr && meets(box.x, box.y), (uint32_t)i);
+  }
+  __syncthreads();
+  const int met = (int)nregs;
+  for (int q0 = 0; q0 < met; q0 += kSmallRound) {
+    constexpr int kAhead = kSmallRound / NW;  // regions in flight per wavefront
+    // (Every slot of a region is allocated; those past its count are read and
+    // not used: loads under conditions wait for each other.)
+    uint4 it[kAhead];
+    uint32_t cnt[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; i++) {
+      const int64_t r = r0 + regs[min(q0 + wave * kAhead + i, met - 1)];
+      it[i] = ((const uint4*)a.items)[r * kRegion + lane];  // {id, draw, columns, rows}
+      cnt[i] = a.region_count[r];
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; i++) {
+      const int q = wave * kAhead + i;
+      // (A region at the job's first or last triangle may hold a neighbour's.)
+      append(&nmatch, match,
+             q0 + q < met && (uint32_t)lane < cnt[i] && it[i].y - (uint32_t)draw0 < (uint32_t)ndraws &&
+                 meets(it[i].z, it[i].w),
+             (uint32_t)(q * kRegion + lane));
+      if (q0 + q < met && __builtin_amdgcn_readfirstlane((int)cnt[i]) > 64) {
+        // near-clipped triangles make two items
+        const int64_t r = r0 + regs[q0 + q];
+        const uint4 x = ((const uint4*)a.items)[r * kRegion + 64 + lane];
+        append(&nmatch, match,
+               64u + lane < cnt[i] && x.y - (uint32_t)draw0 < (uint32_t)ndraws && meets(x.z, x.w),
+               (uint32_t)(q * kRegion + 64 + lane));
+      }
+    }
+    __syncthreads();
+    const uint32_t n = nmatch;
+    for (uint32_t base = 0; base < n; base += NT) {
+      uint2 be = make_uint2(0, 0);
+      if (base + tid < n) {
+        const uint32_t m = match[base + tid];
+        be.x = (uint32_t)((r0 + regs[q0 + m / kRegion]) * kRegion + m % kRegion);
+      }
+      raster_chunk<TW, TH, NT, true>(a, a.jobs[j], lds, base + tid < n, be, x0, y0, 0, TH - 1);
+    }
+    if (n == 0) __syncthreads();
+    if (tid == 0) nmatch = 0;
+    __syncthreads();
+  }
+  int js = j;
+  asm volatile("" : "+s"(js));  // (the job's registers are live from here only)
+  const JobDesc J = uniform_job(a, js);
+  const bool one_draw = ndraws == 1;
+  const int ncached = one_draw ? -1 : fill_draw_cache(dcache, a, J, tid, NT);
+  __syncthreads();
+  for (int p = tid; p < NP; p += NT) {
+    const int c = x0 + p % TW, row = y0 + p / TW;
+    const u64 key = lds.keys[(p / TW) * KS + p % TW];
+    if (c < J.W && row < J.H)
+      shade_pixel<false>(a, J, dcache, ncached, key == ~0ull ? kNoWinner : (uint32_t)key, c, row);
+  }
+  if (blockIdx.x != 0 || !a.host_counters) return;
+  // Statistics of the batch, to the host (the batch counters are not used).
+  const int ng = geom_grid(a);
+  u64 clipped = 0, items = 0, pairs = 0;
+  for (int i = tid; i < ng; i += NT) {
+    clipped += a.block_stats[i];
+    items += a.block_stats[kStatSlots + i] >> 32;
+    pairs += a.block_stats[kStatSlots + i] & 0xFFFFFFFFull;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    clipped += __shfl_xor(clipped, o);
+    items += __shfl_xor(items, o);
+    pairs += __shfl_xor(pairs, o);
+  }
+  __shared__ u64 sums[3][NW];
+  if (lane == 0) sums[0][wave] = clipped, sums[1][wave] = items, sums[2][wave] = pairs;
+  __syncthreads();
+  if (tid < kNumCounters) {
+    u64 v = 0;
+    const int k = tid == kClipped ? 0 : tid == kItems ? 1 : tid == kBinEntries ? 2 : -1;
+    for (int w = 0; w < NW && k >= 0; w++) v += sums[k][w];
+    a.host_counters[tid] = v;
+  }
 }
 
 // ---- the persistent kernel --------------------------------------------------
@@ -2096,7 +2378,7 @@ __device__ __forceinline__ void persist_run(const BatchArgs& a, const PersistPla
   switch (s) {
     case kPClear: stage_clear(a, (int)vb, q.nvb[s]); break;
     case kPVertex: stage_vertex(a, (int)vb, q.nvb[s]); break;
-    case kPGeom: stage_geom(a, (int)vb, q.nvb[s]); break;
+    case kPGeom: stage_geom<false, false>(a, (int)vb, q.nvb[s]); break;
     case kPScan: stage_scan(a); break;
     case kPBin:
       stage_direct(a, (int)vb, q.nvb[s]);
@@ -2345,6 +2627,28 @@ hipError_t launch_vertex(const BatchArgs& a, hipStream_t s) {
 hipError_t launch_geometry(const BatchArgs& a, hipStream_t s) {
   if (a.total_tris == 0) return hipSuccess;
   hipLaunchKernelGGL(k_geom, dim3(geom_grid(a)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_front(const BatchArgs& a, const void* tables, size_t table_bytes,
+                        hipStream_t s) {
+  TableArgs t;
+  static_assert(sizeof(TableArgs) <= 4096, "kernel arguments hold 4 KiB");
+  t.a = a;
+  t.nwords = 0;
+  if (tables && table_bytes <= sizeof(t.words)) {
+    memcpy(t.words, tables, table_bytes);
+    t.nwords = (uint32_t)(table_bytes / 4);
+  }
+  if (a.small) hipLaunchKernelGGL(k_front<true>, dim3(geom_grid(a)), dim3(256), 0, s, t);
+  else hipLaunchKernelGGL(k_front<false>, dim3(geom_grid(a)), dim3(256), 0, s, t);
+  return hipGetLastError();
+}
+
+hipError_t launch_small(const BatchArgs& a, hipStream_t s) {
+  if (a.tile_w == 8) hipLaunchKernelGGL((k_small<8, 64>), dim3(a.ntiles), dim3(64), 0, s, a);
+  else if (a.tile_w == 16) hipLaunchKernelGGL((k_small<16, 256>), dim3(a.ntiles), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((k_small<32, 256>), dim3(a.ntiles), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

@@ -4,19 +4,24 @@
 #include <hip/hip_runtime.h>
 
 #include "common.h"
+#include "exact.h"
 
 namespace mr {
+
+// The setup of an item and its id.
+struct alignas(16) SetupRec {
+  TriSetup s;
+  uint32_t id;
+};
+static_assert(sizeof(SetupRec) == 64, "one record per 64 bytes");
 
 // Device buffers and sizes of one batch.
 struct BatchArgs {
   BinItem* items;            // [nregions * kRegion] survivors, per wavefront
   uint32_t* region_count;    // [nregions] survivors of each wavefront
-  // Direct items of each job, and per job a line of words: their number
-  // (which may exceed the list), then kMaxDim - first column, last column,
-  // kMaxDim - first row and last row of their bounding box.  Both lie behind
-  // the checkpoints, in the checkpoint buffer's last quarter.
+  // Direct items of each job, behind the checkpoints in the checkpoint
+  // buffer's last quarter (their number: direct_line in kernels.hip).
   BinItem* direct;           // [njobs * direct_cap]
-  uint32_t* direct_count;    // [njobs * kCtrStride], null when direct_cap is 0
   uint32_t direct_cap;
   int64_t nregions;
   // [ntiles * kCtrStride64] per tile: (walk work << 32) | (tile, triangle)
@@ -98,7 +103,42 @@ struct BatchArgs {
   // kernel, which reads the items anyway, with the row pre-pass a launch of
   // its own.
   int32_t ckpt_in_scan;
+  // Setups of the items of a small batch, by item slot (in the checkpoint
+  // buffer, which such a batch does not use).
+  SetupRec* recs;
+  uint2* region_box;         // behind them: {first | last << 16} column, row of each
+                             // region's items
+  // The kernels of the batch (launched stages).  front: geometry transforms
+  // the vertices itself (k_front) and needs the batch counters zero before.
+  // small: front, and the tiles test the items themselves (k_small).
+  int32_t front, small;
 };
+
+// The argument of a batch's first kernel: with nwords, the batch tables too.
+constexpr int kInlineWords = 832;
+struct TableArgs {
+  BatchArgs a;
+  uint32_t nwords;
+  alignas(16) uint32_t words[kInlineWords];
+};
+
+// Batches of at most this many triangles run k_front: beyond, transforming
+// each vertex once costs less than once per corner (vertex and geometry
+// kernels together 16.3 -> 12.0 us at 120 k triangles, 35 -> 32.5 at 1 M, but
+// 55 -> 61 at 2.1 M).
+constexpr int64_t kFrontTris = 1500000;
+// Small batches: frames at most kSmallWidth wide (rows are walked from the
+// bbox's left column), at most kSmallTiles tiles (beyond a few rounds of
+// workgroups throughput counts, not latency), which test at most kSmallTests
+// regions together when every region meets every tile (triangles in random
+// order).  Against the general kernels (a frame's call, us): sphere of 4 k
+// triangles at 640 x 480 59 -> 33, grid of 5 k at 1000 x 1000 83 -> 57, 1,000
+// large overlapping triangles at 640 x 480 78 -> 51, 2,500 of them at 1000 x 600
+// 129 -> 133; a batch of 40 frames of 250 x 250 (10,240 tiles) 121 -> 130.
+constexpr int kSmallWidth = 1024;
+constexpr int kSmallTiles = 8192;
+constexpr int64_t kSmallTests = 800000;
+constexpr int kSmallRegions = 2048;  // of one job at most (k_small lists them in LDS)
 
 constexpr int64_t kCkptScanRegions = 65536;
 
@@ -143,6 +183,10 @@ __host__ __device__ inline int32_t direct_grid(const BatchArgs& a) {
 hipError_t launch_clear(const BatchArgs& a, hipStream_t s);
 hipError_t launch_vertex(const BatchArgs& a, hipStream_t s);
 hipError_t launch_geometry(const BatchArgs& a, hipStream_t s);
+// The batch's first kernel when a.front; tables (host memory) go inside its
+// argument when they fit there, else they have been uploaded.
+hipError_t launch_front(const BatchArgs& a, const void* tables, size_t table_bytes, hipStream_t s);
+hipError_t launch_small(const BatchArgs& a, hipStream_t s);  // raster and shading when a.small
 hipError_t launch_scan(const BatchArgs& a, hipStream_t s);
 hipError_t launch_bin(const BatchArgs& a, hipStream_t s);
 hipError_t launch_rows(const BatchArgs& a, hipStream_t s);  // nothing when ckpt_in_scan

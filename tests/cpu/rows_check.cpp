@@ -2,13 +2,16 @@
 // slivers, vertices far beyond the screen, axis-aligned edges) and column ranges, no
 // row it drops covers a pixel in the raster's own walk (edge_start at the
 // bbox's left column, e += n.x per column, Renderer.cpp:238-245), and it
-// drops most rows that cover nothing.  Built with g++ -O2 -ffp-contract=off.
+// drops most rows that cover nothing.  Also: xcd_chunks (common.h) is a
+// bijection on [0, n).  Built with g++ -O2 -ffp-contract=off.
 // Prints "ok" or the first failure.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
+#include <vector>
 
+#include "common.h"
 #include "exact.h"
 
 using namespace mr;
@@ -25,6 +28,16 @@ static double u01() { return (double)(rnd() >> 11) / 9007199254740992.0; }
 int main(int argc, char** argv) {
   const int cases = argc > 1 ? atoi(argv[1]) : 100000;
   st = argc > 2 ? strtoull(argv[2], nullptr, 10) : 1;
+  for (uint32_t n = 1; n < 1200; n++) {
+    std::vector<char> seen(n, 0);
+    for (uint32_t b = 0; b < n; b++) {
+      const uint32_t r = xcd_chunks<kXcdChunk>(b, n);
+      if (r >= n || seen[r]++) {
+        printf("xcd_chunks(%u, %u) = %u\n", b, n, r);
+        return 1;
+      }
+    }
+  }
   long empty = 0, dropped = 0, tested = 0;
   for (int i = 0; i < cases; i++) {
     const float W = (float)(16 + rnd() % 500), H = (float)(16 + rnd() % 300);

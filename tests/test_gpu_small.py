@@ -1,0 +1,132 @@
+"""Small batches (k_front + k_small) against the general kernels and the
+oracle.  The same frames run as a small batch and, in a batch with a frame
+too wide for that, through the general kernels: every output bit for bit.
+The general kernels' special cases (crowded tiles, row bands, several
+triangles per bin) are also run on frames too wide to be small, at the sizes
+the small frames of other tests had them."""
+import math
+
+import numpy as np
+import pytest
+
+import minirender_amd as mra
+from minirender_amd import scenes
+from minirender_amd.scenes import Draw, FrameSpec, Material
+from oracle import oracle_py
+from tests.parity import assert_parity, fuzz_frame, stack_frame
+
+pytestmark = pytest.mark.gpu
+ALL = ("rgb8", "depth", "winner", "rgb", "normals", "points")
+KINDS = ("rgb8", "depth", "winner")
+
+
+def wide():
+    """A frame wider than a small batch's may be."""
+    return FrameSpec(1030, 8, scenes.projection_frustum(1.0, 128, 0.1, 10),
+                     draws=[Draw(scenes.create_cube(1.0), Material(), scenes.translate(0, 0, -3))])
+
+
+def same(g, ref, kinds, what):
+    for k in kinds:
+        assert np.array_equal(g[k].view(np.uint8), ref[k].view(np.uint8)), (what, k)
+
+
+@pytest.mark.parametrize("tile", [8, 16, 32])
+def test_small_equals_general(gpu_ctx, tile):
+    frames = [fuzz_frame(s, 61 + 13 * (s % 9), 47 + 17 * (s % 7)) for s in range(900, 918)]
+    tris = scenes.random_triangles(70, 5, lo=0.2, hi=1.5, center_lo=(-1, -1, -3), center_hi=(1, 1, -1))
+    frames.append(FrameSpec(1024, 33, scenes.projection_frustum(1.0, 31.0, 0.5, 50.0),
+                            draws=[Draw(tris, Material(), no_clip=True), Draw(tris, Material())]))
+    frames.append(scenes.config_sphere(333, 250))
+    gpu_ctx.set_tile(tile, tile)
+    try:
+        for i, f in enumerate(frames):
+            small = gpu_ctx.render(f, ALL)
+            assert gpu_ctx.stats().launches == 2, i
+            pairs = gpu_ctx.stats().bin_entries
+            general = gpu_ctx.render_batch([f, wide()], ALL)[0]
+            assert gpu_ctx.stats().launches > 2, i
+            assert gpu_ctx.stats().bin_entries >= pairs
+            same(small, general, [k for k in ALL if k != "normals" or f.save_normals], f"frame {i}")
+        # as one batch: regions that two jobs share
+        out = gpu_ctx.render_batch(frames[:6], ALL)
+        assert gpu_ctx.stats().launches == 2
+        for i, f in enumerate(frames[:6]):
+            same(out[i], gpu_ctx.render_batch([f, wide()], ALL)[0],
+                 [k for k in ALL if k != "normals" or f.save_normals], f"batch job {i}")
+    finally:
+        gpu_ctx.set_tile(16, 16)
+
+
+def test_more_items_than_a_round(gpu_ctx):
+    """Thousands of items over one tile, some near-clipped into two: several
+    rounds of regions, several chunks of matches."""
+    tris = scenes.random_triangles(5000, 3, lo=0.02, hi=0.6, center_lo=(-0.3, -0.3, -1.2),
+                                   center_hi=(0.3, 0.3, -0.3))
+    f = FrameSpec(70, 50, scenes.projection_frustum(1.0, 1.4, 0.5, 20.0),
+                  draws=[Draw(tris, Material(shininess=9.0))], light=(0.2, 0.4, 1.0))
+    for tile in (8, 32):
+        gpu_ctx.set_tile(tile, tile)
+        try:
+            g = gpu_ctx.render(f, KINDS)
+            assert gpu_ctx.stats().launches == 2
+        finally:
+            gpu_ctx.set_tile(16, 16)
+        assert_parity(g, oracle_py.render(f, KINDS), f"rounds t{tile}")
+
+
+def test_small_and_general_take_turns(gpu_ctx):
+    """The counters a general batch expects zero stay so across small batches,
+    an overflow's re-run, an empty frame and the persistent kernel."""
+    small, big = scenes.config_sphere(160, 120), fuzz_frame(7, 1100, 300)
+    empty = FrameSpec(40, 30, scenes.projection_frustum(1.0, 4 / 3, 0.1, 10))
+    ref = {id(f): oracle_py.render(f, KINDS) for f in (small, big, empty)}
+    with mra.Context(0) as ctx:
+        for step, f in enumerate((small, big, small, big, empty, small, big, big, empty, big)):
+            ctx.set_bin_factor(1.0 if step == 1 else 3.0)
+            ctx.set_persistent(step == 7)
+            assert_parity(ctx.render(f, KINDS), ref[id(f)], f"step {step}")
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+def test_tables_in_the_argument_or_uploaded(graphs):
+    """Batch tables inside the first kernel's argument (few draws) and uploaded
+    (many), eager and captured: frames that differ only in their tables."""
+    def frame(n, shift):
+        cube = scenes.create_cube(0.4)
+        draws = [Draw(cube, Material(diffuse=(0.1 * (i % 9), 0.5, 0.9)),
+                      scenes.translate(0.31 * (i % 6) - 0.8 + shift, 0.33 * (i // 6) - 0.8, -3.0 - 0.01 * i))
+                 for i in range(n)]
+        return FrameSpec(130, 97, scenes.projection_frustum(1.0, 1.34, 0.1, 20.0), draws=draws)
+
+    with mra.Context(0) as ctx:
+        ctx.set_graphs(graphs)
+        for rep in range(3):
+            for n in (1, 5, 31):
+                for shift in (0.0, 0.17):
+                    f = frame(n, shift)
+                    assert_parity(ctx.render(f, KINDS), oracle_py.render(f, KINDS), f"{n} {shift} {rep}")
+
+
+@pytest.mark.parametrize("tile", [8, 16, 32])
+def test_general_special_cases(gpu_ctx, tile):
+    """Row bands, split tiles and several rounds on frames that are not small."""
+    tris = scenes.random_triangles(40, 21, lo=0.2, hi=1.5, center_lo=(-1, -1, -3), center_hi=(1, 1, -2))
+    large = FrameSpec(1100, 620, scenes.projection_frustum(math.radians(60), 16 / 9, 0.1, 50.0),
+                      draws=[Draw(tris, Material(shininess=40.0))], light=(0.3, 0.5, 1.0))
+    gpu_ctx.set_tile(tile, tile)
+    try:
+        for band, frag, f, what in ((64, 1024, fuzz_frame(110, 1060, 100), "bands"),
+                                    (64, 1024, large, "bands large"),
+                                    (64, 64, scenes.config_terrain(n=96, width=1040, height=180), "bands terrain"),
+                                    (32768, 64, stack_frame(500, 1040, 24, seed=tile), "split"),
+                                    (32768, 1024, fuzz_frame(111, 1060, 100), "plain")):
+            gpu_ctx.set_band_work(band)
+            gpu_ctx.set_frag_size(frag)
+            g = gpu_ctx.render(f, KINDS)
+            assert gpu_ctx.stats().launches > 2
+            assert_parity(g, oracle_py.render(f, KINDS), f"{what} t{tile}")
+    finally:
+        gpu_ctx.set_band_work(32768)
+        gpu_ctx.set_frag_size(1024)
+        gpu_ctx.set_tile(16, 16)
