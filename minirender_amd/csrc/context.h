@@ -93,6 +93,9 @@ struct BatchPlan {
   TableLayout layout;
 };
 
+// Chunks of host outputs in flight at once (mr_render, mr_render_batch).
+constexpr int kReadRing = 8;
+
 // An execution slot: scratch, stream and events for one batch in flight.
 struct Slot {
   Scratch sc;
@@ -100,6 +103,7 @@ struct Slot {
   hipStream_t own_stream = nullptr;
   hipEvent_t ev[kStages + 1] = {};  // stage boundaries (profiling)
   hipEvent_t done = nullptr;
+  hipEvent_t read[kReadRing] = {};  // chunks of the outputs read back (created on first use)
   void* h_counters_dev = nullptr;  // device address of sc.h_counters ...
   void* h_counters_of = nullptr;   // ... for this host buffer
   uint32_t heavy_slots = 0;  // merge buffers of split tiles (grown on demand)
@@ -169,8 +173,6 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile);
 // Wait for s.done, handle bin-list / merge-slot overflow by growing and
 // re-running, and record statistics.
 int finish_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile);
-// Copy host outputs back from the slot's staging (synchronous).
-int copy_outputs(mr_ctx* c, Slot& s, const BatchPlan& p, const mr_outputs* outs,
-                 const std::vector<size_t>& staging_offs);
+// A synchronous batch with its outputs where the caller wants them.
 int render_frames(mr_ctx* c, const mr_frame* frames, int n, const mr_outputs* outs);
 }  // namespace mr
