@@ -492,6 +492,16 @@ static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
   return MR_OK;
 }
 
+// Device address (null: none) of a pinned buffer, looked up when it changes.
+static void device_address(const HostBuf& b, void*& of, void*& dev) {
+  if (of == b.p) return;
+  void* d = nullptr;
+  dev = nullptr;
+  if (hipHostGetDevicePointer(&d, b.p, 0) == hipSuccess) dev = d;
+  else (void)hipGetLastError();
+  of = b.p;
+}
+
 static uint64_t bins_wanted(mr_ctx* c, const Slot& s, const BatchPlan& p) {
   uint64_t want = std::max<uint64_t>(
       (uint64_t)((double)p.total_tris * c->bin_factor) + (uint64_t)p.ntiles, 1u << 16);
@@ -531,13 +541,7 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   // (the persistent kernel sets its error word after shading: it keeps the
   // copy).
   if (!persistent) {
-    if (s.h_counters_of != x.h_counters.p) {
-      void* d = nullptr;
-      s.h_counters_dev = nullptr;
-      if (hipHostGetDevicePointer(&d, x.h_counters.p, 0) == hipSuccess) s.h_counters_dev = d;
-      else (void)hipGetLastError();
-      s.h_counters_of = x.h_counters.p;
-    }
+    device_address(x.h_counters, s.h_counters_of, s.h_counters_dev);
     a.host_counters = (unsigned long long*)s.h_counters_dev;
   }
   s.last_geom_grid = p.total_tris ? geom_grid(a) : 0;
@@ -569,12 +573,15 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   const bool prev_counters = s.clean_counters;
   s.clean_tiles = s.clean_scan = 0;  // until the launches below succeed
   // Eager launches of a batch that starts with k_front hand it small tables
-  // in its argument; a captured batch reads them from the staging when it is
-  // replayed.
+  // in its argument, and k_tables fetches larger ones from the staging; a
+  // captured batch copies them from the staging when it is replayed.
   const bool capture = c->graphs && !profile && s.own_stream && s.stream == s.own_stream;
   const bool inl = a.front && !capture && p.layout.bytes <= kInlineWords * 4;
+  if (!inl && !capture) device_address(x.h_tables, s.h_tables_of, s.h_tables_dev);
   auto issue = [&]() -> int {
-    if (!inl)
+    if (!inl && !capture && s.h_tables_dev)
+      HIP_TRY(launch_tables(s.h_tables_dev, x.tables.p, p.layout.bytes, s.stream));
+    else if (!inl)
       HIP_TRY(hipMemcpyAsync(x.tables.p, x.h_tables.p, p.layout.bytes, hipMemcpyHostToDevice,
                              s.stream));
     int r = launch_stages(a, s, profile, clear, persistent, c->wait_us,

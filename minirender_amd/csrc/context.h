@@ -104,8 +104,11 @@ struct Slot {
   hipEvent_t ev[kStages + 1] = {};  // stage boundaries (profiling)
   hipEvent_t done = nullptr;
   hipEvent_t read[kReadRing] = {};  // chunks of the outputs read back (created on first use)
-  void* h_counters_dev = nullptr;  // device address of sc.h_counters ...
-  void* h_counters_of = nullptr;   // ... for this host buffer
+  // Device addresses of pinned buffers, and the host buffers they are of.
+  void* h_counters_dev = nullptr;
+  void* h_counters_of = nullptr;
+  void* h_tables_dev = nullptr;
+  void* h_tables_of = nullptr;
   uint32_t heavy_slots = 0;  // merge buffers of split tiles (grown on demand)
   size_t parts_want = 0;     // raster work items a batch needed (after an overflow)
   int32_t last_geom_grid = 0, last_bin_grid = 0;

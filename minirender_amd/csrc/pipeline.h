@@ -180,6 +180,8 @@ __host__ __device__ inline int32_t direct_grid(const BatchArgs& a) {
   return steps < 1024 ? steps : 1024;
 }
 
+// Copy the batch tables (TableLayout: a multiple of 16 bytes) from pinned host memory.
+hipError_t launch_tables(const void* pinned, void* tables, size_t bytes, hipStream_t s);
 hipError_t launch_clear(const BatchArgs& a, hipStream_t s);
 hipError_t launch_vertex(const BatchArgs& a, hipStream_t s);
 hipError_t launch_geometry(const BatchArgs& a, hipStream_t s);
