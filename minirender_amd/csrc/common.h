@@ -89,7 +89,6 @@ static_assert(sizeof(BinItem) == 16, "BinItem must be 16 bytes");
 // Device counters of a batch (64-bit, cleared by the clear kernel).
 enum Counter : int {
   kItems = 0,        // surviving (sub-)triangles (statistics)
-  kScanTicket = 1,
   kBinOverflow = 2,  // set when the bin list was too small
   kError = 3,        // set when a bounded wait hit its limit
   kClipped = 4,      // input triangles that crossed the near plane
@@ -173,11 +172,9 @@ constexpr int kShadeW = 16;        // shading block: kShadeW x kShadeH pixels
 constexpr int kShadeH = kShadeBlock / kShadeW;
 constexpr int kMaxLdsDraws = 256;  // draw-table entries cached in LDS
 
-// Bounded waits (decoupled look-back): polls before giving up with kError.
-constexpr uint32_t kSpinLimit = 1u << 22;
-
 constexpr int kScanBlock = 256;
-constexpr int kScanItems = 8;    // elements per thread in the tile-count scan
+constexpr int kScanItems = 8;    // tiles per thread in the tile-count scan ...
+constexpr int kScanWide = 16384; // ... of more tiles than this; one up to it
 constexpr uint32_t kNoWinner = 0xFFFFFFFFu;
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 constexpr uint32_t kEmptyTile = 0xFFFFFFFEu;  // tile_heavy of a tile with no bin entry

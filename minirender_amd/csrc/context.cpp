@@ -110,7 +110,7 @@ void slot_free(mr_ctx* c, Slot& s) {
   Scratch& x = s.sc;
   DevBuf* bufs[] = {&x.items, &x.region_count, &x.tile_count, &x.tile_off,
                     &x.tile_cursor, &x.tile_heavy, &x.tile_list, &x.tile_done, &x.parts, &x.bins,
-                    &x.ckpt_base, &x.ckpt, &x.ckpt_ctr, &x.heavy_keys, &x.scan_status, &x.counters, &x.block_stats,
+                    &x.ckpt_base, &x.ckpt, &x.ckpt_ctr, &x.heavy_keys, &x.counters, &x.block_stats,
                     &x.tables, &x.vrec, &x.win, &x.wide, &x.outputs, &x.ctl};
   for (DevBuf* b : bufs) dev_free(c, *b, true);
   HostBuf* hbufs[] = {&x.h_tables, &x.h_counters, &x.h_outputs};
@@ -288,12 +288,11 @@ static size_t ckpt_entries(int64_t npixels) { return (size_t)npixels * 2 + 65536
 
 // Device scratch of a batch, buffer by buffer (bytes), in the order of
 // scratch_bufs().
-constexpr int kScratchBufs = 21;
+constexpr int kScratchBufs = 20;
 
 static void scratch_sizes(mr_ctx* c, const BatchPlan& p, uint64_t bins_cap, uint32_t heavy_slots,
                           size_t parts_want, size_t out[kScratchBufs]) {
   const int64_t T = p.total_tris;
-  const int scb = scan_blocks_for((int32_t)p.ntiles);
   const size_t nt = (size_t)p.ntiles * 4;
   const int64_t nregions = std::max<int64_t>((T + 63) / 64, 1);
   const size_t npt = (size_t)c->tile_w * c->tile_h * 8;
@@ -317,7 +316,6 @@ static void scratch_sizes(mr_ctx* c, const BatchPlan& p, uint64_t bins_cap, uint
       ckpt_entries(p.npixels) * 8,                   // ckpt
       (size_t)kCkptSegs * kCtrStride * 8,            // ckpt_ctr
       (size_t)heavy_slots * npt,                     // heavy_keys
-      (size_t)std::max(scb, 1) * 8,                  // scan_status
       (size_t)kNumCounters * 8,                      // counters
       (size_t)2 * kStatSlots * 8,                    // block_stats
       p.layout.bytes,                                // tables
@@ -332,7 +330,7 @@ static void scratch_bufs(Scratch& x, DevBuf* b[kScratchBufs]) {
   DevBuf* v[kScratchBufs] = {&x.items, &x.region_count, &x.tile_count, &x.tile_off,
                              &x.tile_cursor, &x.tile_heavy, &x.tile_list, &x.tile_done,
                              &x.parts, &x.bins, &x.ckpt_base, &x.ckpt, &x.ckpt_ctr,
-                             &x.heavy_keys, &x.scan_status, &x.counters, &x.block_stats,
+                             &x.heavy_keys, &x.counters, &x.block_stats,
                              &x.tables, &x.vrec, &x.win, &x.wide};
   for (int k = 0; k < kScratchBufs; k++) b[k] = v[k];
 }
@@ -406,7 +404,6 @@ static BatchArgs make_args(mr_ctx* c, Slot& sl, const BatchPlan& p) {
   a.heavy_cap = (uint32_t)(s.heavy_keys.bytes / ((size_t)c->tile_w * c->tile_h * 8));
   a.frag_size = c->frag_size;
   a.band_work = c->band_work;
-  a.scan_status = (unsigned long long*)s.scan_status.p;
   a.counters = (unsigned long long*)s.counters.p;
   a.block_stats = (unsigned long long*)s.block_stats.p;
   char* tb = (char*)s.tables.p;
@@ -559,19 +556,17 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   // (which clears the batch counters) and no shading kernel that left them
   // zero.  A small batch uses none of them.
   const bool same_bufs = s.clean_ref[0] == x.tile_count.p && s.clean_ref[1] == x.tile_done.p &&
-                         s.clean_ref[2] == x.scan_status.p && s.clean_ref[3] == x.counters.p &&
-                         s.clean_ref[4] == x.ckpt_ctr.p;
+                         s.clean_ref[2] == x.counters.p && s.clean_ref[3] == x.ckpt_ctr.p;
   const bool clear = !a.small &&
                      (!same_bufs || p.total_tris == 0 || p.ntiles > s.clean_tiles ||
-                      a.scan_blocks > s.clean_scan || (a.front && !s.clean_counters));
+                      (a.front && !s.clean_counters));
   // Zero prefixes after this batch: the clear kernel (if run) zeroes this
   // batch's range, the shading kernel re-zeroes it, entries past it keep
   // their state.
   const int64_t next_tiles = std::max<int64_t>(p.ntiles, same_bufs ? s.clean_tiles : 0);
-  const int64_t next_scan = std::max<int64_t>(a.scan_blocks, same_bufs ? s.clean_scan : 0);
-  const int64_t prev_tiles = s.clean_tiles, prev_scan = s.clean_scan;
+  const int64_t prev_tiles = s.clean_tiles;
   const bool prev_counters = s.clean_counters;
-  s.clean_tiles = s.clean_scan = 0;  // until the launches below succeed
+  s.clean_tiles = 0;  // until the launches below succeed
   // Eager launches of a batch that starts with k_front hand it small tables
   // in its argument, and k_tables fetches larger ones from the staging; a
   // captured batch copies them from the staging when it is replayed.
@@ -669,17 +664,14 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   HIP_TRY(hipEventRecord(s.done, s.stream));
   if (a.small) {  // left as they were
     s.clean_tiles = prev_tiles;
-    s.clean_scan = prev_scan;
     s.clean_counters = prev_counters;
     return MR_OK;
   }
   s.clean_ref[0] = x.tile_count.p;
   s.clean_ref[1] = x.tile_done.p;
-  s.clean_ref[2] = x.scan_status.p;
-  s.clean_ref[3] = x.counters.p;
-  s.clean_ref[4] = x.ckpt_ctr.p;
+  s.clean_ref[2] = x.counters.p;
+  s.clean_ref[3] = x.ckpt_ctr.p;
   s.clean_tiles = next_tiles;
-  s.clean_scan = next_scan;
   // The shading kernel that hands the host the counters leaves them zero.
   s.clean_counters = a.host_counters != nullptr;
   return MR_OK;
@@ -693,11 +685,11 @@ int finish_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
     HIP_TRY(hipEventSynchronize(s.done));
     if (hc[kError]) {
       // A bounded wait gave up: stages after it did not run, so the tile
-      // counters and look-back words shading re-zeroes may hold this batch's
+      // counters that shading re-zeroes may hold this batch's
       // values; the next batch clears them first.  The persistent kernel's
       // last workgroup clears its control words in any case; cleared again
       // to be sure.
-      s.clean_tiles = s.clean_scan = 0;
+      s.clean_tiles = 0;
       if (x.ctl.p) HIP_TRY(hipMemset(x.ctl.p, 0, kCtlBytes));
       return MR_ERR_DEVICE;
     }
@@ -930,7 +922,7 @@ static int finish_readback(Slot& s, Readback& rb, bool rerun) {
 // batch tables and counters pass through fixed host arrays per device, and
 // outputs must be device buffers.  Stale contents of the array from earlier
 // calls do not matter: the clear kernel and the geometry kernel zero what
-// must start at zero (counters, look-back words, tile counters, checkpoint
+// must start at zero (counters, tile counters, checkpoint
 // segment counters), and every other buffer is written before it is read.
 constexpr size_t kNoAllocTableBytes = (size_t)1 << 20;
 static char g_na_tables[kMaxDevices][kNoAllocTableBytes];

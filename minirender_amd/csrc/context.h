@@ -53,7 +53,7 @@ struct TexRec {
 // Device scratch of one batch in flight, and its pinned staging.
 struct Scratch {
   DevBuf items, region_count, tile_count, tile_off, tile_cursor, tile_heavy, tile_list,
-      tile_done, parts, bins, ckpt_base, ckpt, ckpt_ctr, heavy_keys, scan_status, counters,
+      tile_done, parts, bins, ckpt_base, ckpt, ckpt_ctr, heavy_keys, counters,
       block_stats, tables, vrec, win, wide, outputs;
   // Control words of the persistent kernel (kCtlBytes, zero between
   // launches), then its stage stamps when profiling (kStampBytes).
@@ -124,9 +124,9 @@ struct Slot {
   };
   std::vector<Graph> graphs;
   int64_t graph_replays = 0, graph_captures = 0;
-  // Leading tile counters / look-back words known to be zero (the shading
+  // Leading tile counters known to be zero (the shading
   // kernel re-zeroes what a batch used), valid for the buffers in clean_ref.
-  int64_t clean_tiles = 0, clean_scan = 0;
+  int64_t clean_tiles = 0;
   bool clean_counters = false;  // batch and checkpoint counters too
   const void* clean_ref[5] = {};
 };

@@ -1,7 +1,7 @@
 // kernels.hip -- the rasterization pipeline of minirender's Renderer::render()
 // (src/Renderer.cpp:311-381) as HIP kernels for gfx950 (wave64).
 //
-//   k_clear   look-back words, tile counts and merge counters when the
+//   k_clear   tile counts and merge counters when the
 //             scratch is new (afterwards the shading kernel leaves them
 //             zero); batch and checkpoint counters when the batch has no
 //             triangles (else the vertex kernel zeroes them)
@@ -16,7 +16,7 @@
 //             (ballot + popcount prefix, no global atomic) and counts its
 //             (tile, triangle) pairs with one atomic per distinct tile.
 //             Triangles over many tiles go to their job's direct list instead
-//   k_scan    (c) exclusive scan of the tile counts (decoupled look-back);
+//   k_scan    (c) offsets of the tiles' ranges from the tile counts;
 //             tiles with more pairs than one work item are split into parts,
 //             the others with pairs listed for the raster, empty ones marked.
 //             Beside the scan the launch's other workgroups match the direct
@@ -65,45 +65,6 @@ namespace mr {
 
 using u64 = unsigned long long;
 
-constexpr u64 kFlagAgg = 1ull << 62;
-constexpr u64 kFlagPre = 2ull << 62;
-constexpr u64 kValMask = (1ull << 62) - 1;
-
-// Decoupled look-back (single thread): publish this block's aggregate, sum
-// predecessors back to the first inclusive prefix, publish ours.  Block ids
-// come from a ticket counter, so every predecessor is already running.
-__device__ u64 lookback(u64* status, int idx, u64 aggregate, u64* counters) {
-  if (idx == 0) {
-    __hip_atomic_store(&status[0], kFlagPre | aggregate, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    return 0;
-  }
-  __hip_atomic_store(&status[idx], kFlagAgg | aggregate, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-  u64 excl = 0;
-  int j = idx - 1;
-  uint32_t spins = 0;
-  while (j >= 0) {
-    const u64 w = __hip_atomic_load(&status[j], __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT);
-    const u64 flag = w >> 62;
-    if (flag == 0) {
-      if (++spins > kSpinLimit) {
-        atomicOr(&counters[kError], 1ull);
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-      continue;
-    }
-    excl += w & kValMask;
-    if (flag == 2) break;
-    --j;
-  }
-  __hip_atomic_store(&status[idx], kFlagPre | (excl + aggregate),
-                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return excl;
-}
-
 // Each stage is a device function of its workgroup index vb in a grid of
 // nvb workgroups of 256 threads: run by its own kernel (vb = blockIdx.x),
 // or by the persistent kernel, whose workgroups take stage work from queues.
@@ -133,11 +94,7 @@ __device__ __forceinline__ void stage_clear(const BatchArgs& a, int vb, int nvb)
   // (A batch without triangles runs no vertex kernel, which zeroes them
   // otherwise: it must not leave the row pre-pass the last batch's tasks.)
   if (vb == 0) zero_counters(a);
-  const int n = max(a.scan_blocks, a.ntiles);
-  for (int i = vb * 256 + (int)threadIdx.x; i < n; i += nvb * 256) {
-    if (i < a.scan_blocks) a.scan_status[i] = 0;
-    if (i < a.ntiles) zero_tile(a, i);
-  }
+  for (int i = vb * 256 + (int)threadIdx.x; i < a.ntiles; i += nvb * 256) zero_tile(a, i);
 }
 
 __global__ __launch_bounds__(256) void k_clear(BatchArgs a) {
@@ -917,29 +874,45 @@ __device__ inline uint32_t band_count(const BatchArgs& a, uint32_t cnt, uint32_t
   return nb >= 2 ? nb : 0;
 }
 
-// (c) exclusive scan of (tile, triangle) pairs per tile -> offsets and
-// cursors; tiles with more than frag_size pairs get a merge slot and their
-// parts are listed for the raster, tiles with much walk work their row
-// bands.
-__device__ __forceinline__ void stage_scan(const BatchArgs& a) {
-  __shared__ int sh_blk;
-  __shared__ u64 sh_w[kScanBlock / 64];
-  __shared__ u64 sh_excl;
+// (c) (tile, triangle) pairs per tile -> offsets and cursors; tiles with more
+// than frag_size pairs get a merge slot and their parts are listed for the
+// raster, tiles with much walk work their row bands.  Bound by its chain of
+// trips to memory: the counts, one round of atomics, the stores.  A workgroup
+// sums its tiles and reserves their ranges of the bin list, merge slots, part
+// list and tile list with one atomic each, in one instruction; in which order
+// the workgroups' ranges lie does not matter.  Frames have few tiles: one per
+// thread spreads the scattered lines of the counters over the most CUs
+// (kScanWide), where batches of many tiles would queue at the atomics (about
+// 11 ns each).  Against a prefix sum in tile order (a ticket, a look-back over
+// the workgroups and three atomics one after the other, 8 tiles per thread):
+// launch of 8,160 tiles 15 -> 8 us, of 2,772 14 -> 8, of 130,560 (64 frames)
+// 23 -> 18; and shading, which had the look-back words to zero, 1034 -> 954
+// us on those 64 frames.
+template <int kItems>
+__device__ __forceinline__ void stage_scan(const BatchArgs& a, int blk) {
+  constexpr int NW = kScanBlock / 64;
+  __shared__ u64 sh_w[NW], sh_base[4];
+  __shared__ uint32_t sh_h[NW], sh_p[NW], sh_l[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const u64 ndirect = a.counters[kDirect];  // in flight with the tile counts
-  // (A single workgroup needs no ticket: it is workgroup 0.)
-  if (tid == 0) sh_blk = a.scan_blocks == 1 ? 0 : (int)atomicAdd(&a.counters[kScanTicket], 1ull);
-  __syncthreads();
-  const int blk = sh_blk;
-  const int base = blk * (kScanBlock * kScanItems) + tid * kScanItems;
-  uint32_t v[kScanItems], nbv[kScanItems];
+  const int base = blk * (kScanBlock * kItems) + tid * kItems;
+  uint32_t v[kItems], nbv[kItems];
   u64 sum = 0;
+  uint32_t nh = 0, npt = 0, nl = 0;  // split tiles, parts, tiles rastered whole
 #pragma unroll
-  for (int i = 0; i < kScanItems; i++) {
+  for (int i = 0; i < kItems; i++) {
     const u64 tc = (base + i < a.ntiles) ? a.tile_count[(size_t)(base + i) * kCtrStride64] : 0ull;
     v[i] = (uint32_t)tc;
     nbv[i] = band_count(a, v[i], (uint32_t)(tc >> 32));
     sum += v[i];
+    if (v[i] > a.frag_size) {
+      nh++;
+      npt += (v[i] + a.frag_size - 1) / a.frag_size;
+    } else if (nbv[i]) {
+      npt += nbv[i];
+    } else if (v[i] > 0) {
+      nl++;
+    }
   }
   // Bit i of `listed`: tile base + i belongs to a job with direct items.
   uint32_t listed = 0;
@@ -948,7 +921,7 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a) {
     int next = 0;
     bool any = false;
 #pragma unroll
-    for (int i = 0; i < kScanItems; i++) {
+    for (int i = 0; i < kItems; i++) {
       if (base + i < a.ntiles && (i == 0 || base + i >= next)) {
         if (i) j++;
         any = *direct_line(a, a.job_tile_base[j]) != 0;
@@ -957,91 +930,59 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a) {
       listed |= (any ? 1u : 0u) << i;
     }
   }
-  u64 x = sum;  // wave inclusive scan
+  u64 x = sum;  // wave inclusive scans
+  uint32_t hx = nh, px = npt, lx = nl;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const u64 y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) sh_w[wave] = x;
-  __syncthreads();
-  u64 wpre = 0, btot = 0;
-#pragma unroll
-  for (int w = 0; w < kScanBlock / 64; w++) {
-    if (w < wave) wpre += sh_w[w];
-    btot += sh_w[w];
-  }
-  if (tid == 0) {
-    const u64 excl = lookback(a.scan_status, blk, btot, a.counters);
-    sh_excl = excl;
-    if (blk == a.scan_blocks - 1) {
-      a.counters[kBinEntries] = excl + btot;
-      // More pairs than the bin list holds (32-bit offsets and cursors could
-      // then wrap into it): flagged here, whatever the binner's checks see.
-      if (excl + btot > a.bins_cap) atomicOr(&a.counters[kBinOverflow], 1ull);
-    }
-  }
-  // Split (heavy) tiles: the workgroup reserves its merge slots and part
-  // list entries with one atomic each (same-address atomics serialise); the
-  // same for its entries of the raster's tile list (tiles rastered whole:
-  // with entries, not split).
-  uint32_t nh = 0, npt = 0, nl = 0;
-#pragma unroll
-  for (int i = 0; i < kScanItems; i++)
-    if (base + i < a.ntiles && v[i] > a.frag_size) {
-      nh++;
-      npt += (v[i] + a.frag_size - 1) / a.frag_size;
-    } else if (base + i < a.ntiles && nbv[i]) {
-      npt += nbv[i];
-    } else if (base + i < a.ntiles && v[i] > 0) {
-      nl++;
-    }
-  uint32_t hx = nh, px = npt, lx = nl;  // wave inclusive scans
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
     const uint32_t yh = __shfl_up(hx, o), yp = __shfl_up(px, o), yl = __shfl_up(lx, o);
     if (lane >= o) {
+      x += y;
       hx += yh;
       px += yp;
       lx += yl;
     }
   }
-  __shared__ uint32_t sh_h[kScanBlock / 64], sh_p[kScanBlock / 64], sh_l[kScanBlock / 64];
-  __shared__ u64 sh_hbase, sh_pbase, sh_lbase;
   if (lane == 63) {
+    sh_w[wave] = x;
     sh_h[wave] = hx;
     sh_p[wave] = px;
     sh_l[wave] = lx;
   }
   __syncthreads();
+  u64 wpre = 0, btot = 0;
   uint32_t hpre = 0, ppre = 0, lpre = 0, htot = 0, ptot = 0, ltot = 0;
 #pragma unroll
-  for (int w = 0; w < kScanBlock / 64; w++) {
+  for (int w = 0; w < NW; w++) {
     if (w < wave) {
+      wpre += sh_w[w];
       hpre += sh_h[w];
       ppre += sh_p[w];
       lpre += sh_l[w];
     }
+    btot += sh_w[w];
     htot += sh_h[w];
     ptot += sh_p[w];
     ltot += sh_l[w];
   }
-  if (tid == 0 && a.scan_blocks == 1) {  // the only workgroup: bases 0, totals stored
-    a.counters[kHeavy] = htot;
-    a.counters[kParts] = ptot;
-    a.counters[kListed] = ltot;
-    sh_hbase = sh_pbase = sh_lbase = 0;
-  } else if (tid == 0) {
-    sh_hbase = htot ? atomicAdd(&a.counters[kHeavy], (u64)htot) : 0;
-    sh_pbase = ptot ? atomicAdd(&a.counters[kParts], (u64)ptot) : 0;
-    sh_lbase = ltot ? atomicAdd(&a.counters[kListed], (u64)ltot) : 0;
+  if (tid < 4) {
+    const u64 add = tid == 0 ? btot : tid == 1 ? (u64)htot : tid == 2 ? (u64)ptot : (u64)ltot;
+    u64* const ctr =
+        &a.counters[tid == 0 ? kBinEntries : tid == 1 ? kHeavy : tid == 2 ? kParts : kListed];
+    u64 first = 0;
+    if (a.scan_blocks == 1) *ctr = add;  // the only workgroup
+    else if (add) first = atomicAdd(ctr, add);
+    sh_base[tid] = first;
+    // More pairs than the bin list holds (32-bit offsets and cursors could
+    // then wrap into it): flagged here, whatever the binner's checks see.
+    if (tid == 0 && first + add > a.bins_cap) atomicOr(&a.counters[kBinOverflow], 1ull);
   }
   __syncthreads();
-  u64 hs = sh_hbase + hpre + (hx - nh), ps = sh_pbase + ppre + (px - npt);
-  u64 ls = sh_lbase + lpre + (lx - nl);
-  u64 run = sh_excl + wpre + (x - sum);
+  u64 hs = sh_base[1] + hpre + (hx - nh), ps = sh_base[2] + ppre + (px - npt);
+  u64 ls = sh_base[3] + lpre + (lx - nl);
+  u64 run = sh_base[0] + wpre + (x - sum);
 #pragma unroll
-  for (int i = 0; i < kScanItems; i++) {
+  for (int i = 0; i < kItems; i++) {
     const int t = base + i;
     if (t < a.ntiles) {
       const uint32_t o = run > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)run;
@@ -1480,6 +1421,11 @@ __device__ inline void check_direct_room(const BatchArgs& a) {
   if (a.counters[kBinEntries] > a.bins_cap) atomicOr(&a.counters[kBinOverflow], 1ull);
 }
 
+__device__ __forceinline__ void scan_any(const BatchArgs& a, int blk) {
+  if (a.ntiles <= kScanWide) stage_scan<1>(a, blk);
+  else stage_scan<kScanItems>(a, blk);
+}
+
 // The scan's workgroups first, then (ckpt_in_scan) the checkpoint
 // allocation's and the direct entries', which need only geometry's items and
 // so run beside the scan: one launch for all.
@@ -1487,7 +1433,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan(BatchArgs a) {
   static_assert(kScanBlock == 256, "the other passes run in workgroups of 256");
   const int nd = direct_grid(a);
   const int b = (int)blockIdx.x - a.scan_blocks;
-  if (b < 0) stage_scan(a);
+  if (b < 0) scan_any(a, blockIdx.x);
   else if (b < nd) stage_direct(a, b, nd);
   else stage_ckpt(a, b - nd, (int)gridDim.x - a.scan_blocks - nd);
 }
@@ -2150,12 +2096,12 @@ __device__ __forceinline__ void stage_shade(const BatchArgs& a, int vb, bool rem
   // A job of one draw needs no draw table (ncached = -1).
   const bool one_draw = J.draw_end - J.draw_begin == 1;
   const int ncached = one_draw ? -1 : fill_draw_cache(dcache, a, J, tid, kShadeBlock);
-  // The raster and scan are done with the tile counters, part counters and
-  // look-back words: leave them zero for the next batch on this scratch.
-  for (int64_t i = (int64_t)vb * kShadeBlock + tid; i < a.ntiles || i < a.scan_blocks;
-       i += (int64_t)a.shade_blocks * kShadeBlock) {
-    if (i < a.ntiles) zero_tile(a, (int)i);
-    if (i < a.scan_blocks) a.scan_status[i] = 0;
+  // The raster and scan are done with the tile counters and part counters:
+  // leave them zero for the next batch on this scratch (a shading block covers
+  // at most four tiles: there are threads enough for one tile each).
+  if (vb <= (a.ntiles - 1) / kShadeBlock) {
+    const int i = vb * kShadeBlock + tid;
+    if (i < a.ntiles) zero_tile(a, i);
   }
   if (!one_draw) __syncthreads();
   if (vb == 0) reduce_stats(a, tid);
@@ -2390,7 +2336,7 @@ __device__ __forceinline__ void persist_run(const BatchArgs& a, const PersistPla
     case kPClear: stage_clear(a, (int)vb, q.nvb[s]); break;
     case kPVertex: stage_vertex(a, (int)vb, q.nvb[s]); break;
     case kPGeom: stage_geom<false, false>(a, (int)vb, q.nvb[s]); break;
-    case kPScan: stage_scan(a); break;
+    case kPScan: scan_any(a, (int)vb); break;
     case kPBin:
       stage_direct(a, (int)vb, q.nvb[s]);
       stage_bin<true>(a, (int)vb, q.nvb[s]);
@@ -2602,7 +2548,7 @@ void* noalloc_scratch(int device) {
 // ---- launchers -------------------------------------------------------------
 
 static int clear_grid(const BatchArgs& a) {
-  const int n = std::max(std::max(a.scan_blocks, a.ntiles), (int)kNumCounters);
+  const int n = std::max(a.ntiles, (int)kNumCounters);
   return std::min((n + 255) / 256, 4096);
 }
 

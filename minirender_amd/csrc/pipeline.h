@@ -61,7 +61,6 @@ struct BatchArgs {
   uint32_t heavy_cap;
   uint32_t frag_size;        // max (tile, triangle) pairs per raster work item
   uint32_t band_work;        // a tile with more walk work is rastered in row bands
-  unsigned long long* scan_status;  // [scan_blocks] decoupled look-back words
   unsigned long long* counters;     // [kNumCounters]
   // The counters' copy in pinned host memory (device address), written by
   // the shading kernel's first workgroup once they are final; null: the
@@ -145,7 +144,8 @@ constexpr int64_t kCkptScanRegions = 65536;
 constexpr int kStatSlots = 8192;  // >= the geometry and bin grids
 
 inline int32_t scan_blocks_for(int32_t tiles) {
-  return (tiles + kScanBlock * kScanItems - 1) / (kScanBlock * kScanItems);
+  const int32_t per = kScanBlock * (tiles <= kScanWide ? 1 : kScanItems);
+  return (tiles + per - 1) / per;
 }
 
 // Grid sizes of the grid-stride kernels (also used to sum their statistics).
