@@ -51,15 +51,24 @@ METRIC = "Mtris/s + frames/s at 1080p; p50/p99 ms/request, batched vs plain GPU"
 HBM_PEAK_GBS = 8000.0
 STAGES = ["clear", "geometry", "scan", "bin", "rows", "raster", "shade"]
 CKPT_SCAN_REGIONS = 65536  # batches of at most this many 64-triangle regions: k_bin_rows
+FRONT_TRIS = 1500000  # batches of at most this many triangles: k_front
 
 
-def kernel_of(frame):
-    """The kernel behind each stage of a frame rendered alone.  A batch of at
-    most CKPT_SCAN_REGIONS regions takes its edge checkpoints in the scan's
-    launch and walks their rows at the end of binning (k_bin_rows, no k_rows
-    launch); a larger one bins with k_bin and walks with k_rows."""
+def kernel_of(frame, launches):
+    """The kernel behind each stage of a frame rendered alone, with the
+    launches it took.  A small frame takes two: k_front and k_small.  A batch
+    of at most FRONT_TRIS triangles transforms its vertices in k_front.  A
+    batch of at most CKPT_SCAN_REGIONS regions takes its edge checkpoints in
+    the scan's launch and walks their rows at the end of binning (k_bin_rows,
+    no k_rows launch); a larger one bins with k_bin and walks with k_rows."""
+    if launches == 2:
+        return {"clear": "(no clear)", "geometry": "k_front", "scan": "(no scan)",
+                "bin": "(no bin)", "rows": "(no rows)", "raster": "k_small",
+                "shade": "(in k_small)"}
     small = (frame.ntri + 63) // 64 <= CKPT_SCAN_REGIONS
-    return {"clear": "k_clear", "geometry": "k_vertex+k_geom", "scan": "k_scan",
+    return {"clear": "k_clear",
+            "geometry": "k_front" if frame.ntri <= FRONT_TRIS else "k_vertex+k_geom",
+            "scan": "k_scan",
             "bin": "k_bin_rows" if small else "k_bin",
             "rows": "(in k_bin_rows)" if small else "k_rows", "raster": "k_tile",
             "shade": "k_shade"}
@@ -236,7 +245,7 @@ def plain_section(args, torch, mra, frame, wl_name):
     log(f"plain: {tune}")
     # Timed steps: synchronous mr_render calls with eager launches (on this
     # GPU and ROCm, replaying the frame as a captured HIP graph costs more
-    # host time per frame than the six or seven launches it replaces), no
+    # host time per frame than the launches it replaces), no
     # per-stage events.
     for _ in range(args.warmup):
         step()
@@ -260,7 +269,10 @@ def plain_section(args, torch, mra, frame, wl_name):
     ctx.set_profiling(False)
     stage /= args.steps
     alg = kernel_alg_bytes(frame)
-    kname = kernel_of(frame)
+    kname = kernel_of(frame, st.launches)
+    if kname["shade"].startswith("("):
+        alg["raster"] += alg["shade"]
+        alg["shade"] = 0
     kernels = {}
     for i, name in enumerate(STAGES):
         ms = float(stage[i])
@@ -273,7 +285,7 @@ def plain_section(args, torch, mra, frame, wl_name):
     fb = frame_alg_bytes(frame)
     fmed = float(np.median(fms))
     # Headline: the frame's algorithmic bytes (positions, normals, uvs,
-    # indices, texels in; RGB8 + depth out) over the GPU time of its six
+    # indices, texels in; RGB8 + depth out) over the GPU time of its
     # kernels (events around the launches on the library's stream).  The
     # dominant kernel moves only intermediate data (0 algorithmic bytes),
     # so it is reported beside the headline with its counter traffic.

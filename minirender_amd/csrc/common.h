@@ -92,7 +92,6 @@ enum Counter : int {
   kBinOverflow = 2,  // set when the bin list was too small
   kError = 3,        // set when a bounded wait hit its limit
   kClipped = 4,      // input triangles that crossed the near plane
-  kTileTicket = 5,
   kBinEntries = 6,   // total (tile, triangle) pairs (the scan's and the direct ones)
   kParts = 7,        // work items of split tiles (written by the scan)
   kHeavy = 8,        // tiles split over several work items

@@ -29,7 +29,7 @@ struct BatchArgs {
   // row + 16 (for the group leader's pair, times the group size); in the next
   // word, (direct entries << 32) | the first one's place in the bin list
   unsigned long long* tile_count;
-  uint32_t* tile_off;        // [ntiles] exclusive scan of the pair counts
+  uint32_t* tile_off;        // [ntiles] first place in the bin list
   uint32_t* tile_cursor;     // [ntiles * kCtrStride] scatter cursors
   uint32_t* tile_heavy;      // [ntiles] merge slot of a split tile, kNoSlot, or kEmptyTile
   uint4* tile_list;          // [ntiles] {tile, first bin entry, entries, 1 if its job
@@ -98,7 +98,7 @@ struct BatchArgs {
   // kernel always takes them in its binning stage): 1, by the scan's launch
   // in workgroups beside the scan, with the row pre-pass at the end of the
   // binning kernel (a batch of at most kCkptScanRegions regions, whose items
-  // that pass reads while the one-workgroup scan runs); 0, by the binning
+  // that pass reads while the scan runs); 0, by the binning
   // kernel, which reads the items anyway, with the row pre-pass a launch of
   // its own.
   int32_t ckpt_in_scan;
