@@ -721,8 +721,15 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
   const int64_t r_end = min(r_begin + chunk, a.total_tris);
   int dw = wave_search_last(a.draw_begin, a.ndraws, min(r_begin, a.total_tris));
   dw = __builtin_amdgcn_readfirstlane(dw);
+  // The draws' starts at a wavefront-uniform index, through scalar loads (left
+  // to itself the compiler makes vector loads of them, which wait for the last
+  // region's stores and atomics: geometry and vertices of 64 frames of 1 M
+  // triangles 1092 -> 963 us, of one frame of 8.4 M 159 -> 147 us).
+  typedef const __attribute__((address_space(4))) int64_t* ConstStarts;
+  const ConstStarts starts = (ConstStarts)a.draw_begin;
+  const int wave0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);
   for (int64_t base = r_begin; base < r_end; base += 256) {
-    const int64_t wfirst = base + (threadIdx.x & ~63);
+    const int64_t wfirst = base + wave0;
     if (wfirst >= r_end) continue;
     const int64_t g = wfirst + lane;
     TriSetup s0, s1;
@@ -735,9 +742,8 @@ __device__ __forceinline__ void stage_geom(const BatchArgs& a, int vb, int nvb) 
     // The wave's draw: step the uniform draw index to the wave's first
     // triangle; lanes past the next draw's start step further (draw
     // boundaries inside a wavefront are rare).
-    while (dw + 1 < a.ndraws && a.draw_begin[dw + 1] <= wfirst) dw++;
-    dw = __builtin_amdgcn_readfirstlane(dw);
-    const int64_t next_begin = dw + 1 < a.ndraws ? a.draw_begin[dw + 1] : 0x7FFFFFFFFFFFFFFFll;
+    while (dw + 1 < a.ndraws && starts[dw + 1] <= wfirst) dw++;
+    const int64_t next_begin = dw + 1 < a.ndraws ? starts[dw + 1] : 0x7FFFFFFFFFFFFFFFll;
     if (g < r_end) {
       int d = dw;
       if (g >= next_begin)
