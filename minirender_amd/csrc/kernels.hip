@@ -515,8 +515,8 @@ __device__ inline void wave_pairs_apply(const BatchArgs& a, bool ok, int key, ui
 // The pairs of a binning step on their way: a step reserves its ranges of the
 // tiles' lists and stores the pairs of the step before, whose reservation has
 // had the time of a step's arithmetic to come back (waiting for it in the step
-// itself took 461 us for the 64 M triangles of 64 frames, 419 now; 70 -> 59 us
-// for a 3839 x 2157 frame of 8.4 M).
+// itself took 461 us for the 64 M triangles of 64 frames, 419 with this; 70 -> 59
+// us for a 3839 x 2157 frame of 8.4 M).
 struct Scatter {
   uint32_t old = 0, id = 0, draw = 0;
   int meta = -1;  // rank in the group << 8 | its leader; -1: no pair
@@ -1178,6 +1178,7 @@ __device__ __forceinline__ void stage_bin(const BatchArgs& a, int vb, int nvb) {
   // region is scattered (both loads are independent: every region slot is
   // allocated, slots past the count are read but not used).
   int64_t r = (int64_t)vb * 4 + (threadIdx.x >> 6);
+  if (!kAlloc) r = (int64_t)vb * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   uint32_t cnt = 0;
   BinItem first = BinItem{0, 0, 0, 0, 0, 0};
   if (r < a.nregions) {
@@ -1185,6 +1186,10 @@ __device__ __forceinline__ void stage_bin(const BatchArgs& a, int vb, int nvb) {
     first = a.items[r * kRegion + lane];
   }
   while (r < a.nregions) {
+    // One region per wavefront: its count is the same in every lane, and loops
+    // over it as a scalar (419 -> 405 us on 64 frames of 1 M triangles; with
+    // the checkpoints' registers it spilled: 59 -> 63 us at 8.4 M triangles).
+    if (!kAlloc) cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)cnt);
     const int64_t rn = r + nw;
     uint32_t cnt_n = 0;
     BinItem first_n = BinItem{0, 0, 0, 0, 0, 0};
