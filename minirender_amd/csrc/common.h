@@ -105,6 +105,31 @@ enum Counter : int {
   kNumCounters = 16
 };
 
+// Raster work items of a batch, from its counters: parts and row bands of
+// split tiles, and tiles rastered whole (those with bin entries, then those
+// with direct entries only: `listed` in all).
+struct TileItems {
+  int64_t parts, whole, listed;
+};
+MR_HD inline TileItems tile_items(const unsigned long long* counters, uint32_t parts_cap,
+                                  int32_t ntiles) {
+  // After a bin-list overflow binning may have stored over the direct pairs
+  // at the list's other end: a tile's range can hold pairs of another job,
+  // whose setup with this tile's frame size and near plane gives boxes that
+  // no checkpoints were taken for.  Nothing is drawn (nor shaded); the batch
+  // runs again with a longer list.
+  TileItems r = {0, 0, 0};
+  if (counters[kBinOverflow]) return r;
+  const int64_t parts = (int64_t)counters[kParts], whole = (int64_t)counters[kListed];
+  // After a merge-slot or part-list overflow the part list is incomplete:
+  // split tiles are then skipped (the frame is re-run with larger buffers).
+  if (!counters[kHeavyOverflow]) r.parts = parts < parts_cap ? parts : parts_cap;
+  r.whole = whole < ntiles ? whole : ntiles;
+  r.listed = r.whole + (int64_t)counters[kDirectTilesListed];
+  if (r.listed > ntiles) r.listed = ntiles;
+  return r;
+}
+
 // Workgroup index b in [0, n) -> work index, a bijection under which each of
 // the 8 XCDs (which receive workgroups round-robin) gets one contiguous range
 // of work: neighbouring tiles share vertices, and each XCD has its own L2.

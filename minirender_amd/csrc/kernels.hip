@@ -1441,8 +1441,9 @@ __device__ __forceinline__ void stage_direct(const BatchArgs& a, int vb, int nvb
 }
 
 // The bin list holds the scan's pairs from its start and the direct pairs
-// from its end: more than it holds is an overflow.  Run by one thread after
-// both are known and before the raster.
+// from its end: more than it holds is an overflow, after which the raster
+// draws nothing (tile_items).  Run by one thread after both are known and
+// before the raster.
 __device__ inline void check_direct_room(const BatchArgs& a) {
   const u64 direct = a.counters[kDirectPairs];
   if (direct == 0ull) return;
@@ -1619,19 +1620,8 @@ __device__ __forceinline__ void raster_chunk(const BatchArgs& a, const JobDesc& 
   __syncthreads();
 }
 
-// Raster work items of the batch: parts and row bands, and tiles rastered
-// whole (those with bin entries, then those with direct entries only).
-struct TileItems {
-  int64_t parts, whole, listed;
-};
 __device__ inline TileItems tile_items(const BatchArgs& a) {
-  TileItems r;
-  // After a merge-slot or part-list overflow the part list is incomplete:
-  // split tiles are then skipped (the frame is re-run with larger buffers).
-  r.parts = a.counters[kHeavyOverflow] ? 0 : (int64_t)min(a.counters[kParts], (u64)a.parts_cap);
-  r.whole = (int64_t)min(a.counters[kListed], (u64)a.ntiles);
-  r.listed = min(r.whole + (int64_t)a.counters[kDirectTilesListed], (int64_t)a.ntiles);
-  return r;
+  return tile_items(a.counters, a.parts_cap, a.ntiles);
 }
 
 // (d): one workgroup per raster work item: first the parts of split tiles
@@ -1686,7 +1676,7 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     const int local = tile - J.tile_base;
     const int tyi = local / J.tiles_x, txi = local - tyi * J.tiles_x;
     const int x0 = txi * TW, y0 = tyi * TH;
-    uint32_t avail = cnt;  // entries actually written (bin-list overflow)
+    uint32_t avail = cnt;  // entries inside the bin list
     if ((u64)off >= a.bins_cap) avail = 0;
     else if ((u64)off + cnt > a.bins_cap) avail = (uint32_t)(a.bins_cap - off);
     const uint32_t e_begin = (uint32_t)part * a.frag_size;

@@ -60,3 +60,12 @@ def test_cover_rows_is_conservative(tmp_path_factory, seed):
     r = subprocess.run([str(rows_bin), "1000000", str(seed)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.strip() == "ok"
+
+
+def test_nothing_drawn_from_a_bin_list_that_overflowed(tmp_path_factory):
+    """overflow_check: the raster reads entries of its own tiles only, also
+    when the direct and the binned pairs of a batch meet in the bin list."""
+    out = _build(tmp_path_factory, "overflow_check")
+    r = subprocess.run([str(out), "20000"], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip() == "ok"

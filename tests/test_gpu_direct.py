@@ -75,3 +75,42 @@ def test_bin_list_too_small(gpu_ctx):
         g = ctx.render(frame, KINDS)
         assert ctx.stats().retries >= 1
     assert_parity(g, oracle_py.render(frame, KINDS), "bin list too small")
+
+
+def flat_frame(w, h, tris):
+    """Triangles given in pixel coordinates (x right, y up) under an
+    orthographic projection, at depths of their own."""
+    n = len(tris)
+    rng = np.random.default_rng(n)
+    pos = np.empty((n, 3, 3), np.float32)
+    pos[:, :, :2] = tris
+    pos[:, :, 2] = rng.uniform(-0.9, 0.9, n).astype(np.float32)[:, None]
+    nrm = np.tile(np.array([[0, 0, 1]], np.float32), (3 * n, 1))
+    idx = np.arange(3 * n, dtype=np.int32).reshape(-1, 3)
+    return FrameSpec(w, h, scenes.projection_ortho(0, w, 0, h, -1, 1),
+                     draws=[Draw(scenes.Mesh(pos.reshape(-1, 3), nrm, idx), Material())], lighting=False)
+
+
+@pytest.mark.parametrize("persistent", [False, True])
+@pytest.mark.parametrize("small_first", [False, True])
+def test_both_ends_of_the_bin_list_meet(persistent, small_first):
+    """Two jobs whose listed pairs (48,960 of 6 triangles over a 1920 x 1080
+    frame) and binned pairs (up to 45,000 of 3,000 triangles that leave a
+    200 x 150 frame, 3 x 5 tiles each) both fit the 65,536 entries of the bin
+    list alone, but not together: nothing may be drawn from the list before
+    the batch has run again with a longer one."""
+    import minirender_amd as mra
+    rng = np.random.default_rng(5)
+    large = flat_frame(1920, 1080, np.array([[-10, -10], [4000, -10], [-10, 2300]], np.float32)[None] +
+                       rng.uniform(0, 5, (6, 1, 2)).astype(np.float32))
+    off = flat_frame(200, 150, np.array([[170, 55], [900, 90], [170, 130]], np.float32)[None] +
+                     rng.uniform(0, 4, (3000, 1, 2)).astype(np.float32))
+    frames = [off, large] if small_first else [large, off]
+    with mra.Context(0) as ctx:
+        ctx.set_tile(16, 16)
+        ctx.set_bin_factor(1.0)
+        ctx.set_persistent(persistent)
+        out = ctx.render_batch(frames, KINDS)
+        assert ctx.stats().retries >= 1
+    for i, (g, f) in enumerate(zip(out, frames)):
+        assert_parity(g, oracle_py.render(f, KINDS), f"job {i}")
