@@ -2108,10 +2108,14 @@ __device__ __forceinline__ void stage_shade(const BatchArgs& a, int vb, bool rem
   const uint32_t pix = (uint32_t)row * (uint32_t)J.W + (uint32_t)c;
   uint32_t id = kNoWinner;
   const int sw = __ffs(a.tile_w) - 1, sh = __ffs(a.tile_h) - 1;
-  if (sw >= 4) {  // the block lies in one tile: one scalar load
+  if (sw >= 4) {  // the block lies in one tile: one load
+    // (A scalar load in a launch of its own only: the persistent kernel writes
+    // the flags itself, and the fences between its stages do not reach the
+    // scalar cache.)
     const int ct = (local - byi * bxn) * kShadeW >> sw, rt = byi * kShadeH >> sh;
+    const int at = J.tile_base + rt * J.tiles_x + ct;
     typedef const __attribute__((address_space(4))) uint32_t* ConstWords;
-    const uint32_t flag = ((ConstWords)a.tile_heavy)[J.tile_base + rt * J.tiles_x + ct];
+    const uint32_t flag = remap ? ((ConstWords)a.tile_heavy)[at] : a.tile_heavy[at];
     if (inside && flag != kEmptyTile) id = *px_at(J.win, 4u * pix);
   } else if (inside) {
     const uint32_t flag = a.tile_heavy[J.tile_base + (row >> sh) * J.tiles_x + (c >> sw)];
