@@ -59,6 +59,7 @@ int dev_alloc(mr_ctx* c, DevBuf& b, size_t bytes, bool scratch) {
     return MR_ERR_NOMEM;
   }
   b.bytes = want;
+  b.id = ++c->allocs;
   acct += want;
   return MR_OK;
 }
@@ -555,8 +556,8 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   // be zero: new buffers, more tiles than cleared before, no vertex kernel
   // (which clears the batch counters) and no shading kernel that left them
   // zero.  A small batch uses none of them.
-  const bool same_bufs = s.clean_ref[0] == x.tile_count.p && s.clean_ref[1] == x.tile_done.p &&
-                         s.clean_ref[2] == x.counters.p && s.clean_ref[3] == x.ckpt_ctr.p;
+  const uint64_t ids[4] = {x.tile_count.id, x.tile_done.id, x.counters.id, x.ckpt_ctr.id};
+  const bool same_bufs = memcmp(s.clean_ref, ids, sizeof(ids)) == 0;
   const bool clear = !a.small &&
                      (!same_bufs || p.total_tris == 0 || p.ntiles > s.clean_tiles ||
                       (a.front && !s.clean_counters));
@@ -667,10 +668,7 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
     s.clean_counters = prev_counters;
     return MR_OK;
   }
-  s.clean_ref[0] = x.tile_count.p;
-  s.clean_ref[1] = x.tile_done.p;
-  s.clean_ref[2] = x.counters.p;
-  s.clean_ref[3] = x.ckpt_ctr.p;
+  memcpy(s.clean_ref, ids, sizeof(ids));
   s.clean_tiles = next_tiles;
   // The shading kernel that hands the host the counters leaves them zero.
   s.clean_counters = a.host_counters != nullptr;

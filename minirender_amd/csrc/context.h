@@ -21,6 +21,7 @@ constexpr int kStages = 7;
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  uint64_t id = 0;  // of the allocation, one of its own in the context (dev_alloc)
 };
 
 struct HostBuf {  // pinned (hipHostMalloc)
@@ -125,10 +126,11 @@ struct Slot {
   std::vector<Graph> graphs;
   int64_t graph_replays = 0, graph_captures = 0;
   // Leading tile counters known to be zero (the shading
-  // kernel re-zeroes what a batch used), valid for the buffers in clean_ref.
+  // kernel re-zeroes what a batch used), valid for the allocations in
+  // clean_ref: a buffer grown since may have come back at the same address.
   int64_t clean_tiles = 0;
   bool clean_counters = false;  // batch and checkpoint counters too
-  const void* clean_ref[5] = {};
+  uint64_t clean_ref[4] = {};   // ids of tile_count, tile_done, counters, ckpt_ctr
 };
 
 }  // namespace mr
@@ -138,6 +140,7 @@ struct mr_ctx {
   uint64_t budget = 0;
   uint64_t resident_bytes = 0;
   uint64_t scratch_bytes = 0;
+  uint64_t allocs = 0;  // device allocations made (DevBuf::id)
   std::vector<mr::MeshRec> meshes;
   std::vector<mr::TexRec> textures;
   mr::Slot main;  // synchronous calls (mr_render, mr_render_batch)

@@ -1,0 +1,203 @@
+// CPU check of the host side of a batch (context.cpp), built with g++ against
+// the stand-ins below for the HIP runtime and for the kernel launchers: what
+// is launched, counted and assumed of buffers from one call to the next.
+//   clean     a general batch finds the tile counters zero, whatever ran and
+//             grew the buffers before it
+// Device memory is host memory, filled with 0xAB when it is allocated; a freed
+// block's address is the next allocation's.  A general batch's launches
+// check that the counters they add to are zero, and leave them so at the end,
+// as the kernels do.  Prints "ok" or the first failure.
+#include <sys/mman.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "minirender_amd.h"
+#include "pipeline.h"
+
+#define FAIL(...) (printf(__VA_ARGS__), printf("\n"), exit(1))
+
+// ---- the HIP runtime --------------------------------------------------------
+static std::vector<void*> g_free;
+static void* block(size_t bytes) {
+  constexpr size_t kBlock = (size_t)1 << 32;
+  if (bytes > kBlock) return nullptr;
+  void* p;
+  if (!g_free.empty()) {
+    p = g_free.back();
+    g_free.pop_back();
+  } else {
+    p = mmap(nullptr, kBlock, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (p == MAP_FAILED) return nullptr;
+  }
+  memset(p, 0xAB, bytes);
+  return p;
+}
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) { return (*p = block(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipFree(void* p) { if (p) g_free.push_back(p); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { *d = h; return hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemset(void* d, int v, size_t n) { memset(d, v, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { memset(d, v, n); return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) { a->type = hipMemoryTypeUnregistered; return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)malloc(1); return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = nullptr; return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { *e = nullptr; return hipSuccess; }
+hipError_t hipGraphExecUpdate(hipGraphExec_t, hipGraph_t, hipGraphNode_t*, hipGraphExecUpdateResult*) { return hipErrorNotSupported; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)malloc(1); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
+}
+
+// ---- the launchers ----------------------------------------------------------
+namespace mr {
+static int g_launches = 0;  // kernels launched
+static bool g_general = false, g_small = false;
+
+static void zero(const BatchArgs& a) {
+  memset(a.counters, 0, kNumCounters * 8);
+  memset(a.ckpt_ctr, 0, (size_t)kCkptSegs * kCtrStride * 8);
+}
+static void zero_tiles(const BatchArgs& a) {
+  for (int i = 0; i < a.ntiles; i++) {
+    memset(a.tile_count + (size_t)i * kCtrStride64, 0, 6 * 8);
+    a.tile_done[i] = 0;
+  }
+}
+static void expect_zero(const BatchArgs& a) {
+  for (int i = 0; i < kNumCounters; i++)
+    if (a.counters[i]) FAIL("batch counter %d not zero", i);
+  for (int i = 0; i < kCkptSegs; i++)
+    if (a.ckpt_ctr[i * kCtrStride]) FAIL("checkpoint counter %d not zero", i);
+  for (int i = 0; i < a.ntiles; i++)
+    if (a.tile_count[(size_t)i * kCtrStride64] || a.tile_done[i]) FAIL("counters of tile %d of %d not zero", i, a.ntiles);
+}
+static void hand_counters(const BatchArgs& a) {
+  if (!a.host_counters) return;
+  memcpy(a.host_counters, a.counters, kNumCounters * 8);
+  zero(a);
+}
+
+hipError_t launch_tables(const void* p, void* t, size_t n, hipStream_t) { g_launches++; memcpy(t, p, n); return hipSuccess; }
+hipError_t launch_clear(const BatchArgs& a, hipStream_t) { g_launches++; zero(a); zero_tiles(a); return hipSuccess; }
+hipError_t launch_vertex(const BatchArgs& a, hipStream_t) { if (a.total_verts) g_launches++, zero(a); return hipSuccess; }
+static hipError_t geometry(const BatchArgs& a) {
+  g_launches++;
+  g_general = !a.small;
+  if (a.small) return hipSuccess;
+  expect_zero(a);
+  for (int i = 0; i < a.ntiles; i++) a.tile_count[(size_t)i * kCtrStride64] = 1, a.tile_done[i] = 1;
+  return hipSuccess;
+}
+hipError_t launch_geometry(const BatchArgs& a, hipStream_t) { return a.total_tris ? geometry(a) : hipSuccess; }
+hipError_t launch_front(const BatchArgs& a, const void*, size_t, hipStream_t) { return geometry(a); }
+hipError_t launch_small(const BatchArgs& a, hipStream_t) {
+  g_launches++;
+  g_small = true;
+  memset(a.host_counters, 0, kNumCounters * 8);
+  return hipSuccess;
+}
+hipError_t launch_scan(const BatchArgs&, hipStream_t) { g_launches++; return hipSuccess; }
+hipError_t launch_bin(const BatchArgs&, hipStream_t) { g_launches++; return hipSuccess; }
+hipError_t launch_rows(const BatchArgs& a, hipStream_t) { g_launches += !a.ckpt_in_scan; return hipSuccess; }
+hipError_t launch_tile(const BatchArgs&, hipStream_t) { g_launches++; return hipSuccess; }
+hipError_t launch_shade(const BatchArgs& a, hipStream_t) { g_launches++; zero_tiles(a); hand_counters(a); return hipSuccess; }
+hipError_t launch_persistent(const BatchArgs& a, bool clear, unsigned long long*, unsigned long long*, uint64_t, hipStream_t) {
+  g_launches++;
+  if (clear) zero_tiles(a);
+  zero(a);
+  expect_zero(a);
+  return hipSuccess;
+}
+int geom_blocks_per_cu() { return 7; }
+int noalloc_scratch_init(int) { return -1; }
+void* noalloc_scratch(int) { return nullptr; }
+unsigned long long wall_clock_hz() { return 100000000ull; }
+bool persistent_supported(int w, int h) { return w == 16 && h == 16; }
+bool tile_supported(int w, int h) { return w == h && (w == 8 || w == 16 || w == 32); }
+bool raster_threads_supported(int, int) { return true; }
+int default_raster_threads(int) { return 256; }
+}  // namespace mr
+
+// ---- calls ------------------------------------------------------------------
+static mr_ctx* open_ctx() {
+  mr_ctx* c;
+  if (mr_ctx_create(0, 0, &c)) FAIL("context");
+  return c;
+}
+static int32_t upload(mr_ctx* c, int ntri) {
+  std::vector<float> v(9 * (size_t)ntri);
+  std::vector<int32_t> ix(3 * (size_t)ntri);
+  for (int i = 0; i < 3 * ntri; i++) ix[i] = i;
+  int32_t h;
+  if (mr_mesh_upload(c, v.data(), 3 * ntri, v.data(), 3 * ntri, nullptr, 0, ix.data(), ix.data(), nullptr, ntri, &h))
+    FAIL("upload");
+  return h;
+}
+// A frame of `ndraws` draws of a mesh, its image in host memory; returns the
+// kernels it launched.
+static int render(mr_ctx* c, int32_t mesh, int ndraws, int w, int h) {
+  std::vector<mr_draw> draws(ndraws);
+  for (mr_draw& d : draws) {
+    memset(&d, 0, sizeof(d));
+    d.mesh = mesh;
+    d.texture = -1;
+  }
+  mr_frame f;
+  memset(&f, 0, sizeof(f));
+  f.width = w;
+  f.height = h;
+  f.draws = draws.data();
+  f.ndraws = ndraws;
+  f.projection[15] = 1.0f;
+  std::vector<uint8_t> rgb((size_t)3 * w * h);
+  mr_outputs o;
+  memset(&o, 0, sizeof(o));
+  o.rgb8 = rgb.data();
+  const int before = mr::g_launches;
+  mr::g_general = mr::g_small = false;
+  const int rc = mr_render(c, &f, &o);
+  if (rc) FAIL("%d x %d: status %d", w, h, rc);
+  return mr::g_launches - before;
+}
+
+static void check_clean() {
+  mr_ctx* c = open_ctx();
+  const int32_t mesh = upload(c, 4);
+  const int sizes[][2] = {{1100, 100}, {640, 480}, {1000, 700}, {1100, 100}, {1100, 700}, {1000, 1000}, {1100, 100},
+                          {64, 64}, {1100, 1200}};
+  for (auto& s : sizes) {
+    render(c, mesh, 1, s[0], s[1]);
+    if (mr::g_small != (s[0] <= 1024) || mr::g_general != (s[0] > 1024)) FAIL("%d x %d: route", s[0], s[1]);
+  }
+  mr_ctx_destroy(c);
+}
+
+int main(int argc, char** argv) {
+  const char* what = argc > 1 ? argv[1] : "";
+  if (!strcmp(what, "clean")) check_clean();
+  else FAIL("nothing to check");
+  printf("ok\n");
+  return 0;
+}

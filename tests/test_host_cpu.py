@@ -1,0 +1,28 @@
+"""CPU: the host side of a batch (context.cpp) with stand-ins for the HIP
+runtime and the kernel launchers (tests/cpu/host_check.cpp)."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+CSRC = ROOT / "minirender_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def host_bin(tmp_path_factory):
+    out = tmp_path_factory.mktemp("host") / "host_check"
+    subprocess.run(["g++", "-w", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    f"-I{ROOT / 'include'}", f"-I{CSRC}", str(ROOT / "tests" / "cpu" / "host_check.cpp"),
+                    str(CSRC / "context.cpp"), "-o", str(out), "-lpthread"], check=True)
+    return out
+
+
+def run(host_bin, what):
+    r = subprocess.run([str(host_bin), what], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip() == "ok"
+
+
+def test_general_batches_find_their_counters_zero(host_bin):
+    run(host_bin, "clean")
