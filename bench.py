@@ -60,14 +60,18 @@ def kernel_of(frame, launches):
     of at most FRONT_TRIS triangles transforms its vertices in k_front.  A
     batch of at most CKPT_SCAN_REGIONS regions takes its edge checkpoints in
     the scan's launch and walks their rows at the end of binning (k_bin_rows,
-    no k_rows launch); a larger one bins with k_bin and walks with k_rows."""
-    if launches == 2:
-        return {"clear": "(no clear)", "geometry": "k_front", "scan": "(no scan)",
+    no k_rows launch); a larger one bins with k_bin and walks with k_rows.  One
+    launch more fetches batch tables that the first kernel's argument does not
+    hold (k_tables).  (Clearing is for new buffers only: not in a steady state.)"""
+    if launches <= 3:
+        return {"clear": "k_tables" if launches == 3 else "(no clear)", "geometry": "k_front", "scan": "(no scan)",
                 "bin": "(no bin)", "rows": "(no rows)", "raster": "k_small",
                 "shade": "(in k_small)"}
     small = (frame.ntri + 63) // 64 <= CKPT_SCAN_REGIONS
-    return {"clear": "k_clear",
-            "geometry": "k_front" if frame.ntri <= FRONT_TRIS else "k_vertex+k_geom",
+    front = frame.ntri <= FRONT_TRIS
+    fetched = launches > (1 if front else 2) + (4 if small else 5)
+    return {"clear": "k_tables" if fetched else "(no clear)",
+            "geometry": "k_front" if front else "k_vertex+k_geom",
             "scan": "k_scan",
             "bin": "k_bin_rows" if small else "k_bin",
             "rows": "(in k_bin_rows)" if small else "k_rows", "raster": "k_tile",
@@ -298,7 +302,7 @@ def plain_section(args, torch, mra, frame, wl_name):
     frame_traffic = (sum(ktraffic.values()) if all(v is not None for v in ktraffic.values())
                      else None)
     achieved = fb / (fmed * 1e-3) / 1e9 if fmed > 0 else 0.0
-    launched = [k for n in STAGES[1:] for k in kname[n].split("+") if not k.startswith("(")]
+    launched = [k for n in STAGES for k in kname[n].split("+") if not k.startswith("(")]
     roof = {"bound": "hbm", "kernel": "frame (" + ", ".join(launched) + ")",
             "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),

@@ -100,13 +100,15 @@ typedef struct mr_stats {
   int64_t tiles;              /* screen tiles                                     */
   int64_t retries;            /* re-runs after a bin-capacity overflow           */
   double stage_ms[8];         /* per-stage GPU time when profiling is on:        */
-                              /* 0 clear, 1 geometry, 2 scan, 3 bin, 4 rows      */
+                              /* 0 tables and clear, 1 geometry, 2 scan, 3 bin,   */
+                              /* 4 rows                                           */
                               /* (edge checkpoints), 5 raster, 6 shade; for the   */
                               /* persistent kernel each stage's span (its first   */
                               /* workgroup's start to its last one's end)         */
   double frame_ms;            /* first to last kernel of the frame (profiling)  */
-  int64_t launches;           /* kernel launches of the last batch (1: the     */
-                              /* persistent kernel)                             */
+  int64_t launches;           /* kernel launches of the last batch, the one    */
+                              /* that fetches larger batch tables among them    */
+                              /* (1: the persistent kernel)                     */
   /* Captured batches (mr_ctx_set_graphs) over every slot of the context     */
   /* since its creation: replayed as captured, replayed after updating an    */
   /* instantiated graph of the same kernels in place, newly instantiated.    */

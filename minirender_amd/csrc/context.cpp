@@ -435,18 +435,27 @@ static BatchArgs make_args(mr_ctx* c, Slot& sl, const BatchPlan& p) {
   return a;
 }
 
+// Kernels launch_stages launches.
+static int32_t stage_launches(const BatchArgs& a, bool clear, bool persistent) {
+  if (a.small) return 2;
+  if (persistent) return 1;
+  return (clear ? 1 : 0) + (a.total_verts && !a.front ? 1 : 0) + (a.total_tris ? 1 : 0) +
+         (a.ckpt_in_scan ? 4 : 5);
+}
+
 // persistent: every stage in one launch of the persistent kernel (profiling
-// then times the whole launch as stage 0).  tables: the batch tables in host
-// memory when the first kernel takes them in its argument.
+// then times the whole launch as stage 0).  inl: the batch tables in host
+// memory when the first kernel takes them in its argument; pinned: their
+// device address when a kernel fetches them from there.
 static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
-                         bool persistent, uint64_t wait_us, const void* tables = nullptr,
-                         size_t table_bytes = 0) {
+                         bool persistent, uint64_t wait_us, const void* inl = nullptr,
+                         const void* pinned = nullptr, size_t table_bytes = 0) {
   hipStream_t st = s.stream;
   if (a.small) {
-    s.last_launches = 2;
     if (profile) HIP_TRY(hipEventRecord(s.ev[0], st));
+    if (pinned) HIP_TRY(launch_tables(pinned, s.sc.tables.p, table_bytes, st));
     if (profile) HIP_TRY(hipEventRecord(s.ev[1], st));
-    HIP_TRY(launch_front(a, tables, table_bytes, st));
+    HIP_TRY(launch_front(a, inl, table_bytes, st));
     if (profile)
       for (int i = 2; i <= 5; i++) HIP_TRY(hipEventRecord(s.ev[i], st));
     HIP_TRY(launch_small(a, st));
@@ -462,16 +471,14 @@ static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
     HIP_TRY(launch_persistent(a, clear, ctl, stamps, wait_us, st));
     if (profile)
       for (int i = 1; i <= kStages; i++) HIP_TRY(hipEventRecord(s.ev[i], st));
-    s.last_launches = 1;
     return MR_OK;
   }
-  s.last_launches = (clear ? 1 : 0) + (a.total_verts && !a.front ? 1 : 0) +
-                    (a.total_tris ? 1 : 0) + (a.ckpt_in_scan ? 4 : 5);
   if (profile) HIP_TRY(hipEventRecord(s.ev[0], st));
+  if (pinned) HIP_TRY(launch_tables(pinned, s.sc.tables.p, table_bytes, st));
   if (clear) HIP_TRY(launch_clear(a, st));
   if (profile) HIP_TRY(hipEventRecord(s.ev[1], st));
   if (a.front) {
-    HIP_TRY(launch_front(a, tables, table_bytes, st));
+    HIP_TRY(launch_front(a, inl, table_bytes, st));
   } else {
     HIP_TRY(launch_vertex(a, st));
     HIP_TRY(launch_geometry(a, st));
@@ -489,6 +496,12 @@ static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
   if (profile) HIP_TRY(hipEventRecord(s.ev[7], st));
   return MR_OK;
 }
+
+// Tables of a small batch up to this size come by the runtime's copy, larger
+// ones by k_tables: a frame of 31 draws (9 KB) at 640 x 480 took 42.7 us by the
+// copy and 42.3 by the kernel, of 60 draws (17 KB) 55.3 and 49.2, of 200 97 and
+// 92; 12 frames of 1,000 triangles (7 KB) 38.4 and 37.9, 32 of them 56.6 and 51.1.
+constexpr size_t kCopyTables = 12288;
 
 // Device address (null: none) of a pinned buffer, looked up when it changes.
 static void device_address(const HostBuf& b, void*& of, void*& dev) {
@@ -569,19 +582,24 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   const bool prev_counters = s.clean_counters;
   s.clean_tiles = 0;  // until the launches below succeed
   // Eager launches of a batch that starts with k_front hand it small tables
-  // in its argument, and k_tables fetches larger ones from the staging; a
-  // captured batch copies them from the staging when it is replayed.
+  // in its argument, and k_tables fetches larger ones from the staging.  The
+  // runtime copies them for a captured batch, when it is replayed, for the
+  // persistent kernel, which stays the batch's one launch, and for small
+  // batches up to kCopyTables.
   const bool capture = c->graphs && !profile && s.own_stream && s.stream == s.own_stream;
   const bool inl = a.front && !capture && p.layout.bytes <= kInlineWords * 4;
-  if (!inl && !capture) device_address(x.h_tables, s.h_tables_of, s.h_tables_dev);
+  bool fetch = !inl && !capture && !persistent && !(a.small && p.layout.bytes <= kCopyTables);
+  if (fetch) device_address(x.h_tables, s.h_tables_of, s.h_tables_dev);
+  fetch = fetch && s.h_tables_dev;
+  s.last_launches = stage_launches(a, clear, persistent) + (fetch ? 1 : 0);
+  s.last_persistent = persistent;
   auto issue = [&]() -> int {
-    if (!inl && !capture && s.h_tables_dev)
-      HIP_TRY(launch_tables(s.h_tables_dev, x.tables.p, p.layout.bytes, s.stream));
-    else if (!inl)
+    if (!inl && !fetch)
       HIP_TRY(hipMemcpyAsync(x.tables.p, x.h_tables.p, p.layout.bytes, hipMemcpyHostToDevice,
                              s.stream));
     int r = launch_stages(a, s, profile, clear, persistent, c->wait_us,
-                          inl ? x.h_tables.p : nullptr, p.layout.bytes);
+                          inl ? x.h_tables.p : nullptr, fetch ? s.h_tables_dev : nullptr,
+                          p.layout.bytes);
     if (r) return r;
     if (!a.host_counters)
       HIP_TRY(hipMemcpyAsync(x.h_counters.p, a.counters, kNumCounters * 8,
@@ -721,7 +739,7 @@ int finish_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
     st.launches = s.last_launches;
     st.split_tiles = (int64_t)hc[kHeavy];
     st.raster_parts = (int64_t)hc[kParts];
-    if (profile && s.last_launches == 1 && x.ctl.p) {
+    if (profile && s.last_persistent) {
       // One persistent launch: each stage's span from its workgroups' stamps
       // (first start to last end; the stages of the vertex and geometry
       // kernels are reported together, as the separate launches are).

@@ -14,7 +14,7 @@ namespace mr {
 
 constexpr size_t kGraphCache = 32;
 constexpr int kOutKinds = 6;  // rgb8, depth, winner, rgb, normals, points (mr_outputs order)
-// Stages timed when profiling (mr_stats.stage_ms order): clear, geometry
+// Stages timed when profiling (mr_stats.stage_ms order): tables and clear, geometry
 // (vertex + geometry kernels), scan, bin, rows, raster, shade.
 constexpr int kStages = 7;
 
@@ -114,6 +114,7 @@ struct Slot {
   size_t parts_want = 0;     // raster work items a batch needed (after an overflow)
   int32_t last_geom_grid = 0, last_bin_grid = 0;
   int32_t last_launches = 0;  // kernel launches of the last batch
+  bool last_persistent = false;  // it ran as the persistent kernel
   int64_t retries = 0;
   // Steady state: batches' uploads + stages + counter read-back captured as
   // instantiated graphs, keyed by the launch parameters, most recent first

@@ -3,6 +3,7 @@
 // is launched, counted and assumed of buffers from one call to the next.
 //   clean     a general batch finds the tile counters zero, whatever ran and
 //             grew the buffers before it
+//   launches  mr_stats.launches is the number of kernels launched (replayed)
 // Device memory is host memory, filled with 0xAB when it is allocated; a freed
 // block's address is the next allocation's.  A general batch's launches
 // check that the counters they add to are zero, and leave them so at the end,
@@ -194,9 +195,43 @@ static void check_clean() {
   mr_ctx_destroy(c);
 }
 
+static void check_launches() {
+  mr_ctx* c = open_ctx();
+  const int32_t mesh = upload(c, 4);
+  // Tables inside the argument, copied, fetched by a kernel; small, general,
+  // empty frames; the persistent kernel (one launch).
+  const int draws[] = {1, 20, 60, 0}, widths[] = {300, 1100};
+  for (int persistent = 0; persistent < 2; persistent++) {
+    mr_ctx_set_persistent(c, persistent);
+    for (int w : widths)
+      for (int n : draws) {
+        const int count = render(c, mesh, n, w, 200);
+        mr_stats st;
+        mr_ctx_get_stats(c, &st);
+        if (st.launches != count || (persistent && count != 1))
+          FAIL("%d draws, width %d, persistent %d: %d launches, counted %d", n, w, persistent, count, (int)st.launches);
+      }
+  }
+  // Replays launch what was captured, whatever ran in between.
+  mr_ctx_set_persistent(c, 0);
+  mr_ctx_set_graphs(c, 1);
+  int captured[2];
+  for (int rep = 0; rep < 4; rep++)
+    for (int k = 0; k < 2; k++) {
+      const int count = render(c, mesh, 1, widths[k], 200);
+      if (count) captured[k] = count;
+      mr_stats st;
+      mr_ctx_get_stats(c, &st);
+      if (st.launches != captured[k] || (rep == 3 && count))
+        FAIL("replay %d of width %d: counted %d of %d", rep, widths[k], (int)st.launches, captured[k]);
+    }
+  mr_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "clean")) check_clean();
+  else if (!strcmp(what, "launches")) check_launches();
   else FAIL("nothing to check");
   printf("ok\n");
   return 0;

@@ -26,3 +26,7 @@ def run(host_bin, what):
 
 def test_general_batches_find_their_counters_zero(host_bin):
     run(host_bin, "clean")
+
+
+def test_launches_counts_every_kernel(host_bin):
+    run(host_bin, "launches")
