@@ -141,7 +141,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
   plan.npixels = 0;
   plan.shade_blocks = 0;
   plan.max_width = 0;
-  plan.small_tests = plan.max_regions = 0;
+  plan.small_tests = plan.max_regions = plan.max_excess = plan.max_loose = 0;
   const int tw = c->tile_w, th = c->tile_h;
   for (int j = 0; j < nframes; j++) {
     const mr_frame* f = &frames[j];
@@ -179,6 +179,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     J.lighting = f->lighting != 0;
     J.save_normals = f->save_normals != 0;
     uint64_t order = 0;
+    int64_t loose = 0;
     // (attribute owner, modelview) -> first vertex record
     std::map<std::string, int64_t> groups;
     for (int d = 0; d < f->ndraws; d++) {
@@ -240,6 +241,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
       D.tri_begin = plan.total_tris;
       D.order_base = (uint32_t)order;
       order += 2ull * (uint64_t)m.ntri;
+      loose += m.loose;
       plan.total_tris += m.ntri;
       plan.draws.push_back(D);
       plan.draw_begin.push_back(D.tri_begin);
@@ -250,6 +252,8 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     plan.max_width = std::max(plan.max_width, J.W);
     const int64_t regions = ((J.tri_end + 63) >> 6) - (J.tri_begin >> 6);
     plan.max_regions = std::max(plan.max_regions, regions);
+    plan.max_excess = std::max(plan.max_excess, regions - npix / kSmallRegionPixels);
+    plan.max_loose = std::max(plan.max_loose, loose);
     plan.small_tests += (int64_t)J.tiles_x * J.tiles_y * regions;
   }
   if (2 * plan.total_tris >= 0xFFFFFFFFll || plan.total_verts >= 0x7FFFFFFFll) return MR_ERR_ARG;
@@ -501,7 +505,7 @@ static int launch_stages(const BatchArgs& a, Slot& s, bool profile, bool clear,
 // ones by k_tables: a frame of 31 draws (9 KB) at 640 x 480 took 42.7 us by the
 // copy and 42.3 by the kernel, of 60 draws (17 KB) 55.3 and 49.2, of 200 97 and
 // 92; 12 frames of 1,000 triangles (7 KB) 38.4 and 37.9, 32 of them 56.6 and 51.1.
-constexpr size_t kCopyTables = 12288;
+constexpr size_t kCopyTables = 9216;
 
 // Device address (null: none) of a pinned buffer, looked up when it changes.
 static void device_address(const HostBuf& b, void*& of, void*& dev) {
@@ -511,6 +515,21 @@ static void device_address(const HostBuf& b, void*& of, void*& dev) {
   if (hipHostGetDevicePointer(&d, b.p, 0) == hipSuccess) dev = d;
   else (void)hipGetLastError();
   of = b.p;
+}
+
+// Whether k_small does the batch, and in how many row bands per tile (pipeline.h).
+static bool small_batch(const BatchPlan& p) {
+  return p.max_width <= kSmallWidth && p.ntiles <= kSmallTiles && p.small_tests <= kSmallTests &&
+         (p.ntiles <= kSmallRoundTiles || p.small_tests <= kSmallRoundTests) &&
+         p.max_regions <= kSmallRegions && p.max_loose <= kSmallLoose &&
+         (p.jobs.size() == 1 || p.max_excess <= kSmallExcess);
+}
+
+static int32_t small_bands(const BatchPlan& p) {
+  if (p.max_regions <= kSmallWholeRegions && p.max_loose <= kSmallWholeLoose) return 1;
+  int32_t n = 1;
+  while (n < 8 && 2 * n * p.ntiles <= kSmallGroups) n *= 2;
+  return n;
 }
 
 static uint64_t bins_wanted(mr_ctx* c, const Slot& s, const BatchPlan& p) {
@@ -557,12 +576,13 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   }
   s.last_geom_grid = p.total_tris ? geom_grid(a) : 0;
   s.last_bin_grid = bin_grid(a);
-  // The kernels the batch runs (see BatchArgs): chosen from its size alone.
+  // The kernels the batch runs (see BatchArgs): chosen from its sizes and its
+  // meshes, and whether a small batch's records fit the checkpoint buffer (one
+  // that earlier batches have grown holds more than this batch asks for).
   a.front = !persistent && p.total_tris > 0 && p.total_tris <= kFrontTris;
-  a.small = a.front && a.host_counters && p.max_width <= kSmallWidth &&
-            p.ntiles <= kSmallTiles && p.small_tests <= kSmallTests &&
-            p.max_regions <= kSmallRegions &&
+  a.small = a.front && a.host_counters && small_batch(p) &&
             (uint64_t)a.nregions * (kRegion * sizeof(SetupRec) + 8) <= x.ckpt.bytes;
+  if (a.small) a.small_bands = small_bands(p);
   a.recs = (SetupRec*)x.ckpt.p;
   a.region_box = (uint2*)(a.recs + a.nregions * kRegion);
   // The clear kernel runs only when the counters it zeroes are not known to
@@ -1205,6 +1225,21 @@ static int upload(mr_ctx* c, DevBuf& b, const void* src, size_t bytes) {
   return MR_OK;
 }
 
+// Regions (64 consecutive triangles) of a mesh whose triangles lie apart, from
+// up to 16 of them spread over it: neighbours share corners (32 quads of a grid
+// row have 66), loose triangles or a shuffled mesh have up to 192 of their own.
+static int32_t loose_regions(const int32_t* ix, int32_t ntri) {
+  const int32_t whole = ntri / 64, n = std::min(whole, 16);
+  int32_t loose = 0;
+  for (int32_t k = 0; k < n; k++) {
+    int32_t v[192];
+    memcpy(v, ix + (size_t)((int64_t)k * whole / n) * 192, sizeof(v));
+    std::sort(v, v + 192);
+    loose += std::unique(v, v + 192) - v > 128;
+  }
+  return n ? (int32_t)(((int64_t)ntri + 63) / 64 * loose / n) : 0;
+}
+
 static bool indices_ok(const int32_t* ix, int64_t n, int32_t limit) {
   for (int64_t i = 0; i < n; i++)
     if (ix[i] < 0 || ix[i] >= limit) return false;
@@ -1229,6 +1264,7 @@ int mr_mesh_upload(mr_ctx* c, const float* positions, int32_t npos,
   MeshRec m;
   m.npos = npos; m.nnrm = nnrm; m.nuv = has_uv ? nuv : 0; m.ntri = ntri;
   m.has_uv = has_uv;
+  m.loose = loose_regions(indices, ntri);
   m.nidx_alias = normal_indices == indices;
   m.tidx_alias = has_uv && uv_indices == indices;
   int rc;
@@ -1266,6 +1302,7 @@ int mr_mesh_upload_shared(mr_ctx* c, int32_t base, const int32_t* indices,
   m.npos = o.npos; m.nnrm = o.nnrm; m.nuv = has_uv ? o.nuv : 0; m.ntri = ntri;
   m.has_uv = has_uv;
   m.owner = owner;
+  m.loose = loose_regions(indices, ntri);
   m.nidx_alias = normal_indices == indices;
   m.tidx_alias = has_uv && uv_indices == indices;
   int rc;

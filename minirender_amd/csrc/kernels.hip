@@ -2157,24 +2157,27 @@ __global__ __launch_bounds__(kShadeBlock, 7) void k_shade(BatchArgs a) {
 // Raster and shading of a batch whose tiles test the job's items themselves
 // (no counting, scan or binning, and no kernel boundary before shading): one
 // workgroup per tile tests the boxes of its job's regions, then the items of
-// the regions its tile meets, kSmallRound regions at a time, draws those whose
+// the regions its tile meets, kSmallStep regions at a time, draws those whose
 // bbox meets the tile from the setup records geometry wrote and shades its
 // pixels.  The frames this is for are bound by the chain of launches and of
 // dependent loads in each; no edge checkpoints are taken (their rows are at
 // most kSmallWidth steps).
-constexpr int kSmallRound = 16;
+constexpr int kSmallStep = 16;
 
-template <int TW, int NT>
+template <int TW, int NT, bool kBands>
 __global__ __launch_bounds__(NT, 4) void k_small(BatchArgs a) {
-  constexpr int TH = TW, NP = TW * TH, NW = NT / 64, KS = RasterLds<TW, TH, NT>::KS;
+  constexpr int TH = TW, NW = NT / 64, KS = RasterLds<TW, TH, NT>::KS;
   __shared__ RasterLds<TW, TH, NT> lds;
   __shared__ int64_t dcache[kMaxLdsDraws];
   __shared__ uint16_t regs[kSmallRegions];           // regions met, from the job's first on
-  __shared__ uint16_t match[kSmallRound * kRegion];  // items met: (place in the round, slot)
+  __shared__ uint16_t match[kSmallStep * kRegion];  // items met: (place in the round, slot)
   __shared__ uint32_t nregs, nmatch;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tile = (int)blockIdx.x;  // (neighbours on other XCDs: an even share of the frame)
+  const int band_rows = kBands ? TH / a.small_bands : TH;
+  const int band_lo = kBands ? (int)blockIdx.y * band_rows : 0;
+  const int band_hi = band_lo + band_rows - 1;
   const int j = __builtin_amdgcn_readfirstlane(
       job_lookup(a.tile_hint, a.job_tile_base, a.njobs, tile));
   // What testing needs of the job; shading reads all of it, again, below.
@@ -2200,7 +2203,7 @@ __global__ __launch_bounds__(NT, 4) void k_small(BatchArgs a) {
   };
   auto meets = [&](uint32_t bx, uint32_t by) {  // first | last << 16
     return (int)(bx & 0xFFFFu) < x0 + TW && (int)(bx >> 16) >= x0 &&
-           (int)(by & 0xFFFFu) < y0 + TH && (int)(by >> 16) >= y0;
+           (int)(by & 0xFFFFu) <= y0 + band_hi && (int)(by >> 16) >= y0 + band_lo;
   };
   for (int i = tid; i - tid < nr; i += NT) {
     const uint2 box = a.region_box[r0 + min(i, nr - 1)];
@@ -2208,8 +2211,8 @@ __global__ __launch_bounds__(NT, 4) void k_small(BatchArgs a) {
   }
   __syncthreads();
   const int met = (int)nregs;
-  for (int q0 = 0; q0 < met; q0 += kSmallRound) {
-    constexpr int kAhead = kSmallRound / NW;  // regions in flight per wavefront
+  for (int q0 = 0; q0 < met; q0 += kSmallStep) {
+    constexpr int kAhead = kSmallStep / NW;  // regions in flight per wavefront
     // (Every slot of a region is allocated; those past its count are read and
     // not used: loads under conditions wait for each other.)
     uint4 it[kAhead];
@@ -2245,7 +2248,8 @@ __global__ __launch_bounds__(NT, 4) void k_small(BatchArgs a) {
         const uint32_t m = match[base + tid];
         be.x = (uint32_t)((r0 + regs[q0 + m / kRegion]) * kRegion + m % kRegion);
       }
-      raster_chunk<TW, TH, NT, true>(a, a.jobs[j], lds, base + tid < n, be, x0, y0, 0, TH - 1);
+      raster_chunk<TW, TH, NT, true>(a, a.jobs[j], lds, base + tid < n, be, x0, y0, band_lo,
+                                     band_hi);
     }
     if (n == 0) __syncthreads();
     if (tid == 0) nmatch = 0;
@@ -2257,13 +2261,13 @@ __global__ __launch_bounds__(NT, 4) void k_small(BatchArgs a) {
   const bool one_draw = ndraws == 1;
   const int ncached = one_draw ? -1 : fill_draw_cache(dcache, a, J, tid, NT);
   __syncthreads();
-  for (int p = tid; p < NP; p += NT) {
+  for (int p = band_lo * TW + tid; p < (band_hi + 1) * TW; p += NT) {
     const int c = x0 + p % TW, row = y0 + p / TW;
     const u64 key = lds.keys[(p / TW) * KS + p % TW];
     if (c < J.W && row < J.H)
       shade_pixel<false>(a, J, dcache, ncached, key == ~0ull ? kNoWinner : (uint32_t)key, c, row);
   }
-  if (blockIdx.x != 0 || !a.host_counters) return;
+  if (blockIdx.x != 0 || (kBands && blockIdx.y != 0) || !a.host_counters) return;
   // Statistics of the batch, to the host (the batch counters are not used).
   const int ng = geom_grid(a);
   u64 clipped = 0, items = 0, pairs = 0;
@@ -2646,11 +2650,18 @@ hipError_t launch_front(const BatchArgs& a, const void* tables, size_t table_byt
   return hipGetLastError();
 }
 
-hipError_t launch_small(const BatchArgs& a, hipStream_t s) {
-  if (a.tile_w == 8) hipLaunchKernelGGL((k_small<8, 64>), dim3(a.ntiles), dim3(64), 0, s, a);
-  else if (a.tile_w == 16) hipLaunchKernelGGL((k_small<16, 256>), dim3(a.ntiles), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((k_small<32, 256>), dim3(a.ntiles), dim3(256), 0, s, a);
+template <int TW, int NT>
+static hipError_t launch_small_as(const BatchArgs& a, hipStream_t s) {
+  const dim3 grid(a.ntiles, a.small_bands);
+  if (a.small_bands == 1) hipLaunchKernelGGL((k_small<TW, NT, false>), grid, dim3(NT), 0, s, a);
+  else hipLaunchKernelGGL((k_small<TW, NT, true>), grid, dim3(NT), 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_small(const BatchArgs& a, hipStream_t s) {
+  if (a.tile_w == 8) return launch_small_as<8, 64>(a, s);
+  if (a.tile_w == 16) return launch_small_as<16, 256>(a, s);
+  return launch_small_as<32, 256>(a, s);
 }
 
 hipError_t launch_scan(const BatchArgs& a, hipStream_t s) {

@@ -111,6 +111,7 @@ struct BatchArgs {
   // the vertices itself (k_front) and needs the batch counters zero before.
   // small: front, and the tiles test the items themselves (k_small).
   int32_t front, small;
+  int32_t small_bands;       // workgroups per tile of k_small, each a band of its rows
 };
 
 // The argument of a batch's first kernel: with nwords, the batch tables too.
@@ -126,18 +127,37 @@ struct TableArgs {
 // kernels together 16.3 -> 12.0 us at 120 k triangles, 35 -> 32.5 at 1 M, but
 // 55 -> 61 at 2.1 M).
 constexpr int64_t kFrontTris = 1500000;
-// Small batches: frames at most kSmallWidth wide (rows are walked from the
-// bbox's left column), at most kSmallTiles tiles (beyond a few rounds of
-// workgroups throughput counts, not latency), which test at most kSmallTests
-// regions together when every region meets every tile (triangles in random
-// order).  Against the general kernels (a frame's call, us): sphere of 4 k
-// triangles at 640 x 480 59 -> 33, grid of 5 k at 1000 x 1000 83 -> 57, 1,000
-// large overlapping triangles at 640 x 480 78 -> 51, 2,500 of them at 1000 x 600
-// 129 -> 133; a batch of 40 frames of 250 x 250 (10,240 tiles) 121 -> 130.
-constexpr int kSmallWidth = 1024;
+// Small batches (k_front and k_small, whose tiles test every region of their
+// job): what the two kernels do sooner than the general ones (us a call, small
+// and general; 64 triangles a region).
+constexpr int kSmallWidth = 1024;  // rows are walked from the bbox's left column
 constexpr int kSmallTiles = 8192;
+// (tile, region) pairs tested.  Few tiles run beside each other (a grid of
+// 16,000 at 1000 x 700, 693,000 pairs: 48 and 56), more in rounds: 16 frames of
+// 256 tiles and 74 regions (303,000) 68 and 67, 30 of them 98 and 86, 30 frames
+// of 24 regions (184,000) 81 and 84.
 constexpr int64_t kSmallTests = 800000;
-constexpr int kSmallRegions = 2048;  // of one job at most (k_small lists them in LDS)
+constexpr int kSmallRoundTiles = 3072;
+constexpr int64_t kSmallRoundTests = 300000;  // of batches of more tiles
+// Regions of one job (k_small lists them in LDS): grids at 320 x 240 of 469 take
+// 42 and 47, of 938 48 and 47, of 2,000 56 and 47; spheres 35 and 53, 39 and 53,
+// 40 and 50.
+constexpr int kSmallRegions = 1536;
+// Regions of a job beside others, whose few tiles are not shared out further:
+// one per kSmallRegionPixels and kSmallExcess (24 frames of 1 k - 60 k triangles
+// at 200 x 150 to 33 x 33: 87 and 69).
+constexpr int64_t kSmallRegionPixels = 512, kSmallExcess = 80;
+// Regions of a job with triangles in no spatial order: every tile meets them
+// all, where it meets 1 in 10 of a grid's.  6,000 small triangles 46 and 43 at
+// 320 x 240, 20,000 92 and 46; 6,000 larger ones 62 and 71.
+constexpr int64_t kSmallLoose = 112;
+// A tile is drawn by one workgroup, or by up to 8, each a band of its rows,
+// while that makes at most kSmallGroups (about what the GPU holds at once): a
+// frame of few tiles left most CUs idle while each tile drew thousands of
+// entries (4,000 overlapping triangles at 96 x 64 942 -> 160 us, 5,000 random
+// ones 127 -> 60).  Frames of few regions gain nothing.
+constexpr int kSmallGroups = 1024;
+constexpr int64_t kSmallWholeRegions = 96, kSmallWholeLoose = 4;
 
 constexpr int64_t kCkptScanRegions = 65536;
 

@@ -4,6 +4,8 @@
 //   clean     a general batch finds the tile counters zero, whatever ran and
 //             grew the buffers before it
 //   launches  mr_stats.launches is the number of kernels launched (replayed)
+//   small     which batches the two kernels of small batches get, and in how
+//             many row bands per tile
 // Device memory is host memory, filled with 0xAB when it is allocated; a freed
 // block's address is the next allocation's.  A general batch's launches
 // check that the counters they add to are zero, and leave them so at the end,
@@ -75,6 +77,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0; ret
 namespace mr {
 static int g_launches = 0;  // kernels launched
 static bool g_general = false, g_small = false;
+static int g_bands = 0;  // of the last small batch
 
 static void zero(const BatchArgs& a) {
   memset(a.counters, 0, kNumCounters * 8);
@@ -116,6 +119,9 @@ hipError_t launch_front(const BatchArgs& a, const void*, size_t, hipStream_t) { 
 hipError_t launch_small(const BatchArgs& a, hipStream_t) {
   g_launches++;
   g_small = true;
+  g_bands = a.small_bands;
+  if (a.small_bands < 1 || a.tile_h % a.small_bands || (a.small_bands > 1 && a.small_bands * a.ntiles > kSmallGroups))
+    FAIL("%d bands of %d rows, %d tiles", a.small_bands, a.tile_h, a.ntiles);
   memset(a.host_counters, 0, kNumCounters * 8);
   return hipSuccess;
 }
@@ -147,18 +153,19 @@ static mr_ctx* open_ctx() {
   if (mr_ctx_create(0, 0, &c)) FAIL("context");
   return c;
 }
-static int32_t upload(mr_ctx* c, int ntri) {
+// strip: neighbouring triangles share corners; else each has its own.
+static int32_t upload(mr_ctx* c, int ntri, bool strip = false) {
   std::vector<float> v(9 * (size_t)ntri);
   std::vector<int32_t> ix(3 * (size_t)ntri);
-  for (int i = 0; i < 3 * ntri; i++) ix[i] = i;
+  for (int i = 0; i < 3 * ntri; i++) ix[i] = strip ? i / 3 + i % 3 : i;
   int32_t h;
   if (mr_mesh_upload(c, v.data(), 3 * ntri, v.data(), 3 * ntri, nullptr, 0, ix.data(), ix.data(), nullptr, ntri, &h))
     FAIL("upload");
   return h;
 }
-// A frame of `ndraws` draws of a mesh, its image in host memory; returns the
-// kernels it launched.
-static int render(mr_ctx* c, int32_t mesh, int ndraws, int w, int h) {
+// `n` frames of `ndraws` draws of a mesh, their images in host memory; returns
+// the kernels launched.
+static int render(mr_ctx* c, int32_t mesh, int ndraws, int w, int h, int n = 1) {
   std::vector<mr_draw> draws(ndraws);
   for (mr_draw& d : draws) {
     memset(&d, 0, sizeof(d));
@@ -176,9 +183,11 @@ static int render(mr_ctx* c, int32_t mesh, int ndraws, int w, int h) {
   mr_outputs o;
   memset(&o, 0, sizeof(o));
   o.rgb8 = rgb.data();
+  const std::vector<mr_frame> frames(n, f);
+  const std::vector<mr_outputs> outs(n, o);
   const int before = mr::g_launches;
   mr::g_general = mr::g_small = false;
-  const int rc = mr_render(c, &f, &o);
+  const int rc = mr_render_batch(c, frames.data(), n, outs.data());
   if (rc) FAIL("%d x %d: status %d", w, h, rc);
   return mr::g_launches - before;
 }
@@ -228,10 +237,43 @@ static void check_launches() {
   mr_ctx_destroy(c);
 }
 
+static void check_small() {
+  mr_ctx* c = open_ctx();
+  render(c, upload(c, 4), 1, 3840, 2160);  // buffers large enough for all below
+  const struct { int ntri; bool strip; int w, h, n, bands; } cases[] = {
+      {64, true, 96, 64, 1, 1},         // few regions
+      {4000, true, 96, 64, 1, 1},
+      {7000, true, 96, 64, 1, 8},       // 24 tiles
+      {5000, false, 256, 128, 1, 8},    // 128 tiles
+      {5000, false, 250, 145, 1, 4},    // 160 tiles
+      {5000, false, 512, 256, 1, 2},
+      {5000, false, 432, 304, 1, 1},    // 513 tiles
+      {7168, false, 320, 240, 1, 2},    // 112 loose regions
+      {7169, false, 320, 240, 1, 0},    // one more
+      {20000, false, 640, 480, 1, 0},
+      {20000, true, 640, 480, 1, 1},
+      {98304, true, 320, 240, 1, 2},    // 1,536 regions
+      {98305, true, 320, 240, 1, 0},
+      {4713, true, 250, 250, 12, 1},    // 3,072 tiles
+      {4713, true, 250, 250, 16, 0},    // 303,000 tests of 4,096 tiles
+      {1500, true, 250, 250, 30, 1},
+      {5824, true, 96, 64, 8, 1},       // 91 regions a job, 92 allowed beside others
+      {5952, true, 96, 64, 8, 0},       // 93
+  };
+  for (auto& k : cases) {
+    render(c, upload(c, k.ntri, k.strip), 1, k.w, k.h, k.n);
+    if (mr::g_small != (k.bands != 0) || (k.bands && mr::g_bands != k.bands))
+      FAIL("%d triangles (strip %d), %d of %d x %d: small %d, %d bands, not %d", k.ntri, k.strip, k.n, k.w, k.h,
+           mr::g_small, mr::g_bands, k.bands);
+  }
+  mr_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "clean")) check_clean();
   else if (!strcmp(what, "launches")) check_launches();
+  else if (!strcmp(what, "small")) check_small();
   else FAIL("nothing to check");
   printf("ok\n");
   return 0;

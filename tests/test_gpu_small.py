@@ -130,3 +130,26 @@ def test_general_special_cases(gpu_ctx, tile):
         gpu_ctx.set_band_work(32768)
         gpu_ctx.set_frag_size(1024)
         gpu_ctx.set_tile(16, 16)
+
+
+@pytest.mark.parametrize("tile,w,h", [(16, 256, 128), (16, 250, 125), (16, 48, 688), (16, 256, 256), (16, 16, 4112),
+                                      (16, 512, 256), (16, 432, 304), (8, 128, 64), (8, 60, 61), (8, 256, 64),
+                                      (32, 512, 256), (32, 70, 50), (32, 511, 513)])
+def test_row_bands(gpu_ctx, tile, w, h):
+    """Tiles drawn by several workgroups, each a band of rows: on both sides of
+    128, 256 and 512 tiles (8, 4, 2 and 1 band), frames that end inside a
+    band, near-clipped and large triangles; every output bit for bit."""
+    tris = scenes.random_triangles(500, 11, lo=0.05, hi=1.2, center_lo=(-1, -1, -3), center_hi=(1, 1, -0.4))
+    f = FrameSpec(w, h, scenes.projection_frustum(1.0, w / h, 0.5, 30.0),
+                  draws=[Draw(tris, Material(shininess=9.0))], light=(0.2, 0.4, 1.0), save_normals=True)
+    gpu_ctx.set_tile(tile, tile)
+    try:
+        small = gpu_ctx.render(f, ALL)
+        st = gpu_ctx.stats()
+        assert st.launches == 2
+        general = gpu_ctx.render_batch([f, wide()], ALL)[0]
+        assert gpu_ctx.stats().launches > 2
+    finally:
+        gpu_ctx.set_tile(16, 16)
+    assert st.records > 0
+    same(small, general, ALL, f"{w} x {h} t{tile}")

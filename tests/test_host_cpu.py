@@ -30,3 +30,10 @@ def test_general_batches_find_their_counters_zero(host_bin):
 
 def test_launches_counts_every_kernel(host_bin):
     run(host_bin, "launches")
+
+
+def test_small_batches_are_those_that_gain(host_bin):
+    """Triangles in no order, too many of them for a job's tiles, batches of
+    many tests take the general kernels; frames of few tiles are shared out in
+    row bands."""
+    run(host_bin, "small")
