@@ -76,17 +76,15 @@ __device__ __forceinline__ void zero_counters(const BatchArgs& a) {
 }
 
 // A tile's line of words (tile_count): pairs and work, direct entries, and in
-// a job's first tile the length and box of the job's direct list.
+// a job's first tile the length of the job's direct list.
 __device__ __forceinline__ void zero_tile(const BatchArgs& a, int i) {
   ulonglong2* const line = (ulonglong2*)(a.tile_count + (size_t)i * kCtrStride64);
-  line[0] = line[1] = line[2] = make_ulonglong2(0ull, 0ull);
+  line[0] = line[1] = make_ulonglong2(0ull, 0ull);
   a.tile_done[i] = 0;
 }
 
-// The direct list's line of the job with first tile `tile_base`: the number
-// of its items, then kMaxDim - first column, last column, kMaxDim - first row
-// and last row of their bounding box.
-__device__ __forceinline__ uint32_t* direct_line(const BatchArgs& a, int tile_base) {
+// The length of the direct list of the job with first tile `tile_base`.
+__device__ __forceinline__ uint32_t* direct_length(const BatchArgs& a, int tile_base) {
   return (uint32_t*)(a.tile_count + (size_t)tile_base * kCtrStride64 + 2);
 }
 
@@ -611,24 +609,8 @@ __device__ inline void direct_append(const BatchArgs& a, int job, int tile_base,
     const bool mine = (d0 || d1) && ((pend >> lane) & 1ull) && job == jj;
     const u64 g0 = __ballot(mine && d0), g1 = __ballot(mine && d1);
     uint32_t base = 0;
-    uint32_t* const line = direct_line(a, __builtin_amdgcn_readlane(tile_base, l));
-    if (lane == l) base = atomicAdd(line, (uint32_t)(__popcll(g0) + __popcll(g1)));
-    // Bounding box of the job's list (as maxima: the words start at zero).
-    uint32_t box[4] = {0, 0, 0, 0};
-    if (mine) {
-      const BinItem& p = d0 ? i0 : i1;
-      const BinItem& q = d1 ? i1 : i0;
-      box[0] = (uint32_t)(kMaxDim - min(p.bx0, q.bx0));
-      box[1] = max(p.bx1, q.bx1);
-      box[2] = (uint32_t)(kMaxDim - min(p.by0, q.by0));
-      box[3] = max(p.by1, q.by1);
-    }
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) box[k] = max(box[k], (uint32_t)__shfl_xor(box[k], o));
-      if (lane == l) atomicMax(line + 1 + k, box[k]);
-    }
+    uint32_t* const length = direct_length(a, __builtin_amdgcn_readlane(tile_base, l));
+    if (lane == l) base = atomicAdd(length, (uint32_t)(__popcll(g0) + __popcll(g1)));
     base = (uint32_t)__builtin_amdgcn_readlane((int)base, l);
     pend &= ~(g0 | g1);
     if (mine) {
@@ -949,7 +931,7 @@ __device__ __forceinline__ void stage_scan(const BatchArgs& a, int blk) {
     for (int i = 0; i < kItems; i++) {
       if (base + i < a.ntiles && (i == 0 || base + i >= next)) {
         if (i) j++;
-        any = *direct_line(a, a.job_tile_base[j]) != 0;
+        any = *direct_length(a, a.job_tile_base[j]) != 0;
         next = j + 1 < a.njobs ? a.job_tile_base[j + 1] : 0x7FFFFFFF;
       }
       listed |= (any ? 1u : 0u) << i;
@@ -1337,7 +1319,7 @@ __device__ __forceinline__ void stage_direct(const BatchArgs& a, int vb, int nvb
     int groups = 0;    // of the lists of the jobs here
     bool own = false;  // this tile's job has a list
     for (int j = j0; j < a.njobs && a.job_tile_base[j] < t_end; j++) {
-      const int nd = (int)min(*direct_line(a, a.job_tile_base[j]), a.direct_cap);
+      const int nd = (int)min(*direct_length(a, a.job_tile_base[j]), a.direct_cap);
       groups += (nd + kDirectGroup - 1) / kDirectGroup;
       if (t >= a.job_tile_base[j]) own = nd != 0;
     }
@@ -1349,7 +1331,7 @@ __device__ __forceinline__ void stage_direct(const BatchArgs& a, int vb, int nvb
     for (int pass = 0; pass < 2; pass++) {
       // (The tiles usually lie in one job.)
       for (int j = j0; j < a.njobs && a.job_tile_base[j] < t_end; j++) {
-        const int nd = (int)min(*direct_line(a, a.job_tile_base[j]), a.direct_cap);
+        const int nd = (int)min(*direct_length(a, a.job_tile_base[j]), a.direct_cap);
         if (nd == 0) continue;
         const JobDesc& J = a.jobs[j];
         const int local = t - J.tile_base;

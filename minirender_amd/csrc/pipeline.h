@@ -20,7 +20,7 @@ struct BatchArgs {
   BinItem* items;            // [nregions * kRegion] survivors, per wavefront
   uint32_t* region_count;    // [nregions] survivors of each wavefront
   // Direct items of each job, behind the checkpoints in the checkpoint
-  // buffer's last quarter (their number: direct_line in kernels.hip).
+  // buffer's last quarter (their number: direct_length in kernels.hip).
   BinItem* direct;           // [njobs * direct_cap]
   uint32_t direct_cap;
   int64_t nregions;

@@ -73,3 +73,17 @@ def test_persistent_shading_reads_tile_flags_by_vector_loads(assembly, tmp_path)
     bad, found = scalar_reads_of(body[:body.index(".Lfunc_end")], offset)
     assert found
     assert not bad, bad
+
+
+@pytest.mark.parametrize("kernel", ["k_geom", "k_front"])
+def test_geometry_takes_no_maxima_to_memory(assembly, kernel):
+    """Geometry adds to counters only: a direct list is a length and its items
+    (a bounding box of it, kept by atomic maxima on one line per job, was read
+    by nothing)."""
+    names = re.findall(rf"^(_ZN2mr\S*{kernel}\S*):", assembly, re.M)
+    assert names
+    for name in names:
+        body = assembly[assembly.index(f"\n{name}:"):]
+        body = body[:body.index(".Lfunc_end")]
+        assert "global_atomic_add" in body or "ILb1E" in name  # (small batches count nothing)
+        assert not re.findall(r"(?:global|flat)_atomic_u?max\S*", body)
