@@ -97,7 +97,7 @@ enum Counter : int {
   kHeavy = 8,        // tiles split over several work items
   kHeavyOverflow = 9,
   kListed = 10,      // tiles in the raster's tile list (written by the scan)
-  kDirect = 11,      // direct items of all jobs (0: the direct lists are empty)
+  kDirect = 11,      // direct items of all jobs, listed or (no room) binned after all
   kDirectPairs = 14, // (tile, direct item) pairs, at the end of the bin list
   kDirectTilesListed = 15,  // tiles with such pairs only, at the end of the tile list
   kWidePx = 12,      // bbox pixels of the items that want edge checkpoints ...
@@ -128,6 +128,39 @@ MR_HD inline TileItems tile_items(const unsigned long long* counters, uint32_t p
   r.listed = r.whole + (int64_t)counters[kDirectTilesListed];
   if (r.listed > ntiles) r.listed = ntiles;
   return r;
+}
+
+// Row bands that each tile rastered whole is shared out in.  A tile's direct
+// entries (up to kDirectCap) are not among those that the scan splits tiles
+// by, so one workgroup a tile would draw them all, however few tiles there are.
+// From kBandDirect items (a chunk of the raster) up to 8 workgroups draw a
+// tile while these are at most kBandGroups, about what the GPU holds, and the
+// raster's grid (ntiles + parts_cap) holds them anyway.  With the shares of
+// split tiles (direct_share), us a call: 8,000 triangles over a 96 x 64 frame
+// 376 -> 310 (335 with all of them binned and split), 20,000 690 -> 404 (430);
+// 20,000 over 320 x 240 885 -> 636.
+constexpr int64_t kBandGroups = 1024;
+constexpr unsigned long long kBandDirect = 256;
+MR_HD inline int whole_bands(const unsigned long long* counters, const TileItems& r,
+                             uint32_t parts_cap, int32_t ntiles, int tile_h) {
+  int n = 1;
+  if (counters[kDirect] < kBandDirect) return n;
+  while (n < 8 && 2 * n <= tile_h && 2 * n * r.listed <= kBandGroups &&
+         r.parts + 2 * n * r.listed <= (int64_t)ntiles + parts_cap)
+    n *= 2;
+  return n;
+}
+
+// Entries [first, end) of a tile's n direct ones that part `part` of the tile
+// draws.
+struct DirectShare {
+  uint32_t first, end;
+};
+MR_HD inline DirectShare direct_share(uint32_t n, uint32_t part, uint32_t nparts) {
+  if (nparts == 1) return {0, n};
+  const uint32_t q = n / nparts, rest = n % nparts;
+  const uint32_t first = part * q + (part < rest ? part : rest);
+  return {first, first + q + (part < rest ? 1u : 0u)};
 }
 
 // Workgroup index b in [0, n) -> work index, a bijection under which each of

@@ -602,7 +602,8 @@ __device__ inline void direct_append(const BatchArgs& a, int job, int tile_base,
   const int lane = threadIdx.x & 63;
   const u64 lt = (1ull << lane) - 1ull;
   u64 pend = __ballot(d0 || d1);
-  if (lane == (int)__builtin_ctzll(pend)) atomicAdd(&a.counters[kDirect], 1ull);
+  const int nd = __popcll(__ballot(d0)) + __popcll(__ballot(d1));
+  if (lane == (int)__builtin_ctzll(pend)) atomicAdd(&a.counters[kDirect], (u64)nd);
   while (pend) {
     const int l = __builtin_ctzll(pend);
     const int jj = __builtin_amdgcn_readlane(job, l);
@@ -1620,7 +1621,8 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
   const int tid = threadIdx.x;
   bool direct = a.counters[kDirect] != 0ull;
   const TileItems items = tile_items(a);
-  if (b >= items.parts + items.listed) return;
+  const int bands = whole_bands(a.counters, items, a.parts_cap, a.ntiles, TH);
+  if (b >= items.parts + items.listed * bands) return;
   int tile, part;
   uint32_t cnt, off;  // the tile's bin entries: number and first
   int band_lo = 0, band_hi = TH - 1;  // tile rows of this work item
@@ -1642,7 +1644,13 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     // (one load fewer before the bin entries); tiles without bin entries
     // are not in it (shading writes their background).
     // (Tiles with direct entries only are listed from the end.)
-    const int64_t t = b - items.parts;
+    int64_t t = b - items.parts;
+    if (bands > 1) {  // (few tiles)
+      const int bi = (int)((uint32_t)t / (uint32_t)items.listed);
+      t -= bi * items.listed;
+      band_lo = bi * (TH / bands);
+      band_hi = band_lo + TH / bands - 1;
+    }
     const int64_t li = remap ? (int64_t)xcd_chunks<kXcdChunk>((uint32_t)t, (uint32_t)items.listed) : t;
     const uint4 le = a.tile_list[li < items.whole ? li : a.ntiles - 1 - (li - items.whole)];
     tile = (int)le.x;
@@ -1663,14 +1671,15 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     else if ((u64)off + cnt > a.bins_cap) avail = (uint32_t)(a.bins_cap - off);
     const uint32_t e_begin = (uint32_t)part * a.frag_size;
     const uint32_t e_end = min(avail, e_begin + a.frag_size);
-    // The entries: the bin entries, then (by the first part of a split tile)
-    // the direct ones.
+    // The entries: the bin entries, then the direct ones (a split tile's
+    // parts share them).
     const uint32_t nbin = e_end > e_begin ? e_end - e_begin : 0u;
     uint32_t nall = nbin, off2 = 0;
-    if (direct && part == 0) {
+    if (direct) {
       const u64 range = a.tile_count[(size_t)tile * kCtrStride64 + 1];
-      off2 = (uint32_t)range - nbin;
-      nall += (uint32_t)(range >> 32);
+      const DirectShare ds = direct_share((uint32_t)(range >> 32), (uint32_t)part, nparts);
+      off2 = (uint32_t)range + ds.first - nbin;
+      nall += ds.end - ds.first;
     }
     for (int p = tid; p < TH * KS; p += NT) keys[p] = ~0ull;
     __syncthreads();
@@ -2306,7 +2315,8 @@ __device__ inline u64 ctl_load(const u64* p) {
 __device__ inline int64_t persist_stage_size(const BatchArgs& a, const PersistPlan& q, int s) {
   if (s != kPTile) return q.nvb[s];
   const TileItems items = tile_items(a);
-  return min((int64_t)q.nvb[s], items.parts + items.listed);
+  const int bands = whole_bands(a.counters, items, a.parts_cap, a.ntiles, a.tile_h);
+  return min((int64_t)q.nvb[s], items.parts + items.listed * bands);
 }
 
 // Queue x's share of a stage of n workgroups: first workgroup, count, and

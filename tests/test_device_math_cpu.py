@@ -69,3 +69,12 @@ def test_nothing_drawn_from_a_bin_list_that_overflowed(tmp_path_factory):
     r = subprocess.run([str(out), "20000"], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.strip() == "ok"
+
+
+def test_direct_entries_are_shared_out(tmp_path_factory):
+    """share_check: no workgroup draws all of a long list of large triangles
+    alone while others have nothing to do, and each entry is drawn once."""
+    out = _build(tmp_path_factory, "share_check")
+    r = subprocess.run([str(out)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.strip() == "ok"

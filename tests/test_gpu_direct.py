@@ -114,3 +114,37 @@ def test_both_ends_of_the_bin_list_meet(persistent, small_first):
         assert ctx.stats().retries >= 1
     for i, (g, f) in enumerate(zip(out, frames)):
         assert_parity(g, oracle_py.render(f, KINDS), f"job {i}")
+
+
+@pytest.mark.parametrize("tile,n,w,h,persistent", [
+    (16, 1300, 1040, 16, False), (16, 1300, 1040, 31, False), (16, 1300, 1033, 64, False), (16, 1300, 1040, 128, False),
+    (16, 1300, 1040, 31, True), (16, 1300, 1033, 64, True), (8, 1300, 1026, 8, False), (32, 2000, 1057, 70, False)])
+def test_bands_of_listed_items(gpu_ctx, tile, n, w, h, persistent):
+    """Few tiles (8, 4, 2 and 1 row bands each) and more large triangles than
+    one round of the raster: tiles with binned entries, with listed ones only
+    and with both, frames that end inside a band."""
+    tris = scenes.random_triangles(600, 13, lo=0.02, hi=0.02, center_lo=(-30, -2, -3), center_hi=(30, 2, -1))
+    big = scenes.random_triangles(n, 12, lo=0.5, hi=8.0, center_lo=(-20, -0.2, -3), center_hi=(8, 0.2, -1))
+    f = FrameSpec(w, h, scenes.projection_frustum(math.radians(5), w / h, 0.5, 50.0),
+                  draws=[Draw(big, Material()), Draw(tris, Material())], light=(0.3, 0.5, 1.0))
+    gpu_ctx.set_tile(tile, tile)
+    gpu_ctx.set_persistent(persistent)
+    try:
+        check(gpu_ctx, f, f"bands {w} x {h} t{tile}")
+    finally:
+        gpu_ctx.set_persistent(False)
+        gpu_ctx.set_tile(16, 16)
+
+
+@pytest.mark.parametrize("frag", [256, 1000])
+def test_split_tiles_share_listed_items(gpu_ctx, frag):
+    """Tiles split by their binned entries, with listed ones beside them: a
+    list that runs over, in parts of both kinds."""
+    tris = scenes.random_triangles(14000, 14, lo=0.3, hi=3.0, center_lo=(-8, -0.3, -3), center_hi=(8, 0.3, -1))
+    f = FrameSpec(1100, 40, scenes.projection_frustum(math.radians(10), 27.5, 0.5, 50.0),
+                  draws=[Draw(tris, Material(shininess=5.0))], light=(0.3, 0.5, 1.0))
+    gpu_ctx.set_frag_size(frag)
+    try:
+        check(gpu_ctx, f, f"split {frag}")
+    finally:
+        gpu_ctx.set_frag_size(1024)
