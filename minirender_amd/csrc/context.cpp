@@ -14,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 #include <map>
+#include <memory>
 #include <new>
 #include <string>
 #include <vector>
@@ -141,7 +142,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
   plan.npixels = 0;
   plan.shade_blocks = 0;
   plan.max_width = 0;
-  plan.small_tests = plan.max_regions = plan.max_excess = plan.max_loose = 0;
+  plan.small_tests = plan.max_regions = plan.max_excess = plan.max_loose = plan.max_scatter = 0;
   const int tw = c->tile_w, th = c->tile_h;
   for (int j = 0; j < nframes; j++) {
     const mr_frame* f = &frames[j];
@@ -179,7 +180,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     J.lighting = f->lighting != 0;
     J.save_normals = f->save_normals != 0;
     uint64_t order = 0;
-    int64_t loose = 0;
+    int64_t loose = 0, scatter = 0;
     // (attribute owner, modelview) -> first vertex record
     std::map<std::string, int64_t> groups;
     for (int d = 0; d < f->ndraws; d++) {
@@ -242,6 +243,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
       D.order_base = (uint32_t)order;
       order += 2ull * (uint64_t)m.ntri;
       loose += m.loose;
+      scatter += m.scatter;
       plan.total_tris += m.ntri;
       plan.draws.push_back(D);
       plan.draw_begin.push_back(D.tri_begin);
@@ -254,6 +256,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     plan.max_regions = std::max(plan.max_regions, regions);
     plan.max_excess = std::max(plan.max_excess, regions - npix / kSmallRegionPixels);
     plan.max_loose = std::max(plan.max_loose, loose);
+    plan.max_scatter = std::max(plan.max_scatter, scatter);
     plan.small_tests += (int64_t)J.tiles_x * J.tiles_y * regions;
   }
   if (2 * plan.total_tris >= 0xFFFFFFFFll || plan.total_verts >= 0x7FFFFFFFll) return MR_ERR_ARG;
@@ -521,7 +524,7 @@ static void device_address(const HostBuf& b, void*& of, void*& dev) {
 static bool small_batch(const BatchPlan& p) {
   return p.max_width <= kSmallWidth && p.ntiles <= kSmallTiles && p.small_tests <= kSmallTests &&
          (p.ntiles <= kSmallRoundTiles || p.small_tests <= kSmallRoundTests) &&
-         p.max_regions <= kSmallRegions && p.max_loose <= kSmallLoose &&
+         p.max_regions <= kSmallRegions && p.max_scatter <= kSmallLoose * kScatterWeight &&
          (p.jobs.size() == 1 || p.max_excess <= kSmallExcess);
 }
 
@@ -1046,6 +1049,60 @@ int render_frames(mr_ctx* c, const mr_frame* frames, int n, const mr_outputs* ou
 // ---------------------------------------------------------------------------
 // C-ABI
 // ---------------------------------------------------------------------------
+// Regions (64 consecutive triangles) of a mesh whose triangles lie apart, from
+// up to 16 of them spread over it: neighbours share corners (32 quads of a grid
+// row have 66), loose triangles or a shuffled mesh have up to 192 of their own.
+// m.scatter: how far such regions count against kSmallLoose, by the triangles'
+// extent in the region's (root of the mean square of the longest sides).
+// Meshes of more triangles than a small batch takes are not looked at.
+// positions(lo, n): n vertices from lo on in host memory, or null.
+template <typename Positions>
+static void look_at_regions(MeshRec& m, const int32_t* ix, Positions&& positions) {
+  const int32_t whole = m.ntri / 64, n = std::min(whole, 16);
+  if (n == 0 || whole > kSmallRegions) return;
+  const int32_t* apart[16];
+  int32_t loose = 0, lo = INT32_MAX, hi = 0;
+  for (int32_t k = 0; k < n; k++) {
+    const int32_t* const r = ix + (size_t)((int64_t)k * whole / n) * 192;
+    int32_t v[192];
+    memcpy(v, r, sizeof(v));
+    std::sort(v, v + 192);
+    if (std::unique(v, v + 192) - v <= 128) continue;
+    lo = std::min(lo, v[0]);
+    hi = std::max(hi, *std::max_element(r, r + 192));
+    apart[loose++] = r;
+  }
+  if (loose == 0) return;
+  const float* const pos = positions(lo, hi - lo + 1);
+  int32_t weight = 0;
+  for (int32_t k = 0; k < loose; k++) {
+    // Longest side of the box of `count` vertices.
+    auto extent = [&](const int32_t* r, int count) {
+      float e = 0.0f;
+      for (int c = 0; c < 3; c++) {
+        float a = INFINITY, b = -INFINITY;
+        for (int i = 0; i < count; i++) {
+          const float x = pos[3 * (size_t)(r[i] - lo) + c];
+          a = std::min(a, x);
+          b = std::max(b, x);
+        }
+        e = std::max(e, b - a);
+      }
+      return (double)e;
+    };
+    double sum = 0.0, all = 0.0;
+    if (pos) {
+      all = extent(apart[k], 192);
+      for (int t = 0; t < 64; t++) sum += std::pow(extent(apart[k] + 3 * t, 3), 2) / 64;
+    }
+    const double size = all > 0.0 ? std::sqrt(sum) / all : 0.0;
+    weight += size >= kScatterLarge ? 0 : size >= kScatterMiddle ? kScatterMiddleWeight : kScatterWeight;
+  }
+  const int64_t regions = ((int64_t)m.ntri + 63) / 64;
+  m.loose = (int32_t)(regions * loose / n);
+  m.scatter = (int32_t)(regions * weight / n);
+}
+
 extern "C" {
 
 int mr_device_count(int32_t* count) {
@@ -1225,21 +1282,6 @@ static int upload(mr_ctx* c, DevBuf& b, const void* src, size_t bytes) {
   return MR_OK;
 }
 
-// Regions (64 consecutive triangles) of a mesh whose triangles lie apart, from
-// up to 16 of them spread over it: neighbours share corners (32 quads of a grid
-// row have 66), loose triangles or a shuffled mesh have up to 192 of their own.
-static int32_t loose_regions(const int32_t* ix, int32_t ntri) {
-  const int32_t whole = ntri / 64, n = std::min(whole, 16);
-  int32_t loose = 0;
-  for (int32_t k = 0; k < n; k++) {
-    int32_t v[192];
-    memcpy(v, ix + (size_t)((int64_t)k * whole / n) * 192, sizeof(v));
-    std::sort(v, v + 192);
-    loose += std::unique(v, v + 192) - v > 128;
-  }
-  return n ? (int32_t)(((int64_t)ntri + 63) / 64 * loose / n) : 0;
-}
-
 static bool indices_ok(const int32_t* ix, int64_t n, int32_t limit) {
   for (int64_t i = 0; i < n; i++)
     if (ix[i] < 0 || ix[i] >= limit) return false;
@@ -1264,7 +1306,7 @@ int mr_mesh_upload(mr_ctx* c, const float* positions, int32_t npos,
   MeshRec m;
   m.npos = npos; m.nnrm = nnrm; m.nuv = has_uv ? nuv : 0; m.ntri = ntri;
   m.has_uv = has_uv;
-  m.loose = loose_regions(indices, ntri);
+  look_at_regions(m, indices, [&](int32_t lo, int32_t) { return positions + 3 * (size_t)lo; });
   m.nidx_alias = normal_indices == indices;
   m.tidx_alias = has_uv && uv_indices == indices;
   int rc;
@@ -1302,7 +1344,16 @@ int mr_mesh_upload_shared(mr_ctx* c, int32_t base, const int32_t* indices,
   m.npos = o.npos; m.nnrm = o.nnrm; m.nuv = has_uv ? o.nuv : 0; m.ntri = ntri;
   m.has_uv = has_uv;
   m.owner = owner;
-  m.loose = loose_regions(indices, ntri);
+  std::unique_ptr<float[]> host;  // the vertices are on the device
+  look_at_regions(m, indices, [&](int32_t lo, int32_t n) -> const float* {
+    host.reset(new (std::nothrow) float[3 * (size_t)n]);
+    if (host && hipMemcpy(host.get(), (const char*)o.pos.p + 12 * (size_t)lo, 12 * (size_t)n,
+                          hipMemcpyDeviceToHost) != hipSuccess) {
+      (void)hipGetLastError();
+      host.reset();
+    }
+    return host.get();
+  });
   m.nidx_alias = normal_indices == indices;
   m.tidx_alias = has_uv && uv_indices == indices;
   int rc;

@@ -148,9 +148,18 @@ constexpr int kSmallRegions = 1536;
 // at 200 x 150 to 33 x 33: 87 and 69).
 constexpr int64_t kSmallRegionPixels = 512, kSmallExcess = 80;
 // Regions of a job with triangles in no spatial order: every tile meets them
-// all, where it meets 1 in 10 of a grid's.  6,000 small triangles 46 and 43 at
-// 320 x 240, 20,000 92 and 46; 6,000 larger ones 62 and 71.
+// all, where it meets 1 in 10 of a grid's.  For small triangles the general
+// kernels are the better ones from about 7,000 on, large ones cost these more
+// (they bin or list each for every tile), the larger and the more of them: so
+// regions count in full, for 7/12 or not at all by the size of their
+// triangles relative to the region.  At 640 x 480, sizes of 0.03, 0.12 and 0.21:
+// 6,000 triangles 54 and 50, 66 and 97, 82 and 135; 16,000 95 and 55, 132 and
+// 176, 169 and 298; 32,000 of the middle size 232 and 218.  Of 0.12 at other
+// sizes of frame, 8,000 and 16,000: 96 x 64 61 and 79, 96 and 97; 320 x 240 73 and
+// 76, 120 and 87; 1000 x 700 153 and 136, 265 and 217.
 constexpr int64_t kSmallLoose = 112;
+constexpr int32_t kScatterWeight = 12, kScatterMiddleWeight = 7;
+constexpr double kScatterMiddle = 0.09, kScatterLarge = 0.16;
 // A tile is drawn by one workgroup, or by up to 8, each a band of its rows,
 // while that makes at most kSmallGroups (about what the GPU holds at once): a
 // frame of few tiles left most CUs idle while each tile drew thousands of

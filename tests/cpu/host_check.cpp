@@ -269,11 +269,53 @@ static void check_small() {
   mr_ctx_destroy(c);
 }
 
+// Loose triangles of side `side` with centres in a box of side 1; shared: the
+// mesh refers to the vertices of another one.
+static int32_t upload_loose(mr_ctx* c, int ntri, float side, bool shared) {
+  std::vector<float> v(9 * (size_t)ntri);
+  std::vector<int32_t> ix(3 * (size_t)ntri);
+  unsigned seed = 1;
+  auto rnd = [&] { return (float)((seed = seed * 1664525u + 1013904223u) >> 8) / 16777216.0f; };
+  for (int t = 0; t < ntri; t++) {
+    const float m[3] = {rnd(), rnd(), rnd()};
+    for (int k = 0; k < 9; k++) v[9 * (size_t)t + k] = m[k % 3] + (k / 3 == k % 3 ? side : 0.0f);
+  }
+  for (int i = 0; i < 3 * ntri; i++) ix[i] = i;
+  int32_t h, first[3] = {0, 1, 2};
+  const int32_t* own = shared ? first : ix.data();
+  if (mr_mesh_upload(c, v.data(), 3 * ntri, v.data(), 3 * ntri, nullptr, 0, own, own, nullptr, shared ? 1 : ntri, &h))
+    FAIL("upload");
+  if (shared && mr_mesh_upload_shared(c, h, ix.data(), ix.data(), nullptr, ntri, &h)) FAIL("shared upload");
+  return h;
+}
+
+static void check_scatter() {
+  mr_ctx* c = open_ctx();
+  render(c, upload(c, 4), 1, 3840, 2160);  // buffers large enough for all below
+  const struct { int ntri; float side; bool small; } cases[] = {
+      {7168, 0.03f, true}, {7169, 0.03f, false},   // 112 regions of small triangles
+      {12288, 0.14f, true}, {12353, 0.14f, false}, // 192 of middling ones (0.14 / 1.14 of the region)
+      {8000, 0.3f, true}, {20000, 0.3f, true},     // large ones count by the other limits only
+      {98304, 0.3f, true}, {98305, 0.3f, false},
+  };
+  for (auto& k : cases)
+    for (int shared = 0; shared < 2; shared++) {
+      render(c, upload_loose(c, k.ntri, k.side, shared), 1, 320, 240);
+      if (mr::g_small != k.small) FAIL("%d triangles of %g, shared %d: small %d", k.ntri, k.side, shared, mr::g_small);
+    }
+  render(c, upload_loose(c, 5000, 0.3f, false), 2, 320, 240);
+  if (!mr::g_small) FAIL("two draws");
+  render(c, upload_loose(c, 5000, 0.03f, true), 2, 320, 240);
+  if (mr::g_small) FAIL("two draws of small triangles");
+  mr_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "clean")) check_clean();
   else if (!strcmp(what, "launches")) check_launches();
   else if (!strcmp(what, "small")) check_small();
+  else if (!strcmp(what, "scatter")) check_scatter();
   else FAIL("nothing to check");
   printf("ok\n");
   return 0;

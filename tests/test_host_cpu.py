@@ -37,3 +37,9 @@ def test_small_batches_are_those_that_gain(host_bin):
     many tests take the general kernels; frames of few tiles are shared out in
     row bands."""
     run(host_bin, "small")
+
+
+def test_large_loose_triangles_take_the_small_kernels(host_bin):
+    """Loose triangles are held to a limit by their size: the general kernels
+    bin each for every tile, which costs more the larger they are."""
+    run(host_bin, "scatter")
