@@ -1483,7 +1483,10 @@ __device__ inline void raster_pixel(u64* keys, int p, float e1, float e2, float 
   if (key < keys[p]) atomicMin(&keys[p], key);
 }
 
-constexpr int kCoverRowsMin = 4;  // wide entries of a wavefront from which rows are tested
+// Wide entries of a wavefront from which rows are tested (cover_rows): a frame
+// of 3,000 large triangles at 1080p takes 430 us a call without the test, 279
+// from 1 or 4 entries on, 282 from 16; other frames are within 1 % either way.
+constexpr int kCoverRowsMin = 4;
 
 // Workgroup memory of the raster.  Key rows are padded by one entry: pixels of
 // one column in different rows fall in different LDS banks.
@@ -2770,9 +2773,8 @@ hipError_t launch_persistent(const BatchArgs& a, bool clear, unsigned long long*
   q.nvb[kPTile] = (int32_t)std::min<int64_t>((int64_t)a.ntiles + (int64_t)a.parts_cap, INT32_MAX);
   q.nvb[kPShade] = a.shade_blocks;
   // Items per queue workgroup: one for the even stages, several for the
-  // raster and shading, whose workgroups differ in cost; the scan's
-  // workgroups one at a time (each waits on its predecessors).
-  const int32_t depth[kPStages] = {1, 1, 1, 1 << 30, 1, 1, 8, 4};
+  // raster and shading, whose workgroups differ in cost.
+  const int32_t depth[kPStages] = {1, 1, 1, 1, 1, 1, 8, 4};
   const int32_t wait[kPStages] = {0, 0, 1, 1, 1, 1, 1, 1};
   for (int i = 0; i < kPStages; i++) {
     q.depth[i] = depth[i];

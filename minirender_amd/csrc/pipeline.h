@@ -125,7 +125,9 @@ struct TableArgs {
 // Batches of at most this many triangles run k_front: beyond, transforming
 // each vertex once costs less than once per corner (vertex and geometry
 // kernels together 16.3 -> 12.0 us at 120 k triangles, 35 -> 32.5 at 1 M, but
-// 55 -> 61 at 2.1 M).
+// 55 -> 61 at 2.1 M).  Meshes that no call before has brought into a cache gain
+// the same: 1.5 GB of meshes in turn, us a call with two kernels and one, 72.9
+// and 66.5 at 100 k triangles, 103.8 and 96.9 at 1 M, 115.5 and 109.5 at 1.4 M.
 constexpr int64_t kFrontTris = 1500000;
 // Small batches (k_front and k_small, whose tiles test every region of their
 // job): what the two kernels do sooner than the general ones (us a call, small
