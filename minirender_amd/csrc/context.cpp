@@ -142,7 +142,8 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
   plan.npixels = 0;
   plan.shade_blocks = 0;
   plan.max_width = 0;
-  plan.small_tests = plan.max_regions = plan.max_excess = plan.max_loose = plan.max_scatter = 0;
+  plan.max_regions = plan.max_ordered = plan.max_loose = plan.max_scatter = 0;
+  plan.small_tests = plan.ordered_tests = plan.ordered_regions = 0;
   const int tw = c->tile_w, th = c->tile_h;
   for (int j = 0; j < nframes; j++) {
     const mr_frame* f = &frames[j];
@@ -180,7 +181,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     J.lighting = f->lighting != 0;
     J.save_normals = f->save_normals != 0;
     uint64_t order = 0;
-    int64_t loose = 0, scatter = 0;
+    int64_t loose = 0, scatter = 0, large = 0;
     // (attribute owner, modelview) -> first vertex record
     std::map<std::string, int64_t> groups;
     for (int d = 0; d < f->ndraws; d++) {
@@ -244,6 +245,7 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
       order += 2ull * (uint64_t)m.ntri;
       loose += m.loose;
       scatter += m.scatter;
+      large += m.large;
       plan.total_tris += m.ntri;
       plan.draws.push_back(D);
       plan.draw_begin.push_back(D.tri_begin);
@@ -254,10 +256,12 @@ int build_batch(mr_ctx* c, const mr_frame* frames, int nframes, BatchPlan& plan)
     plan.max_width = std::max(plan.max_width, J.W);
     const int64_t regions = ((J.tri_end + 63) >> 6) - (J.tri_begin >> 6);
     plan.max_regions = std::max(plan.max_regions, regions);
-    plan.max_excess = std::max(plan.max_excess, regions - npix / kSmallRegionPixels);
+    plan.max_ordered = std::max(plan.max_ordered, regions - large);
     plan.max_loose = std::max(plan.max_loose, loose);
     plan.max_scatter = std::max(plan.max_scatter, scatter);
     plan.small_tests += (int64_t)J.tiles_x * J.tiles_y * regions;
+    plan.ordered_regions += regions - large;
+    plan.ordered_tests += (int64_t)J.tiles_x * J.tiles_y * (regions - large);
   }
   if (2 * plan.total_tris >= 0xFFFFFFFFll || plan.total_verts >= 0x7FFFFFFFll) return MR_ERR_ARG;
   // Job hints for the raster's and shading's job lookup: every kHintSpan-th
@@ -521,11 +525,12 @@ static void device_address(const HostBuf& b, void*& of, void*& dev) {
 }
 
 // Whether k_small does the batch, and in how many row bands per tile (pipeline.h).
-static bool small_batch(const BatchPlan& p) {
+static bool small_batch(const BatchPlan& p, int tile) {
+  const SmallWork w = small_work(tile);
   return p.max_width <= kSmallWidth && p.ntiles <= kSmallTiles && p.small_tests <= kSmallTests &&
-         (p.ntiles <= kSmallRoundTiles || p.small_tests <= kSmallRoundTests) &&
-         p.max_regions <= kSmallRegions && p.max_scatter <= kSmallLoose * kScatterWeight &&
-         (p.jobs.size() == 1 || p.max_excess <= kSmallExcess);
+         p.ordered_tests + w.region * p.ordered_regions + w.tile * p.ntiles <= w.most &&
+         p.max_regions <= kSmallRegions && p.max_ordered <= small_ordered_regions(tile) &&
+         p.max_scatter <= kSmallLoose * kScatterWeight;
 }
 
 static int32_t small_bands(const BatchPlan& p) {
@@ -583,7 +588,7 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
   // meshes, and whether a small batch's records fit the checkpoint buffer (one
   // that earlier batches have grown holds more than this batch asks for).
   a.front = !persistent && p.total_tris > 0 && p.total_tris <= kFrontTris;
-  a.small = a.front && a.host_counters && small_batch(p) &&
+  a.small = a.front && a.host_counters && small_batch(p, c->tile_w) &&
             (uint64_t)a.nregions * (kRegion * sizeof(SetupRec) + 8) <= x.ckpt.bytes;
   if (a.small) a.small_bands = small_bands(p);
   a.recs = (SetupRec*)x.ckpt.p;
@@ -1053,7 +1058,8 @@ int render_frames(mr_ctx* c, const mr_frame* frames, int n, const mr_outputs* ou
 // up to 16 of them spread over it: neighbours share corners (32 quads of a grid
 // row have 66), loose triangles or a shuffled mesh have up to 192 of their own.
 // m.scatter: how far such regions count against kSmallLoose, by the triangles'
-// extent in the region's (root of the mean square of the longest sides).
+// extent in the region's (root of the mean square of the longest sides);
+// m.large: those that do not.
 // Meshes of more triangles than a small batch takes are not looked at.
 // positions(lo, n): n vertices from lo on in host memory, or null.
 template <typename Positions>
@@ -1074,7 +1080,7 @@ static void look_at_regions(MeshRec& m, const int32_t* ix, Positions&& positions
   }
   if (loose == 0) return;
   const float* const pos = positions(lo, hi - lo + 1);
-  int32_t weight = 0;
+  int32_t weight = 0, large = 0;
   for (int32_t k = 0; k < loose; k++) {
     // Longest side of the box of `count` vertices.
     auto extent = [&](const int32_t* r, int count) {
@@ -1096,11 +1102,13 @@ static void look_at_regions(MeshRec& m, const int32_t* ix, Positions&& positions
       for (int t = 0; t < 64; t++) sum += std::pow(extent(apart[k] + 3 * t, 3), 2) / 64;
     }
     const double size = all > 0.0 ? std::sqrt(sum) / all : 0.0;
-    weight += size >= kScatterLarge ? 0 : size >= kScatterMiddle ? kScatterMiddleWeight : kScatterWeight;
+    if (size >= kScatterLarge) large++;
+    else weight += size >= kScatterMiddle ? kScatterMiddleWeight : kScatterWeight;
   }
   const int64_t regions = ((int64_t)m.ntri + 63) / 64;
   m.loose = (int32_t)(regions * loose / n);
   m.scatter = (int32_t)(regions * weight / n);
+  m.large = (int32_t)(regions * large / n);
 }
 
 extern "C" {

@@ -39,7 +39,7 @@ struct MeshRec {
   int32_t npos = 0, nnrm = 0, nuv = 0, ntri = 0;
   // Regions of triangles in no spatial order, and their weight in the choice of
   // small batches (look_at_regions).
-  int32_t loose = 0, scatter = 0;
+  int32_t loose = 0, scatter = 0, large = 0;
   int32_t owner = -1;   // mesh holding the attribute arrays, -1: this one
   int32_t sharers = 0;  // meshes using this mesh's attribute arrays
   bool has_uv = false;
@@ -92,11 +92,12 @@ struct BatchPlan {
   int64_t npixels = 0;
   int64_t shade_blocks = 0;
   int32_t max_width = 0;
-  // For the choice of small batches: regions of one job at most (and above
-  // one per kSmallRegionPixels of its pixels), its loose ones at most (and
-  // weighted by their triangles' size), and regions that the tiles test
-  // together.
-  int64_t max_regions = 0, max_excess = 0, max_loose = 0, max_scatter = 0, small_tests = 0;
+  // For the choice of small batches: regions of one job at most (without those
+  // of large triangles in no order: "ordered"), its regions in no order at most
+  // (and weighted by their triangles' size); all jobs' regions, and regions that
+  // the tiles test together.
+  int64_t max_regions = 0, max_ordered = 0, max_loose = 0, max_scatter = 0;
+  int64_t ordered_regions = 0, small_tests = 0, ordered_tests = 0;
   TableLayout layout;
 };
 

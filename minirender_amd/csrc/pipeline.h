@@ -134,21 +134,33 @@ constexpr int64_t kFrontTris = 1500000;
 // and general; 64 triangles a region).
 constexpr int kSmallWidth = 1024;  // rows are walked from the bbox's left column
 constexpr int kSmallTiles = 8192;
-// (tile, region) pairs tested.  Few tiles run beside each other (a grid of
-// 16,000 at 1000 x 700, 693,000 pairs: 48 and 56), more in rounds: 16 frames of
-// 256 tiles and 74 regions (303,000) 68 and 67, 30 of them 98 and 86, 30 frames
-// of 24 regions (184,000) 81 and 84.
-constexpr int64_t kSmallTests = 800000;
-constexpr int kSmallRoundTiles = 3072;
-constexpr int64_t kSmallRoundTests = 300000;  // of batches of more tiles
+constexpr int64_t kSmallTests = 800000;  // (tile, region) pairs tested
+// The work that makes the general kernels the sooner ones, in pairs tested: a
+// region is also set up and drawn tile by tile, a tile is a workgroup whose
+// latency counts once a few rounds of them run.  Fitted to 750 calls of 1 to 150
+// grids of 300 to 40,000 triangles at 33 x 33 to 1000 x 800; in 16-pixel tiles
+// (their pairs, regions and tiles): one grid at 1000 x 800 of 9,000 (444,000, 141,
+// 3,150) 48 and 56; 2 frames at 120 x 90 of 9,000 37 and 44; 16 at 250 x 250 of 4,700
+// (303,000, 1,184, 4,096) 69 and 66, 30 of them 98 and 86; 150 at 120 x 90 of 2,500
+// (288,000, 6,000, 7,200) 128 and 100.  A 32-pixel tile holds four times the pixels
+// and their items: 32 frames at 250 x 250 of 1,000 (32,000, 512, 2,048) 77 and 78, of
+// 4,700 (152,000, 2,368, 2,048) 99 and 80; 8 at 120 x 90 of 9,000 48 and 59.  In
+// 8-pixel tiles: a sphere of 4 k at 640 x 480 (298,000, 62, 4,800) 37 and 68, 64
+// frames at 64 x 64 of 4,700 (303,000, 4,736, 4,096) 85 and 63.
+struct SmallWork {
+  int64_t region, tile, most;
+};
+constexpr SmallWork small_work(int tile) {
+  if (tile >= 32) return {60, 75, 300000};
+  return {tile >= 16 ? 400 : 550, 75, 1200000};
+}
 // Regions of one job (k_small lists them in LDS): grids at 320 x 240 of 469 take
 // 42 and 47, of 938 48 and 47, of 2,000 56 and 47; spheres 35 and 53, 39 and 53,
-// 40 and 50.
+// 40 and 50.  The one wavefront of an 8-pixel tile tests them by itself: grids at
+// 120 x 90 of 74 regions take 44 and 44, of 282 51 and 41, of 625 54 and 41 (at
+// 250 x 250 39 and 47, 57 and 47, 60 and 47).
 constexpr int kSmallRegions = 1536;
-// Regions of a job beside others, whose few tiles are not shared out further:
-// one per kSmallRegionPixels and kSmallExcess (24 frames of 1 k - 60 k triangles
-// at 200 x 150 to 33 x 33: 87 and 69).
-constexpr int64_t kSmallRegionPixels = 512, kSmallExcess = 80;
+constexpr int small_ordered_regions(int tile) { return tile <= 8 ? 192 : kSmallRegions; }
 // Regions of a job with triangles in no spatial order: every tile meets them
 // all, where it meets 1 in 10 of a grid's.  For small triangles the general
 // kernels are the better ones from about 7,000 on, large ones cost these more
@@ -159,6 +171,8 @@ constexpr int64_t kSmallRegionPixels = 512, kSmallExcess = 80;
 // 176, 169 and 298; 32,000 of the middle size 232 and 218.  Of 0.12 at other
 // sizes of frame, 8,000 and 16,000: 96 x 64 61 and 79, 96 and 97; 320 x 240 73 and
 // 76, 120 and 87; 1000 x 700 153 and 136, 265 and 217.
+// Large ones count neither in small_work nor for small_ordered_regions (8,000 at
+// 640 x 480 in 8-pixel tiles 884 and 3,239).
 constexpr int64_t kSmallLoose = 112;
 constexpr int32_t kScatterWeight = 12, kScatterMiddleWeight = 7;
 constexpr double kScatterMiddle = 0.09, kScatterLarge = 0.16;

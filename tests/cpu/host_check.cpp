@@ -255,10 +255,11 @@ static void check_small() {
       {98304, true, 320, 240, 1, 2},    // 1,536 regions
       {98305, true, 320, 240, 1, 0},
       {4713, true, 250, 250, 12, 1},    // 3,072 tiles
-      {4713, true, 250, 250, 16, 0},    // 303,000 tests of 4,096 tiles
+      {4713, true, 250, 250, 16, 1},    // 303,000 tests of 4,096 tiles
+      {4713, true, 250, 250, 18, 0},
       {1500, true, 250, 250, 30, 1},
-      {5824, true, 96, 64, 8, 1},       // 91 regions a job, 92 allowed beside others
-      {5952, true, 96, 64, 8, 0},       // 93
+      {9024, true, 120, 90, 8, 2},      // 141 regions a job
+      {9024, true, 120, 90, 24, 0},
   };
   for (auto& k : cases) {
     render(c, upload(c, k.ntri, k.strip), 1, k.w, k.h, k.n);
@@ -310,12 +311,43 @@ static void check_scatter() {
   mr_ctx_destroy(c);
 }
 
+static void check_tiles() {
+  mr_ctx* c = open_ctx();
+  render(c, upload(c, 4), 1, 3840, 2160);  // buffers large enough for all below
+  const struct { int tile, ntri, w, h, n; bool small; } cases[] = {
+      {8, 12288, 120, 90, 1, true}, {8, 12289, 120, 90, 1, false},    // 192 regions
+      {16, 12289, 120, 90, 1, true},
+      {16, 2560, 120, 90, 54, true}, {16, 2560, 120, 90, 56, false},  // 40 regions, 48 tiles a frame
+      {16, 9024, 1000, 800, 1, true},
+      {32, 4736, 250, 250, 20, true}, {32, 4736, 250, 250, 22, false},  // 74 regions, 64 tiles
+      {32, 1024, 250, 250, 40, true}, {32, 1024, 250, 250, 64, false},
+      {32, 640, 250, 250, 64, false}, {32, 9024, 120, 90, 8, true},
+      {8, 4736, 64, 64, 20, true}, {8, 4736, 64, 64, 32, false},
+      {8, 3968, 640, 480, 1, true}, {8, 3968, 200, 150, 12, true},
+  };
+  for (auto& k : cases) {
+    mr_ctx_set_tile(c, k.tile, k.tile);
+    render(c, upload(c, k.ntri, true), 1, k.w, k.h, k.n);
+    if (mr::g_small != k.small) FAIL("%d triangles, %d of %d x %d, tile %d: small %d", k.ntri, k.n, k.w, k.h, k.tile, mr::g_small);
+  }
+  mr_ctx_set_tile(c, 8, 8);
+  for (int ntri : {20000, 8000}) {
+    render(c, upload_loose(c, ntri, 0.3f, false), 1, ntri == 20000 ? 320 : 640, ntri == 20000 ? 240 : 480);
+    if (!mr::g_small) FAIL("%d large loose triangles, tile 8", ntri);
+  }
+  mr_ctx_set_tile(c, 16, 16);
+  render(c, upload_loose(c, 12000, 0.3f, true), 1, 1000, 1000);
+  if (!mr::g_small) FAIL("large loose triangles, 3,969 tiles");
+  mr_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "clean")) check_clean();
   else if (!strcmp(what, "launches")) check_launches();
   else if (!strcmp(what, "small")) check_small();
   else if (!strcmp(what, "scatter")) check_scatter();
+  else if (!strcmp(what, "tiles")) check_tiles();
   else FAIL("nothing to check");
   printf("ok\n");
   return 0;

@@ -43,3 +43,9 @@ def test_large_loose_triangles_take_the_small_kernels(host_bin):
     """Loose triangles are held to a limit by their size: the general kernels
     bin each for every tile, which costs more the larger they are."""
     run(host_bin, "scatter")
+
+
+def test_small_batches_by_tile_size(host_bin):
+    """8-pixel tiles test regions with one wavefront, 32-pixel tiles draw four
+    times the pixels each: limits of their own."""
+    run(host_bin, "tiles")
