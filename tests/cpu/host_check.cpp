@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <string>
 #include <vector>
 
 #include "minirender_amd.h"
@@ -24,6 +25,8 @@
 
 // ---- the HIP runtime --------------------------------------------------------
 static std::vector<void*> g_free;
+static std::string* g_captured = nullptr;  // the graph being captured
+static int g_updates = 0;
 static void* block(size_t bytes) {
   constexpr size_t kBlock = (size_t)1 << 32;
   if (bytes > kBlock) return nullptr;
@@ -58,12 +61,19 @@ hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)malloc(1); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = nullptr; return hipSuccess; }
-hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
-hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) { *e = nullptr; return hipSuccess; }
-hipError_t hipGraphExecUpdate(hipGraphExec_t, hipGraph_t, hipGraphNode_t*, hipGraphExecUpdateResult*) { return hipErrorNotSupported; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+// A graph is the names of the kernels launched while it was captured; an update
+// keeps the kernels, so it has to be of the same ones.
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { g_captured = new std::string; return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = (hipGraph_t)g_captured; g_captured = nullptr; return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t g) { delete (std::string*)g; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t) { *e = (hipGraphExec_t)new std::string(*(std::string*)g); return hipSuccess; }
+hipError_t hipGraphExecUpdate(hipGraphExec_t e, hipGraph_t g, hipGraphNode_t*, hipGraphExecUpdateResult* r) {
+  if (*(std::string*)e != *(std::string*)g) FAIL("a graph of %s updated by one of %s", ((std::string*)e)->c_str(), ((std::string*)g)->c_str());
+  g_updates++;
+  *r = hipGraphExecUpdateSuccess;
+  return hipSuccess;
+}
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete (std::string*)e; return hipSuccess; }
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)malloc(1); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
@@ -78,6 +88,11 @@ namespace mr {
 static int g_launches = 0;  // kernels launched
 static bool g_general = false, g_small = false;
 static int g_bands = 0;  // of the last small batch
+
+static void launched(const char* name, int kind = 0) {
+  g_launches++;
+  if (g_captured) *g_captured += name + std::to_string(kind) + " ";
+}
 
 static void zero(const BatchArgs& a) {
   memset(a.counters, 0, kNumCounters * 8);
@@ -103,11 +118,11 @@ static void hand_counters(const BatchArgs& a) {
   zero(a);
 }
 
-hipError_t launch_tables(const void* p, void* t, size_t n, hipStream_t) { g_launches++; memcpy(t, p, n); return hipSuccess; }
-hipError_t launch_clear(const BatchArgs& a, hipStream_t) { g_launches++; zero(a); zero_tiles(a); return hipSuccess; }
-hipError_t launch_vertex(const BatchArgs& a, hipStream_t) { if (a.total_verts) g_launches++, zero(a); return hipSuccess; }
+hipError_t launch_tables(const void* p, void* t, size_t n, hipStream_t) { launched("tables"); memcpy(t, p, n); return hipSuccess; }
+hipError_t launch_clear(const BatchArgs& a, hipStream_t) { launched("clear"); zero(a); zero_tiles(a); return hipSuccess; }
+hipError_t launch_vertex(const BatchArgs& a, hipStream_t) { if (a.total_verts) launched("vertex"), zero(a); return hipSuccess; }
 static hipError_t geometry(const BatchArgs& a) {
-  g_launches++;
+  launched("geometry", 2 * a.front + a.small);
   g_general = !a.small;
   if (a.small) return hipSuccess;
   expect_zero(a);
@@ -117,7 +132,7 @@ static hipError_t geometry(const BatchArgs& a) {
 hipError_t launch_geometry(const BatchArgs& a, hipStream_t) { return a.total_tris ? geometry(a) : hipSuccess; }
 hipError_t launch_front(const BatchArgs& a, const void*, size_t, hipStream_t) { return geometry(a); }
 hipError_t launch_small(const BatchArgs& a, hipStream_t) {
-  g_launches++;
+  launched("small", 2 * a.tile_w + (a.small_bands > 1));
   g_small = true;
   g_bands = a.small_bands;
   if (a.small_bands < 1 || a.tile_h % a.small_bands || (a.small_bands > 1 && a.small_bands * a.ntiles > kSmallGroups))
@@ -125,13 +140,13 @@ hipError_t launch_small(const BatchArgs& a, hipStream_t) {
   memset(a.host_counters, 0, kNumCounters * 8);
   return hipSuccess;
 }
-hipError_t launch_scan(const BatchArgs&, hipStream_t) { g_launches++; return hipSuccess; }
-hipError_t launch_bin(const BatchArgs&, hipStream_t) { g_launches++; return hipSuccess; }
-hipError_t launch_rows(const BatchArgs& a, hipStream_t) { g_launches += !a.ckpt_in_scan; return hipSuccess; }
-hipError_t launch_tile(const BatchArgs&, hipStream_t) { g_launches++; return hipSuccess; }
-hipError_t launch_shade(const BatchArgs& a, hipStream_t) { g_launches++; zero_tiles(a); hand_counters(a); return hipSuccess; }
+hipError_t launch_scan(const BatchArgs&, hipStream_t) { launched("scan"); return hipSuccess; }
+hipError_t launch_bin(const BatchArgs& a, hipStream_t) { launched("bin", a.ckpt_in_scan); return hipSuccess; }
+hipError_t launch_rows(const BatchArgs& a, hipStream_t) { if (!a.ckpt_in_scan) launched("rows"); return hipSuccess; }
+hipError_t launch_tile(const BatchArgs& a, hipStream_t) { launched("tile", a.tile_w); return hipSuccess; }
+hipError_t launch_shade(const BatchArgs& a, hipStream_t) { launched("shade"); zero_tiles(a); hand_counters(a); return hipSuccess; }
 hipError_t launch_persistent(const BatchArgs& a, bool clear, unsigned long long*, unsigned long long*, uint64_t, hipStream_t) {
-  g_launches++;
+  launched("persistent");
   if (clear) zero_tiles(a);
   zero(a);
   expect_zero(a);
@@ -341,6 +356,23 @@ static void check_tiles() {
   mr_ctx_destroy(c);
 }
 
+// Frames of many sizes in turn, replayed: a graph is updated in place to one of
+// the same kernels only.
+static void check_graphs() {
+  mr_ctx* c = open_ctx();
+  mr_ctx_set_graphs(c, 1);
+  const int32_t few = upload(c, 64, true), many = upload(c, 7000, true);
+  const int sizes[][2] = {{96, 64}, {90, 60}, {250, 145}, {640, 480}, {600, 400}, {1000, 700}, {1100, 64}, {1100, 80}, {1100, 1000}, {1200, 900}};
+  for (int rep = 0; rep < 3; rep++)
+    for (int tile : {16, 32}) {
+      mr_ctx_set_tile(c, tile, tile);
+      for (auto& s : sizes) render(c, few, 1, s[0], s[1]);
+      for (auto& s : sizes) render(c, many, 1, s[0], s[1]);
+    }
+  if (!g_updates) FAIL("no graph was updated");
+  mr_ctx_destroy(c);
+}
+
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "clean")) check_clean();
@@ -348,6 +380,7 @@ int main(int argc, char** argv) {
   else if (!strcmp(what, "small")) check_small();
   else if (!strcmp(what, "scatter")) check_scatter();
   else if (!strcmp(what, "tiles")) check_tiles();
+  else if (!strcmp(what, "graphs")) check_graphs();
   else FAIL("nothing to check");
   printf("ok\n");
   return 0;

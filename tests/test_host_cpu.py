@@ -49,3 +49,9 @@ def test_small_batches_by_tile_size(host_bin):
     """8-pixel tiles test regions with one wavefront, 32-pixel tiles draw four
     times the pixels each: limits of their own."""
     run(host_bin, "tiles")
+
+
+def test_graphs_are_updated_to_the_same_kernels(host_bin):
+    """An instantiated graph takes another batch's parameters only when that
+    batch launches the same kernels."""
+    run(host_bin, "graphs")
