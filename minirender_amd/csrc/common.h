@@ -130,17 +130,18 @@ MR_HD inline TileItems tile_items(const unsigned long long* counters, uint32_t p
   return r;
 }
 
-// Row bands that each tile rastered whole is shared out in.  A tile's direct
-// entries (up to kDirectCap) are not among those that the scan splits tiles
-// by, so one workgroup a tile would draw them all, however few tiles there are.
-// From kBandDirect items (a chunk of the raster) up to 8 workgroups draw a
-// tile while these are at most kBandGroups, about what the GPU holds, and the
-// raster's grid (ntiles + parts_cap) holds them anyway.  With the shares of
+// Row bands that each tile rastered whole is shared out in, in batches of few
+// tiles.  A tile's direct entries (up to kDirectCap) are not among those that
+// the scan splits tiles by, so one workgroup a tile would draw them all, however
+// few tiles there are.  From kBandDirect items (a chunk of the raster) up to 8
+// workgroups draw a tile while these are at most kBandGroups, about what the GPU
+// holds, and the raster's grid (ntiles + parts_cap) holds them anyway.  With the shares of
 // split tiles (direct_share), us a call: 8,000 triangles over a 96 x 64 frame
 // 376 -> 310 (335 with all of them binned and split), 20,000 690 -> 404 (430);
 // 20,000 over 320 x 240 885 -> 636.
 constexpr int64_t kBandGroups = 1024;
 constexpr unsigned long long kBandDirect = 256;
+MR_HD inline bool few_tiles(int32_t ntiles) { return ntiles <= kBandGroups; }
 MR_HD inline int whole_bands(const unsigned long long* counters, const TileItems& r,
                              uint32_t parts_cap, int32_t ntiles, int tile_h) {
   int n = 1;

@@ -652,10 +652,10 @@ int enqueue_batch(mr_ctx* c, Slot& s, BatchPlan& p, bool profile) {
     // geometry launches, raster template, persistent or not) updates the
     // parameters of an instantiated graph in place instead of instantiating
     // a new one, so a service of mixed batches keeps replaying a few graphs.
-    const int32_t topo_v[9] = {clear ? 1 : 0, a.total_verts ? 1 : 0, a.total_tris ? 1 : 0,
+    const int32_t topo_v[10] = {clear ? 1 : 0, a.total_verts ? 1 : 0, a.total_tris ? 1 : 0,
                                a.tile_w, a.raster_threads, persistent ? 1 : 0,
                                persistent ? 0 : a.ckpt_in_scan, 2 * a.small + a.front,
-                               a.small_bands > 1 ? 1 : 0};
+                               a.small_bands > 1 ? 1 : 0, few_tiles(a.ntiles) ? 1 : 0};
     std::vector<unsigned char> topo((const unsigned char*)topo_v,
                                     (const unsigned char*)topo_v + sizeof(topo_v));
     if (hit == s.graphs.size()) {

@@ -1615,16 +1615,19 @@ __device__ inline TileItems tile_items(const BatchArgs& a) {
 // parts_cap + ntiles workgroups; workgroups past the actual number of items
 // exit at once.  remap: listed tiles in XCD-interleaved order (own launch,
 // where consecutive workgroups go to different XCDs), else in list order.
-template <int TW, int TH, int NT>
-__device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool remap) {
+// kFew (few_tiles): tiles rastered whole are shared out in row bands, and the
+// direct entries of a split tile over its parts.  An instantiation of its own:
+// the bands' arithmetic in every workgroup took the raster of 48 mixed frames
+// from 287 to 314 us.
+template <int TW, int TH, int NT, bool kFew>
+__device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool remap,
+                                           RasterLds<TW, TH, NT>& lds, int& sh_last) {
   constexpr int NP = TW * TH, KS = RasterLds<TW, TH, NT>::KS;
-  __shared__ RasterLds<TW, TH, NT> lds;
   u64* const keys = lds.keys;
-  __shared__ int sh_last;
   const int tid = threadIdx.x;
   bool direct = a.counters[kDirect] != 0ull;
   const TileItems items = tile_items(a);
-  const int bands = whole_bands(a.counters, items, a.parts_cap, a.ntiles, TH);
+  const int bands = kFew ? whole_bands(a.counters, items, a.parts_cap, a.ntiles, TH) : 1;
   if (b >= items.parts + items.listed * bands) return;
   int tile, part;
   uint32_t cnt, off;  // the tile's bin entries: number and first
@@ -1648,7 +1651,7 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     // are not in it (shading writes their background).
     // (Tiles with direct entries only are listed from the end.)
     int64_t t = b - items.parts;
-    if (bands > 1) {  // (few tiles)
+    if (kFew && bands > 1) {
       const int bi = (int)((uint32_t)t / (uint32_t)items.listed);
       t -= bi * items.listed;
       band_lo = bi * (TH / bands);
@@ -1674,13 +1677,14 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
     else if ((u64)off + cnt > a.bins_cap) avail = (uint32_t)(a.bins_cap - off);
     const uint32_t e_begin = (uint32_t)part * a.frag_size;
     const uint32_t e_end = min(avail, e_begin + a.frag_size);
-    // The entries: the bin entries, then the direct ones (a split tile's
-    // parts share them).
+    // The entries: the bin entries, then the direct ones (by the first part of
+    // a split tile, or shared out).
     const uint32_t nbin = e_end > e_begin ? e_end - e_begin : 0u;
     uint32_t nall = nbin, off2 = 0;
-    if (direct) {
+    if (direct && (kFew || part == 0)) {
       const u64 range = a.tile_count[(size_t)tile * kCtrStride64 + 1];
-      const DirectShare ds = direct_share((uint32_t)(range >> 32), (uint32_t)part, nparts);
+      DirectShare ds = {0, (uint32_t)(range >> 32)};
+      if (kFew) ds = direct_share(ds.end, (uint32_t)part, nparts);
       off2 = (uint32_t)range + ds.first - nbin;
       nall += ds.end - ds.first;
     }
@@ -1744,9 +1748,11 @@ __device__ __forceinline__ void stage_tile(const BatchArgs& a, int64_t b, bool r
   }
 }
 
-template <int TW, int TH, int NT>
+template <int TW, int TH, int NT, bool kFew>
 __global__ __launch_bounds__(NT, 6) void k_tile(BatchArgs a) {
-  stage_tile<TW, TH, NT>(a, blockIdx.x, true);
+  __shared__ RasterLds<TW, TH, NT> lds;
+  __shared__ int sh_last;
+  stage_tile<TW, TH, NT, kFew>(a, blockIdx.x, true, lds, sh_last);
 }
 
 // Range image of the pixel from its depth (Renderer.cpp:388-415).
@@ -2318,7 +2324,8 @@ __device__ inline u64 ctl_load(const u64* p) {
 __device__ inline int64_t persist_stage_size(const BatchArgs& a, const PersistPlan& q, int s) {
   if (s != kPTile) return q.nvb[s];
   const TileItems items = tile_items(a);
-  const int bands = whole_bands(a.counters, items, a.parts_cap, a.ntiles, a.tile_h);
+  const int bands =
+      few_tiles(a.ntiles) ? whole_bands(a.counters, items, a.parts_cap, a.ntiles, a.tile_h) : 1;
   return min((int64_t)q.nvb[s], items.parts + items.listed * bands);
 }
 
@@ -2381,7 +2388,13 @@ __device__ __forceinline__ void persist_run(const BatchArgs& a, const PersistPla
       if (vb == 0 && threadIdx.x == 0) check_direct_room(a);
       stage_rows(a, (int)vb, q.nvb[s]);
       break;
-    case kPTile: stage_tile<TW, TW, 256>(a, vb, false); break;
+    case kPTile: {
+      __shared__ RasterLds<TW, TW, 256> lds;
+      __shared__ int sh_last;
+      if (few_tiles(a.ntiles)) stage_tile<TW, TW, 256, true>(a, vb, false, lds, sh_last);
+      else stage_tile<TW, TW, 256, false>(a, vb, false, lds, sh_last);
+      break;
+    }
     default: stage_shade(a, (int)vb, false); break;
   }
 }
@@ -2698,12 +2711,14 @@ bool raster_threads_supported(int tw, int nt) {
 
 #define MR_TILE_CASE(TW, NT)                                                         \
   if (a.tile_w == TW && a.raster_threads == NT) {                                     \
-    hipLaunchKernelGGL((k_tile<TW, TW, NT>), dim3(grid), dim3(NT), 0, s, a);          \
+    if (few) hipLaunchKernelGGL((k_tile<TW, TW, NT, true>), dim3(grid), dim3(NT), 0, s, a); \
+    else hipLaunchKernelGGL((k_tile<TW, TW, NT, false>), dim3(grid), dim3(NT), 0, s, a); \
     return hipGetLastError();                                                         \
   }
 
 hipError_t launch_tile(const BatchArgs& a, hipStream_t s) {
   const int grid = a.ntiles + (int)a.parts_cap;
+  const bool few = few_tiles(a.ntiles);
   if (a.tile_w != a.tile_h) return hipErrorInvalidValue;
   MR_TILE_CASE(8, 64)
   MR_TILE_CASE(8, 128)

@@ -143,7 +143,7 @@ hipError_t launch_small(const BatchArgs& a, hipStream_t) {
 hipError_t launch_scan(const BatchArgs&, hipStream_t) { launched("scan"); return hipSuccess; }
 hipError_t launch_bin(const BatchArgs& a, hipStream_t) { launched("bin", a.ckpt_in_scan); return hipSuccess; }
 hipError_t launch_rows(const BatchArgs& a, hipStream_t) { if (!a.ckpt_in_scan) launched("rows"); return hipSuccess; }
-hipError_t launch_tile(const BatchArgs& a, hipStream_t) { launched("tile", a.tile_w); return hipSuccess; }
+hipError_t launch_tile(const BatchArgs& a, hipStream_t) { launched("tile", 2 * a.tile_w + few_tiles(a.ntiles)); return hipSuccess; }
 hipError_t launch_shade(const BatchArgs& a, hipStream_t) { launched("shade"); zero_tiles(a); hand_counters(a); return hipSuccess; }
 hipError_t launch_persistent(const BatchArgs& a, bool clear, unsigned long long*, unsigned long long*, uint64_t, hipStream_t) {
   launched("persistent");
