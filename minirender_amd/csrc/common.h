@@ -118,15 +118,18 @@ MR_HD inline TileItems tile_items(const unsigned long long* counters, uint32_t p
   // whose setup with this tile's frame size and near plane gives boxes that
   // no checkpoints were taken for.  Nothing is drawn (nor shaded); the batch
   // runs again with a longer list.
-  TileItems r = {0, 0, 0};
-  if (counters[kBinOverflow]) return r;
-  const int64_t parts = (int64_t)counters[kParts], whole = (int64_t)counters[kListed];
   // After a merge-slot or part-list overflow the part list is incomplete:
   // split tiles are then skipped (the frame is re-run with larger buffers).
-  if (!counters[kHeavyOverflow]) r.parts = parts < parts_cap ? parts : parts_cap;
-  r.whole = whole < ntiles ? whole : ntiles;
-  r.listed = r.whole + (int64_t)counters[kDirectTilesListed];
-  if (r.listed > ntiles) r.listed = ntiles;
+  // (All words are loaded before one is looked at: every raster workgroup
+  // waits for them, also the many past the last item.)
+  const unsigned long long over = counters[kBinOverflow], heavy = counters[kHeavyOverflow];
+  const int64_t parts = (int64_t)counters[kParts], whole = (int64_t)counters[kListed],
+                direct = (int64_t)counters[kDirectTilesListed];
+  TileItems r;
+  const int64_t listed = over ? 0 : ntiles, split = over | heavy ? 0 : parts_cap;
+  r.parts = parts < split ? parts : split;
+  r.whole = whole < listed ? whole : listed;
+  r.listed = r.whole + direct < listed ? r.whole + direct : listed;
   return r;
 }
 
