@@ -1071,11 +1071,16 @@ static void look_at_regions(MeshRec& m, const int32_t* ix, Positions&& positions
   int32_t loose = 0, lo = INT32_MAX, hi = 0;
   for (int32_t k = 0; k < n; k++) {
     const int32_t* const r = ix + (size_t)((int64_t)k * whole / n) * 192;
-    int32_t v[192];
-    memcpy(v, r, sizeof(v));
-    std::sort(v, v + 192);
-    if (std::unique(v, v + 192) - v <= 128) continue;
-    lo = std::min(lo, v[0]);
+    // Distinct vertices, through a hash table: 8 us an upload, by sorting 33.
+    int32_t seen[512], distinct = 0;
+    std::fill(seen, seen + 512, -1);
+    for (int i = 0; i < 192; i++) {
+      uint32_t at = (uint32_t)r[i] * 2654435761u >> 23;
+      while (seen[at] >= 0 && seen[at] != r[i]) at = (at + 1) & 511;
+      if (seen[at] < 0) seen[at] = r[i], distinct++;
+    }
+    if (distinct <= 128) continue;
+    lo = std::min(lo, *std::min_element(r, r + 192));
     hi = std::max(hi, *std::max_element(r, r + 192));
     apart[loose++] = r;
   }
